@@ -49,7 +49,7 @@ struct JobDesc {
 };
 
 // Per-particle state a MEGNO job carries from one segment to the next: the
-// tangent matrix (16), L1, L2 and |M|_F^2 of the last turn.
+// tangent matrix (16), L1, L2 and log10|M|_F of the last turn.
 constexpr int kMegnoState = 19;
 
 struct BatchQueue {
@@ -130,7 +130,7 @@ __global__ void k_megno_init(double *__restrict__ state, uint64_t n_particles)
     for (int q = 0; q < 16; q++) st[q] = (q % 5 == 0) ? 1.0 : 0.0;
     st[16] = 0.0;
     st[17] = 0.0;
-    st[18] = 4.0;  // |I|_F^2
+    st[18] = 0.0;  // formed from the matrix in the first segment
 }
 
 template <int MODE>
@@ -176,7 +176,7 @@ __global__ void __launch_bounds__(256, 8) k_batch_track(BatchSeg S)
 // same results), with the matrix and sums kept per particle between segments.
 template <int MODE, bool OCT>
 __device__ __forceinline__ void megno_chunk(const BatchSeg &S, ConstPtr<JobDesc> J, uint32_t job, uint32_t base,
-                                            uint32_t n)
+                                            uint32_t n, const LogBin *log_tab)
 {
     const uint32_t lane = __lane_id(), i = base + lane;
     const bool in = i < n;
@@ -187,7 +187,8 @@ __device__ __forceinline__ void megno_chunk(const BatchSeg &S, ConstPtr<JobDesc>
     uint32_t *gsteps = J->steps;
     uint32_t j = 0, s = 0;
     double x = __builtin_nan(""), px = x, y = x, py = x;
-    double m[16], l1 = 0.0, l2 = 0.0, fb2 = 0.0;
+    double m[16];
+    MegnoSums sums{0.0, 0.0, 0.0};
     double *st = nullptr;
     if (in) {
         j = S.first ? i : S.lists_cur[list_off + i];
@@ -196,7 +197,8 @@ __device__ __forceinline__ void megno_chunk(const BatchSeg &S, ConstPtr<JobDesc>
         st = J->state + (size_t)j * kMegnoState;
 #pragma unroll
         for (int q = 0; q < 16; q++) m[q] = st[q];
-        l1 = st[16]; l2 = st[17]; fb2 = st[18];
+        sums = MegnoSums{st[16], st[17], st[18]};
+        if (S.first) sums.lh = half_log10(frob2_fused(m), log_tab);
     } else {
 #pragma unroll
         for (int q = 0; q < 16; q++) m[q] = 0.0;
@@ -228,10 +230,7 @@ __device__ __forceinline__ void megno_chunk(const BatchSeg &S, ConstPtr<JobDesc>
     bool pending = false;
     double w_prev = 0.0, inv_prev = 0.0;
     auto megno_update = [&]() {
-        const double fa2 = frob2_fused(m);
-        l1 = l1 + (0.5 * log10_fdl(fa2 / fb2)) * w_prev;
-        l2 = l2 + inv_prev * l1;
-        fb2 = fa2;
+        sums.add(half_log10_or_inf(frob2_fused(m), log_tab), w_prev, inv_prev);
         pending = false;
     };
     double xx = x * x, yy = y * y;  // carried between turns in exact mode
@@ -248,30 +247,35 @@ __device__ __forceinline__ void megno_chunk(const BatchSeg &S, ConstPtr<JobDesc>
             if (renorm_in) stop = min(stop, k + renorm_in - 1);
             if (stop > k) {
                 const bool alive_start = alive;
+                bool zero_m = false;  // settled when the run ends, as in k_indicators
                 TabEntry t = load_record(tp + k);
                 double inv_k = inv_idx[S.seg_start + k];
-                for (uint32_t kk = k; kk < stop; ++kk) {
-                    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): this turn's entries
-                    __builtin_amdgcn_sched_barrier(0);
-                    const uint32_t kn = min(kk + 1, turns - 1);
-                    const TabEntry tn = load_record(tp + kn);
-                    const double inv_n = inv_idx[S.seg_start + kn];
-                    {
-                        const double fa2 = frob2_fused(m);
-                        l1 = l1 + (0.5 * log10_fdl(fa2 / fb2)) * w_prev;
-                        l2 = l2 + inv_prev * l1;
-                        fb2 = fa2;
+                uint32_t k2 = k;  // two turns per pass, an odd last one left to the code below
+                for (; k2 + 2 <= stop; k2 += 2) {
+#pragma unroll
+                    for (uint32_t u = 0; u < 2; ++u) {
+                        const uint32_t kk = k2 + u;
+                        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): this turn's entries
+                        __builtin_amdgcn_sched_barrier(0);
+                        const uint32_t kn = min(kk + 1, turns - 1);
+                        const TabEntry tn = load_record(tp + kn);
+                        const double inv_n = inv_idx[S.seg_start + kn];
+                        const double f2 = frob2_fused(m);
+                        zero_m = zero_m | (f2 == 0.0);
+                        sums.add(half_log10(f2, log_tab), w_prev, inv_prev);
+                        const Jac jc = jac_coeffs<MODE>(x, y, mu3, mu6);
+                        mat_mul_structured<MODE>(jc, t, m);
+                        const bool out = forward_turn_out<MODE, OCT>(x, px, y, py, xx, yy, mu, m3mu, t, b2);
+                        done = (alive & out) ? kk : done;
+                        alive = alive & !out;
+                        w_prev = (double)(S.seg_start + kk + 1);
+                        inv_prev = inv_k;
+                        t = tn;
+                        inv_k = inv_n;
                     }
-                    const Jac jc = jac_coeffs<MODE>(x, y, mu3, mu6);
-                    mat_mul_structured<MODE>(jc, t, m);
-                    const bool out = forward_turn_out<MODE, OCT>(x, px, y, py, xx, yy, mu, m3mu, t, b2, b2s);
-                    done = (alive & out) ? kk : done;
-                    alive = alive & !out;
-                    w_prev = (double)(S.seg_start + kk + 1);
-                    inv_prev = inv_k;
-                    t = tn;
-                    inv_k = inv_n;
                 }
+                stop = k2;
+                if (zero_m) sums = MegnoSums{__builtin_nan(""), __builtin_nan(""), -HUGE_VAL};
                 if (alive_start && !alive) {
                     x = px = y = py = xx = yy = __builtin_nan("");
 #pragma unroll
@@ -316,7 +320,7 @@ __device__ __forceinline__ void megno_chunk(const BatchSeg &S, ConstPtr<JobDesc>
                 const double inv = 1.0 / fa;
 #pragma unroll
                 for (int q = 0; q < 16; q++) m[q] = m[q] * inv;
-                fb2 = frob2_fused(m);
+                sums.lh = half_log10_or_inf(frob2_fused(m), log_tab);
             }
         }
         if (!__any(alive || held)) break;
@@ -329,13 +333,13 @@ __device__ __forceinline__ void megno_chunk(const BatchSeg &S, ConstPtr<JobDesc>
     if (alive0 || held) {
 #pragma unroll
         for (int q = 0; q < 16; q++) st[q] = m[q];
-        st[16] = l1; st[17] = l2; st[18] = fb2;
+        st[16] = sums.l1; st[17] = sums.l2; st[18] = sums.lh;
     }
     // a particle leaves the live list when lost (or all NaN from the start):
     // its MEGNO is final then; survivors and held particles get theirs after
     // the job's last turn
     const bool keep = alive || held;
-    if (in && (!keep || last)) J->megno[j] = keep ? inv_idx[n_turns - 1] * l2 : __builtin_nan("");
+    if (in && (!keep || last)) J->megno[j] = keep ? inv_idx[n_turns - 1] * sums.l2 : __builtin_nan("");
     if (!last) {
         const uint64_t mlive = __ballot(keep);
         if (mlive) {
@@ -352,6 +356,8 @@ __device__ __forceinline__ void megno_chunk(const BatchSeg &S, ConstPtr<JobDesc>
 template <int MODE>
 __global__ void __launch_bounds__(256) k_batch_megno(BatchSeg S)
 {
+    __shared__ LogBin log_tab[kLogBins];
+    fill_log_bins(log_tab);
     const uint32_t lane = __lane_id();
     const ConstPtr<uint32_t> chunk_off = as_const(S.chunk_off);
     const ConstPtr<uint32_t> count_cur = as_const(S.count_cur);
@@ -372,8 +378,8 @@ __global__ void __launch_bounds__(256) k_batch_megno(BatchSeg S)
         const ConstPtr<JobDesc> J = jobs + job;
         const uint32_t n = S.first ? J->n : count_cur[job];
         const uint32_t base = (c - chunk_off[job]) * 64u;
-        if (J->mu != 0.0) megno_chunk<MODE, true>(S, J, job, base, n);
-        else megno_chunk<MODE, false>(S, J, job, base, n);
+        if (J->mu != 0.0) megno_chunk<MODE, true>(S, J, job, base, n, log_tab);
+        else megno_chunk<MODE, false>(S, J, job, base, n, log_tab);
     }
 }
 

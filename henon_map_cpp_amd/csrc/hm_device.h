@@ -217,18 +217,16 @@ __device__ __forceinline__ bool forward_turn_lost(double &x, double &px, double 
     return !(radius2<kFast>(x, px, y, py) < b2);
 }
 
-// forward_turn_lost without branches: both radius tests are evaluated (exact
-// mode: the screen, then the reference's expression), so a plain turn stays one
-// basic block. Same decisions as forward_turn_lost.
+// forward_turn_lost without branches, so a plain turn stays one basic block: the
+// reference's expression alone (the screen would only add to it). Same decisions
+// as forward_turn_lost.
 template <int MODE, bool OCT>
 __device__ __forceinline__ bool forward_turn_out(double &x, double &px, double &y, double &py, double &xx, double &yy,
-                                                 double mu, double m3mu, const TabEntry &t, double b2, double b2s)
+                                                 double mu, double m3mu, const TabEntry &t, double b2)
 {
     if (MODE == kExact) {
-        const double r2 = fwd_exact_carry<OCT>(x, px, y, py, xx, yy, mu, t);
-        const bool screen = !(r2 < b2s);
-        const bool out = !(exact_radius2(xx, px, yy, py) < b2);
-        return screen & out;
+        (void)fwd_exact_carry<OCT>(x, px, y, py, xx, yy, mu, t);
+        return !(exact_radius2(xx, px, yy, py) < b2);
     }
     map_step<kFast, false, OCT>(x, px, y, py, mu, m3mu, t);
     return !(radius2<kFast>(x, px, y, py) < b2);
@@ -252,16 +250,17 @@ __device__ __forceinline__ Jac jac_coeffs(double x, double y, double mu3, double
 {
     Jac j;
     if (MODE == kExact) {
-        j.a = ((2.0 * x) + ((mu3 * x) * x)) - ((mu3 * y) * y);
-        j.b = (-2.0 * y) - ((mu6 * x) * y);
-        // the reference evaluates the y-row term separately; equal to -a up to
-        // the sign of an exact zero
-        j.an = ((-2.0 * x) - ((mu3 * x) * x)) + ((mu3 * y) * y);
+        // ((2 x) + (mu3 x) x) - (mu3 y) y and (-2 y) - (mu6 x) y: doubling is
+        // exact, so fusing it into the sum leaves every rounding as it is. The
+        // reference evaluates the y-row term separately; it equals -a up to the
+        // sign of an exact zero.
+        j.a = fma(2.0, x, (mu3 * x) * x) - ((mu3 * y) * y);
+        j.b = fma(-2.0, y, -((mu6 * x) * y));
     } else {
         j.a = fma(mu3 * x, x, fma(-mu3 * y, y, 2.0 * x));
         j.b = fma(-mu6 * x, y, -2.0 * y);
-        j.an = -j.a;
     }
+    j.an = -j.a;
     return j;
 }
 

@@ -5,8 +5,35 @@
 #include <hip/hip_runtime.h>
 
 #include "hm_device.h"
+#include "hm_lognorm.h"
 
 namespace hm {
+
+// Fills a workgroup's table of half_log10 in LDS; every thread takes part.
+__device__ __forceinline__ void fill_log_bins(LogBin *tab)
+{
+    for (int q = threadIdx.x; q < kLogBins; q += blockDim.x) tab[q] = log_bin(q);
+    __syncthreads();
+}
+
+// The MEGNO recursion of one add (src/henon.cu:2259-2283) in the form of norms'
+// logarithms: L1 += (log10|M_{k+1}| - log10|M_k|) idx, L2 += L1 / idx.
+struct MegnoSums {
+    double l1, l2, lh;  // lh = log10|M| before the add
+    __device__ __forceinline__ void add(double lh_new, double idx, double inv_idx)
+    {
+        l1 = fma(lh_new - lh, idx, l1);
+        l2 = fma(inv_idx, l1, l2);
+        lh = lh_new;
+    }
+};
+
+// half_log10 with log10(0) = -inf.
+__device__ __forceinline__ double half_log10_or_inf(double F, const LogBin *tab)
+{
+    const double v = half_log10(F, tab);
+    return F == 0.0 ? -HUGE_VAL : v;
+}
 
 // M <- J M with J's structure: rows 0-1 touch M rows 0,1,2; rows 2-3 M rows 0,2,3.
 template <int MODE>

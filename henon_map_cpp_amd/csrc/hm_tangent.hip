@@ -159,7 +159,7 @@ struct IndicatorArgs {
     uint32_t first, last;
 };
 
-// Per-particle state between segments: M (16), log10 scale, L1, L2, |M|_F^2;
+// Per-particle state between segments: M (16), log10 scale, L1, L2, log10|M|_F;
 // with Birkhoff windows the last angles (2) and the window sums (2 per window);
 // with construct windows the megno_birkhoff sums (1 per window), the
 // tune_birkhoff sums (4 per window) and their last angles (2).
@@ -172,12 +172,11 @@ constexpr int ind_state_len(int V) { return V == 2 ? kIndConsState + 5 * kMaxBir
 // One thread per particle; the table index of turn k is steps+k for both the
 // tangent matrix (evaluated at the pre-step point) and the step.
 //   MEGNO (construct form): with idx = k+1, L1 += log10(|M_{k+1}|_F / |M_k|_F) idx,
-//     L2 += L1 / idx; recorded at sample t as L2 / t. The ratio is evaluated as
-//     0.5 log10(|M_{k+1}|^2 / |M_k|^2) with fused squared norms (one division,
-//     no square root), the logarithm by log10_fdl (hm_log10.h: within 2 ulps
-//     of the library's, in about half its instructions) and 1/idx from a host
-//     table; the result agrees with the separate-rounding form to a few ulps
-//     per turn.
+//     L2 += L1 / idx; recorded at sample t as L2 / t. The ratio's logarithm is
+//     the difference of consecutive values of log10|M|, each taken once from the
+//     fused squared norm by a table in LDS (hm_lognorm.h; no division, no square
+//     root), 1/idx comes from a host table; the result agrees with the
+//     separate-rounding form to a few ulps per turn.
 //   FLI: log10(|M_t v0|) / t with v0 = fli_dir / |fli_dir|, including the
 //     log10 of the scale factored out by renormalisation.
 //   Renormalisation every renorm_every turns: M <- M / |M|_F, after the MEGNO
@@ -185,6 +184,11 @@ constexpr int ind_state_len(int V) { return V == 2 ? kIndConsState + 5 * kMaxBir
 //   Birkhoff windows (sample indices from < m <= to): acc += w[m-1-from] dtheta_m
 //     with dtheta wrapped into [0, 2pi) (dynamic_indicator.cpp:110-117); tune =
 //     1 - acc / 2pi (NaN once a sample of the window is NaN).
+// Bound by VALU issue: in exact mode 80 of the plain turn's instructions are the
+// unfused matrix product and 33 the unfused map. With the norm's logarithm from
+// the table instead of a ratio's, the loss test by the reference's expression
+// alone and two turns per pass of the loop, a plain turn is 180 instructions
+// (256 before): 131072 particles x 1e5 turns, whole call, 105.7 -> 80.1 ms.
 // Variants V: 0 MEGNO/FLI only; 1 with Birkhoff windows; 2 with any of the
 // trajectory window and the construct windows as well. Every variant runs the
 // straight runs of plain turns and loss-compaction segments (its sums kept in
@@ -214,6 +218,8 @@ __global__ void __launch_bounds__(256) k_indicators(IndicatorArgs a)
     constexpr bool EXTRA = V == 2, BW = V >= 1;
     constexpr int SL = ind_state_len(V);
     constexpr int MAP = map_mode(MODE), TAN = tangent_mode(MODE);
+    __shared__ LogBin log_tab[kLogBins];
+    fill_log_bins(log_tab);
     const uint32_t li = blockIdx.x * blockDim.x + threadIdx.x;  // position in the live list
     const uint32_t n_live = a.count_in ? *a.count_in : a.n;
     const bool in_range = li < n_live;
@@ -226,7 +232,8 @@ __global__ void __launch_bounds__(256) k_indicators(IndicatorArgs a)
         s = a.steps[i];
     }
     double m[16];
-    double lscale = 0.0, l1 = 0.0, l2 = 0.0, f0;
+    double lscale = 0.0;
+    MegnoSums sums{0.0, 0.0, 0.0};
     double bacc[kMaxBirk][2];
 #pragma unroll
     for (int w = 0; w < kMaxBirk; w++) bacc[w][0] = bacc[w][1] = 0.0;
@@ -235,7 +242,7 @@ __global__ void __launch_bounds__(256) k_indicators(IndicatorArgs a)
         const double *st = a.state + (size_t)i * SL;
 #pragma unroll
         for (int q = 0; q < 16; q++) m[q] = st[q];
-        lscale = st[16]; l1 = st[17]; l2 = st[18]; f0 = st[19];
+        lscale = st[16]; sums = MegnoSums{st[17], st[18], st[19]};
         if (BW && a.n_birk) {
             thx = st[kIndBirkState]; thy = st[kIndBirkState + 1];
 #pragma unroll
@@ -253,7 +260,7 @@ __global__ void __launch_bounds__(256) k_indicators(IndicatorArgs a)
             for (int q = 0; q < 16; q++) m[q] = (q % 5 == 0) ? 1.0 : 0.0;
         }
         lscale = (a.log_scale && in_range) ? a.log_scale[i] : 0.0;
-        f0 = frob2_fused(m);
+        sums.lh = half_log10_or_inf(frob2_fused(m), log_tab);
     }
     const double mu3 = a.mu * 3, mu6 = a.mu * 6, m3mu = -3.0 * a.mu;
     const bool alive0 = in_range && !any_nan(x, px, y, py);
@@ -267,13 +274,6 @@ __global__ void __launch_bounds__(256) k_indicators(IndicatorArgs a)
     if (held) s += k0;
     bool alive = alive0;
     uint32_t done = k1;  // the turn a particle is lost in (k1: survived the launch)
-    double v0[4];
-    {
-        const double nn = sqrt(((a.fli_dir[0] * a.fli_dir[0] + a.fli_dir[1] * a.fli_dir[1]) +
-                                a.fli_dir[2] * a.fli_dir[2]) + a.fli_dir[3] * a.fli_dir[3]);
-#pragma unroll
-        for (int q = 0; q < 4; q++) v0[q] = a.fli_dir[q] / nn;
-    }
     if (BW && a.n_birk && a.first) {
         thx = atan2(px, x);
         thy = atan2(py, y);
@@ -324,9 +324,6 @@ __global__ void __launch_bounds__(256) k_indicators(IndicatorArgs a)
     uint32_t next_sample = sample_q < a.n_samples ? a.samples[sample_q] : 0;
     uint32_t next_megno = next_sample;
     uint32_t k = k0;
-    // squared Frobenius norm of M before the turn; the MEGNO ratio
-    // |M_{k+1}|/|M_k| is taken as sqrt(fa2 / fb2): one division, no square root
-    double fb2 = f0;
     uint32_t renorm_in = a.renorm_every ? a.renorm_every - k0 % a.renorm_every : 0;
     double xx = x * x, yy = y * y;  // carried between turns in exact mode
     const double b2s = screen_bound(a.b2);
@@ -343,16 +340,13 @@ __global__ void __launch_bounds__(256) k_indicators(IndicatorArgs a)
 #pragma unroll
         for (int w = 0; w < kMaxBirk; w++)
             if (w < (int)a.n_mb && idx <= a.mb_T[w])
-                mbacc[w] = mbacc[w] + (l1 * a.birk_w[a.mb_off[w] + idx - 1]) * inv;
+                mbacc[w] = mbacc[w] + (sums.l1 * a.birk_w[a.mb_off[w] + idx - 1]) * inv;
     };
     auto megno_update = [&]() {
-        const double fa2 = frob2_fused(m);
-        l1 = l1 + (0.5 * log10_fdl(fa2 / fb2)) * w_prev;
-        l2 = l2 + inv_prev * l1;
-        fb2 = fa2;
+        sums.add(half_log10_or_inf(frob2_fused(m), log_tab), w_prev, inv_prev);
         if (EXTRA && a.n_mb) megno_birkhoff_turn(idx_prev, inv_prev);
         if (idx_prev == next_megno) {
-            if (in_range && a.megno) a.megno[(size_t)sample_m * a.n + i] = inv_prev * l2;
+            if (in_range && a.megno) a.megno[(size_t)sample_m * a.n + i] = inv_prev * sums.l2;
             ++sample_m;
             next_megno = sample_m < a.n_samples ? a.samples[sample_m] : 0;
         }
@@ -412,35 +406,48 @@ __global__ void __launch_bounds__(256) k_indicators(IndicatorArgs a)
                 // a particle lost in the run is marked (its loss turn kept) and
                 // set to NaN when the run ends: nothing reads it before that
                 const bool alive_start = alive;
+                bool zero_m = false;
+                // Two turns per pass of the loop where registers allow: the second
+                // reads the registers that the first wrote, where a loop of single
+                // turns copies the 22 doubles it carries (62 of its 240
+                // instructions). An odd last turn is left to the code below.
+                constexpr uint32_t U = V == 0 ? 2 : 1;
                 TabEntry t = load_record(tp + k);
                 double inv_k = inv_idx[k];
-                for (uint32_t kk = k; kk < stop; ++kk) {
-                    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): this turn's entries
-                    __builtin_amdgcn_sched_barrier(0);
-                    const uint32_t kn = min(kk + 1, k1 - 1);
-                    const TabEntry tn = load_record(tp + kn);
-                    const double inv_n = inv_idx[kn];
-                    {
-                        const double fa2 = frob2_fused(m);
-                        l1 = l1 + (0.5 * log10_fdl(fa2 / fb2)) * w_prev;
-                        l2 = l2 + inv_prev * l1;
-                        fb2 = fa2;
+                uint32_t k2 = k;
+                for (; k2 + U <= stop; k2 += U) {
+#pragma unroll
+                    for (uint32_t u = 0; u < U; ++u) {
+                        const uint32_t kk = k2 + u;
+                        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): this turn's entries
+                        __builtin_amdgcn_sched_barrier(0);
+                        const uint32_t kn = min(kk + 1, k1 - 1);
+                        const TabEntry tn = load_record(tp + kn);
+                        const double inv_n = inv_idx[kn];
+                        // a zero matrix (its log10 is -inf, the sums NaN from the
+                        // next turn on) is marked and settled when the run ends;
+                        // the construct windows take the sums turn by turn
+                        const double f2 = frob2_fused(m);
+                        zero_m = zero_m | (f2 == 0.0);
+                        sums.add(EXTRA ? half_log10_or_inf(f2, log_tab) : half_log10(f2, log_tab), w_prev, inv_prev);
+                        if (EXTRA && a.n_mb) megno_birkhoff_turn(idx_prev, inv_prev);
+                        const Jac jc = jac_coeffs<TAN>(x, y, mu3, mu6);
+                        mat_mul_structured<TAN>(jc, t, m);
+                        const bool out = forward_turn_out<MAP, OCT>(x, px, y, py, xx, yy, a.mu, m3mu, t, a.b2);
+                        done = (alive & out) ? kk : done;
+                        alive = alive & !out;
+                        if (BW && a.n_birk) birkhoff_turn(kk + 1);
+                        if (EXTRA && a.n_tb) tune_birkhoff_turn(kk + 1);
+                        if (EXTRA && a.hist_len && alive) hist_store(kk + 1, x, px, y, py);
+                        w_prev = (double)(kk + 1);
+                        inv_prev = inv_k;
+                        idx_prev = kk + 1;
+                        t = tn;
+                        inv_k = inv_n;
                     }
-                    if (EXTRA && a.n_mb) megno_birkhoff_turn(idx_prev, inv_prev);
-                    const Jac jc = jac_coeffs<TAN>(x, y, mu3, mu6);
-                    mat_mul_structured<TAN>(jc, t, m);
-                    const bool out = forward_turn_out<MAP, OCT>(x, px, y, py, xx, yy, a.mu, m3mu, t, a.b2, b2s);
-                    done = (alive & out) ? kk : done;
-                    alive = alive & !out;
-                    if (BW && a.n_birk) birkhoff_turn(kk + 1);
-                    if (EXTRA && a.n_tb) tune_birkhoff_turn(kk + 1);
-                    if (EXTRA && a.hist_len && alive) hist_store(kk + 1, x, px, y, py);
-                    w_prev = (double)(kk + 1);
-                    inv_prev = inv_k;
-                    idx_prev = kk + 1;
-                    t = tn;
-                    inv_k = inv_n;
                 }
+                stop = k2;
+                if (!EXTRA && zero_m) sums = MegnoSums{__builtin_nan(""), __builtin_nan(""), -HUGE_VAL};
                 if (alive_start && !alive) {
                     x = px = y = py = xx = yy = __builtin_nan("");
 #pragma unroll
@@ -489,7 +496,13 @@ __global__ void __launch_bounds__(256) k_indicators(IndicatorArgs a)
         if (idx == next_sample) {
             const size_t o = (size_t)sample_q * a.n + i;
             if (in_range && a.fli) {
-                double v[4];
+                // v0 = fli_dir / |fli_dir|, formed here: kept, it would cost eight
+                // registers throughout
+                const double nn = sqrt(((a.fli_dir[0] * a.fli_dir[0] + a.fli_dir[1] * a.fli_dir[1]) +
+                                        a.fli_dir[2] * a.fli_dir[2]) + a.fli_dir[3] * a.fli_dir[3]);
+                double v0[4], v[4];
+#pragma unroll
+                for (int q = 0; q < 4; q++) v0[q] = a.fli_dir[q] / nn;
 #pragma unroll
                 for (int r = 0; r < 4; r++)
                     v[r] = (((m[r * 4] * v0[0]) + (m[r * 4 + 1] * v0[1])) + (m[r * 4 + 2] * v0[2])) +
@@ -509,7 +522,7 @@ __global__ void __launch_bounds__(256) k_indicators(IndicatorArgs a)
 #pragma unroll
                 for (int q = 0; q < 16; q++) m[q] = m[q] * inv;
                 lscale = lscale + log10(fa);
-                fb2 = frob2_fused(m);
+                sums.lh = half_log10_or_inf(frob2_fused(m), log_tab);
             }
         }
         if (BW && a.n_birk) birkhoff_turn(idx);
@@ -542,7 +555,7 @@ __global__ void __launch_bounds__(256) k_indicators(IndicatorArgs a)
         double *st = a.state + (size_t)i * SL;
 #pragma unroll
         for (int q = 0; q < 16; q++) st[q] = m[q];
-        st[16] = lscale; st[17] = l1; st[18] = l2; st[19] = fb2;
+        st[16] = lscale; st[17] = sums.l1; st[18] = sums.l2; st[19] = sums.lh;
         if (BW && a.n_birk) {
             st[kIndBirkState] = thx; st[kIndBirkState + 1] = thy;
 #pragma unroll
