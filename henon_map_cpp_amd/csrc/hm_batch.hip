@@ -41,11 +41,11 @@ struct JobDesc {
     uint32_t *steps;
     const TabEntry *tab;
     uint32_t n, n_turns, tab_len, list_off;
-    double mu, b2;
+    double mu, b2, safe1;  // safe1: TrackArgs
     double *megno;    // MEGNO jobs: output [n]; NULL for tracking-only jobs
     double *state;    // MEGNO jobs: [n][kMegnoState] tangent matrix and sums
     uint32_t renorm;  // MEGNO jobs: renormalisation interval (0 = never)
-    uint32_t pad;
+    uint32_t oct;     // octupole_kind
 };
 
 // Per-particle state a MEGNO job carries from one segment to the next: the
@@ -163,11 +163,19 @@ __global__ void __launch_bounds__(256, 8) k_batch_track(BatchSeg S)
         const bool last = S.seg_start + S.seg_len >= n_turns;
         const double mu = J->mu;
         TrackArgs A{J->x, J->px, J->y, J->py, J->steps,
-                    S.first ? nullptr : S.lists_cur + list_off, nullptr, n, 0u,
-                    J->tab, J->tab_len, turns, mu, J->b2,
+                    S.first ? nullptr : S.lists_cur + list_off, nullptr, n,
+                    J->tab, J->tab_len, turns, mu, J->b2, J->safe1,
                     last ? nullptr : S.lists_next + list_off, last ? nullptr : S.count_next + job, S.status};
-        if (mu != 0.0) track_wave<MODE, false, true, 1>(A, base, n);
-        else track_wave<MODE, false, false, 1>(A, base, n);
+        const uint32_t oct = J->oct;
+        auto out = [&] {
+            ConstPtr<JobDesc> d = J;
+            asm volatile("" : "+s"(d));  // read again
+            return TrackOut{d->x, d->px, d->y, d->py, d->steps, last ? nullptr : S.lists_next + list_off,
+                            last ? nullptr : S.count_next + job};
+        };
+        if (oct == 0) track_wave<MODE, false, 0>(A, base, n, out);
+        else if (MODE == kExact && oct == 2) track_wave<MODE, false, 2>(A, base, n, out);
+        else track_wave<MODE, false, 1>(A, base, n, out);
     }
 }
 
@@ -495,6 +503,8 @@ void batch_run(const hm_job *jobs, size_t n_jobs, int mode, int block, int every
         d.list_off = (uint32_t)total_n;
         d.mu = j.mu;
         d.b2 = j.barrier * j.barrier;  // henon.cu:2717
+        d.safe1 = safe_radius2(j.barrier, j.mu);
+        d.oct = (uint32_t)octupole_kind(mode, j.mu);
         total_n += j.n;
         if (total_n > 0xffffffffull) throw Error(HM_ERR_ARG, "batch: more than 2^32 particles in total");
         max_turns = std::max(max_turns, d.n_turns);

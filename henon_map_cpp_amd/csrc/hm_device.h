@@ -115,6 +115,61 @@ __device__ __forceinline__ double fwd_exact_carry(double &x, double &px, double 
     return fma(px, px, xx) + fma(py, py, yy);
 }
 
+// Exact turns with every fused operation that leaves the roundings as they are:
+// -2 (x y) is the reference's (-2 x) y, and exact, so it joins the sum that takes
+// it; with OCT = 2, mu is a power of two, mu d is exact, and it joins its sum the
+// same way (OCT = 1: any mu, OCT = 0: none): 32 operations a turn, 30 with OCT = 2,
+// for 33. This fails only where x y or mu d leaves the normal range: for states
+// whose coordinates are all zero or at least kTinyCoord, with |mu| between 2^-64
+// and 2^64 for OCT = 2, no turn of an orbit comes near it (each plane's two
+// coordinates change by a matrix of determinant one, so rounding puts a floor of
+// about 2^-27 under how far they can shrink together, and a sum that cancels is
+// zero or at least 2^-106 of its terms). xx, yy: x*x, y*y of the point.
+constexpr double kTinyCoord = 0x1p-100;
+
+template <int OCT>
+__device__ __forceinline__ void fwd_exact_fused(double &x, double &px, double &y, double &py, double &xx,
+                                                double &yy, double mu, const TabEntry &t)
+{
+    px = px + (xx - yy);
+    py = fma(-2.0, x * y, py);
+    if (OCT) {
+        const double dx = (xx * x) - (((3.0 * y) * y) * x);
+        const double dy = (yy * y) - (((3.0 * x) * x) * y);
+        px = OCT == 2 ? fma(mu, dx, px) : px + mu * dx;
+        py = OCT == 2 ? fma(mu, dy, py) : py + mu * dy;
+    }
+    const double xt = x, pt = px, yt = y, qt = py;
+    x = (xt * t.cx) + (pt * t.sx);
+    px = ((-xt) * t.sx) + (pt * t.cx);
+    y = (yt * t.cy) + (qt * t.sy);
+    py = ((-yt) * t.sy) + (qt * t.cy);
+    xx = x * x;
+    yy = y * y;
+}
+
+// The inverse turn (inv_exact below) in the same way.
+template <int OCT>
+__device__ __forceinline__ void inv_exact_fused(double &x, double &px, double &y, double &py, double &xx,
+                                                double &yy, double mu, const TabEntry &t)
+{
+    const double xt = x, pt = px, yt = y, qt = py;
+    x = (xt * t.cx) - (pt * t.sx);
+    px = (xt * t.sx) + (pt * t.cx);
+    y = (yt * t.cy) - (qt * t.sy);
+    py = (yt * t.sy) + (qt * t.cy);
+    xx = x * x;
+    yy = y * y;
+    if (OCT) {
+        const double dx = (xx * x) - (((3.0 * y) * y) * x);
+        const double dy = (yy * y) - (((3.0 * x) * x) * y);
+        px = OCT == 2 ? fma(-mu, dx, px) : px - mu * dx;
+        py = OCT == 2 ? fma(-mu, dy, py) : py - mu * dy;
+    }
+    px = px - (xx - yy);
+    py = fma(2.0, x * y, py);
+}
+
 // Loss screening for the exact mode. The reference's radius
 // ((x^2 + px^2) + (y^2 + py^2)) (henon.cu:113-116) and the fused form
 // fma(px, px, x^2) + fma(py, py, y^2) each lie within 3 roundings (3 * 2^-53,

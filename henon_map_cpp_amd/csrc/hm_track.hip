@@ -16,25 +16,19 @@
 
 namespace hm {
 
-// Wavefront w owns 64*P consecutive list entries. In mixed mode (slots > 0,
-// exactly `slots` wavefronts launched) the first w2 wavefronts take two particles
-// per lane so that n particles fit in one resident round of wavefronts:
-// w2 = ceil((n - 64 slots) / 64) when n exceeds 64 slots.
-// RING: the table records come through a per-wavefront LDS ring instead of
-// scalar loads (the launch picks it when there are few wavefronts per SIMD).
-template <int MODE, bool INV, bool OCT, bool RING>
-__global__ void __launch_bounds__(256, RING ? 2 : 8) k_track(TrackArgs A)
+// Wavefront w owns 64 consecutive list entries.
+template <int MODE, bool INV, int OCT>
+__global__ void __launch_bounds__(256, 8) k_track(TrackArgs A)
 {
     const uint32_t n = A.count_in ? *A.count_in : A.n_arg;
-    const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-    uint32_t w2 = 0;
-    if (A.slots && n > 64u * A.slots) w2 = min((n - 64u * A.slots + 63u) / 64u, A.slots);
-    if (wave < w2) {
-        track_wave<MODE, INV, OCT, 2, RING>(A, wave * 128u, n);
-    } else {
-        const uint32_t base = w2 * 128u + (wave - w2) * 64u;
-        if (base < n) track_wave<MODE, INV, OCT, 1, RING>(A, base, n);
-    }
+    const uint32_t base = ((blockIdx.x * blockDim.x + threadIdx.x) >> 6) * 64u;
+    if (base >= n) return;
+    track_wave<MODE, INV, OCT>(A, base, n, [] {
+        // A, from the kernel's argument segment again
+        ConstPtr<TrackArgs> a = (ConstPtr<TrackArgs>)__builtin_amdgcn_kernarg_segment_ptr();
+        asm volatile("" : "+s"(a));
+        return TrackOut{a->gx, a->gpx, a->gy, a->gpy, a->gsteps, a->idx_out, a->count_out};
+    });
 }
 
 struct TrackLaunch {
@@ -44,59 +38,45 @@ struct TrackLaunch {
     uint32_t n_arg, grid_bound;  // exact count when count_in is NULL; upper bound of it otherwise
     const TabEntry *tab;
     uint32_t tab_len, n_turns;
-    double mu, b2;
+    double mu, b2, safe1;
     uint32_t *idx_out, *count_out;
-    int block;
-    uint32_t slots;  // resident wavefront slots of the device (0 = plain one-per-lane launch)
-    int staging;     // HM_STAGING_*: table records by scalar loads or through the LDS ring
-    uint32_t simds;  // SIMDs of the device (CUs x 4)
+    int block;  // 0: chosen per launch
 };
 
-// Automatic table staging: the LDS ring up to this many wavefronts per SIMD.
-static constexpr uint64_t kRingMaxWavesPerSimd = 2;
+static constexpr int kDefaultBlock = 256;
 
-template <int MODE, bool INV, bool OCT>
+template <int MODE, bool INV, int OCT>
 static void launch_track(const TrackLaunch &a, hipStream_t s)
 {
-    TrackArgs A{a.x, a.px, a.y, a.py, a.steps, a.idx_in, a.count_in, a.n_arg, 0u, a.tab, a.tab_len, a.n_turns,
-                a.mu, a.b2, a.idx_out, a.count_out, status_word()};
-    uint64_t waves = ((uint64_t)a.grid_bound + 63) / 64;
-    // mixed mode when one particle per lane would need more than one round of
-    // resident wavefronts and two per lane suffice
-    if (a.slots && waves > a.slots && (uint64_t)a.grid_bound <= 128ull * a.slots) {
-        A.slots = a.slots;
-        waves = a.slots;
-    }
-    const uint64_t grid = (waves * 64 + a.block - 1) / a.block;
+    TrackArgs A{a.x, a.px, a.y, a.py, a.steps, a.idx_in, a.count_in, a.n_arg, a.tab, a.tab_len, a.n_turns,
+                a.mu, a.b2, a.safe1, a.idx_out, a.count_out, status_word()};
+    const uint64_t waves = ((uint64_t)a.grid_bound + 63) / 64;
+    // Up to one wavefront per SIMD, workgroups of one wavefront: they spread over
+    // all CUs, where four of a workgroup would share one CU's scalar and
+    // instruction caches (1e4 turns of 1e4 particles, mu = 0.5: 0.93 ms against
+    // 1.16 ms; 65536 particles, one wavefront on every SIMD either way, 1.26
+    // against 1.27 ms, and no difference beyond).
+    const int block = a.block ? a.block : waves <= device_simds() ? 64 : kDefaultBlock;
+    const uint64_t grid = (waves * 64 + block - 1) / block;
     if (grid == 0) return;
-    const bool ring = a.staging == HM_STAGING_RING ||
-                      (a.staging == HM_STAGING_AUTO && waves <= (uint64_t)kRingMaxWavesPerSimd * a.simds);
     LaunchTimer timer("k_track", s);
-    if (ring) hipLaunchKernelGGL((k_track<MODE, INV, OCT, true>), dim3((uint32_t)grid), dim3(a.block), 0, s, A);
-    else hipLaunchKernelGGL((k_track<MODE, INV, OCT, false>), dim3((uint32_t)grid), dim3(a.block), 0, s, A);
+    hipLaunchKernelGGL((k_track<MODE, INV, OCT>), dim3((uint32_t)grid), dim3(block), 0, s, A);
     launch_check("k_track");
 }
 
 using TrackFn = void (*)(const TrackLaunch &, hipStream_t);
 
-static TrackFn pick_track(int mode, bool inv, bool oct)
+static TrackFn pick_track(int mode, bool inv, double mu)
 {
+    const int oct = octupole_kind(mode, mu);  // henon.cu:445-448: no octupole kick at mu = 0
     if (mode == kExact) {
-        if (inv) return oct ? launch_track<kExact, true, true> : launch_track<kExact, true, false>;
-        return oct ? launch_track<kExact, false, true> : launch_track<kExact, false, false>;
+        static constexpr TrackFn f[2][3] = {
+            {launch_track<kExact, false, 0>, launch_track<kExact, false, 1>, launch_track<kExact, false, 2>},
+            {launch_track<kExact, true, 0>, launch_track<kExact, true, 1>, launch_track<kExact, true, 2>}};
+        return f[inv][oct];
     }
-    if (inv) return oct ? launch_track<kFast, true, true> : launch_track<kFast, true, false>;
-    return oct ? launch_track<kFast, false, true> : launch_track<kFast, false, false>;
-}
-
-// Resident wavefront slots: CUs x 4 SIMDs x 8 wavefronts (the kernel keeps
-// its VGPRs within 64 so that 8 fit per SIMD).
-static uint32_t resident_slots()
-{
-    int dev = 0, cus = 0;
-    hip_check(hipGetDevice(&dev), "hipGetDevice");
-    hip_check(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev), "hipDeviceGetAttribute");
-    return (uint32_t)cus * 32u;
+    if (inv) return oct ? launch_track<kFast, true, 1> : launch_track<kFast, true, 0>;
+    return oct ? launch_track<kFast, false, 1> : launch_track<kFast, false, 0>;
 }
 
 // ---------------------------------------------------------------- observables
@@ -161,7 +141,6 @@ __global__ void k_tangent_matrix(const double *__restrict__ x, const double *__r
 
 using namespace hm;
 
-static constexpr int kDefaultBlock = 256;
 static constexpr int kDefaultCompactEvery = 1000;  // turns between compactions
 static constexpr uint32_t kFirstSegment = 125;     // first segments are short: fast losses go early
 
@@ -229,27 +208,24 @@ static bool prepare_track(double *x, double *px, double *y, double *py, uint32_t
     if (n > 0x7fffffffull || table_len > 0xffffffffull) throw Error(HM_ERR_ARG, w + ": size exceeds 2^31");
     hm_launch_cfg tuned{};
     if (!cfg && tuned_config(mode, mu != 0.0, n, &tuned)) cfg = &tuned;
-    const int block = cfg && cfg->block ? cfg->block : kDefaultBlock;
-    if (block < 64 || block > 256 || block % 64) throw Error(HM_ERR_ARG, w + ": block must be 64, 128, 192 or 256");
+    const int block = cfg ? cfg->block : 0;
+    if (block && (block < 64 || block > 256 || block % 64)) throw Error(HM_ERR_ARG, w + ": block must be 64, 128, 192 or 256");
     every = cfg && cfg->compact_every ? cfg->compact_every : kDefaultCompactEvery;
-    // 1: one particle per lane; 2: one or two (mixed launch). The default is
-    // one in exact mode and mixed in fast mode, the faster of the two for each
-    // on the 1000x1000-grid, 1e5-turn scan.
-    int pair_mode = cfg ? cfg->particles_per_lane : 0;
-    if (pair_mode < 0 || pair_mode > 2) throw Error(HM_ERR_ARG, w + ": particles_per_lane must be 0, 1 or 2");
-    if (pair_mode == 0) pair_mode = mode == HM_MODE_EXACT ? 1 : 2;
+    // particles_per_lane and table_staging are accepted for callers that set them:
+    // there is one way now, a particle per lane and records by scalar loads
+    const int per_lane = cfg ? cfg->particles_per_lane : 0;
+    if (per_lane < 0 || per_lane > 2) throw Error(HM_ERR_ARG, w + ": particles_per_lane must be 0, 1 or 2");
     a = TrackLaunch{};
     a.x = x; a.px = px; a.y = y; a.py = py; a.steps = steps;
     a.tab = reinterpret_cast<const TabEntry *>(table);
     a.tab_len = (uint32_t)table_len;
     a.mu = mu;
     a.b2 = barrier * barrier;  // henon.cu:2717, :3173
+    a.safe1 = safe_radius2(barrier, mu);
     a.block = block;
-    a.slots = pair_mode == 1 ? 0u : resident_slots();
-    a.staging = cfg ? cfg->table_staging : HM_STAGING_AUTO;
-    if (a.staging < HM_STAGING_AUTO || a.staging > HM_STAGING_RING)
+    const int staging = cfg ? cfg->table_staging : HM_STAGING_AUTO;
+    if (staging < HM_STAGING_AUTO || staging > HM_STAGING_RING)
         throw Error(HM_ERR_ARG, w + ": table_staging must be 0 (auto), 1 (scalar) or 2 (ring)");
-    a.simds = device_simds();
     return true;
 }
 
@@ -277,13 +253,12 @@ extern "C" int hm_track(double *x, double *px, double *y, double *py, uint32_t *
                            "track", a, every))
             return;
         hipStream_t s = as_stream(stream);
-        const bool oct = mu != 0.0;  // henon.cu:445-448
         const uint32_t N = (uint32_t)n;
 
         if (every < 0 || (uint32_t)every >= n_turns) {
             a.n_arg = a.grid_bound = N;
             a.n_turns = n_turns;
-            pick_track(mode, inverse != 0, oct)(a, s);
+            pick_track(mode, inverse != 0, mu)(a, s);
             return;
         }
         // Segments: kFirstSegment turns, doubling up to `every`. Survivors of a
@@ -320,7 +295,7 @@ extern "C" int hm_track(double *x, double *px, double *y, double *py, uint32_t *
                 a.grid_bound = (uint32_t)bound;
                 a.idx_out = last ? nullptr : (i % 2 ? lists + N : lists);
                 a.count_out = last ? nullptr : counts + i + 1;
-                pick_track(mode, inverse != 0, oct)(a, s);
+                pick_track(mode, inverse != 0, mu)(a, s);
                 if (!last) {
                     hip_check(hipMemcpyAsync(host + i + 1, counts + i + 1, sizeof(uint32_t), hipMemcpyDeviceToHost, s),
                               "hipMemcpyAsync");
@@ -385,9 +360,8 @@ extern "C" int hm_track_noalloc(double *x, double *px, double *y, double *py, ui
                            "track_noalloc", a, every))
             return;
         hipStream_t s = as_stream(stream);
-        const bool oct = mu != 0.0;
         const uint32_t N = (uint32_t)n;
-        const TrackFn launch = pick_track(mode, inverse != 0, oct);
+        const TrackFn launch = pick_track(mode, inverse != 0, mu);
         if (every < 0 || (uint32_t)every >= n_turns) {
             a.n_arg = a.grid_bound = N;
             a.n_turns = n_turns;
@@ -458,7 +432,7 @@ extern "C" int hm_autotune_track(const double *x, const double *px, const double
         hip_check(hipMemcpyAsync(ws, steps, n * sizeof(uint32_t), hipMemcpyDeviceToDevice, s), "hipMemcpyAsync");
         const double nan = std::nan("");
         hm_launch_cfg base{};
-        base.particles_per_lane = mode == HM_MODE_EXACT ? 1 : 2;
+        base.particles_per_lane = 1;
         if (warm_turns) {
             const int rc = hm_track(w[0], w[1], w[2], w[3], ws, n, table, table_len, warm_turns, mu, barrier, nan, 0,
                                     mode, &base, stream);
@@ -473,21 +447,21 @@ extern "C" int hm_autotune_track(const double *x, const double *px, const double
         try {
             for (int block : {64, 256})
                 for (int every : {500, 1000, 2000})
-                    for (int pair : {1, 2}) {
-                        hm_launch_cfg c{block, every, pair, 0};
-                        hip_check(hipMemcpyAsync(work, warm, state, hipMemcpyDeviceToDevice, s), "hipMemcpyAsync");
-                        hip_check(hipEventRecord(e0, s), "hipEventRecord");
-                        const int rc = hm_track(w[0], w[1], w[2], w[3], ws, n, table, table_len, trial_turns, mu,
-                                                barrier, nan, 0, mode, &c, stream);
-                        if (rc != HM_OK) throw Error(rc, hm_last_error());
-                        hip_check(hipEventRecord(e1, s), "hipEventRecord");
-                        hip_check(hipEventSynchronize(e1), "hipEventSynchronize");
-                        float ms = 0.0f;
-                        hip_check(hipEventElapsedTime(&ms, e0, e1), "hipEventElapsedTime");
-                        if (best_t < 0.0f || ms < best_t) {
-                            best_t = ms;
-                            best_c = c;
-                        }
+                {
+                    hm_launch_cfg c{block, every, 1, 0};
+                    hip_check(hipMemcpyAsync(work, warm, state, hipMemcpyDeviceToDevice, s), "hipMemcpyAsync");
+                    hip_check(hipEventRecord(e0, s), "hipEventRecord");
+                    const int rc = hm_track(w[0], w[1], w[2], w[3], ws, n, table, table_len, trial_turns, mu,
+                                            barrier, nan, 0, mode, &c, stream);
+                    if (rc != HM_OK) throw Error(rc, hm_last_error());
+                    hip_check(hipEventRecord(e1, s), "hipEventRecord");
+                    hip_check(hipEventSynchronize(e1), "hipEventSynchronize");
+                    float ms = 0.0f;
+                    hip_check(hipEventElapsedTime(&ms, e0, e1), "hipEventElapsedTime");
+                    if (best_t < 0.0f || ms < best_t) {
+                        best_t = ms;
+                        best_c = c;
+                    }
                     }
         } catch (...) {
             (void)hipEventDestroy(e0);

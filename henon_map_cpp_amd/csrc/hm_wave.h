@@ -5,6 +5,7 @@
 // src/henon.cu:636-691 / :3155-3185 and the host loop :2701-2752.
 #pragma once
 #include <hip/hip_runtime.h>
+#include <cmath>
 #include <cstdint>
 
 #include "hm_device.h"
@@ -13,6 +14,12 @@ namespace hm {
 
 constexpr uint32_t kFlagRange = 1u;
 
+// Lanes whose v is not below s (NaN included), as a mask.
+__device__ __forceinline__ uint64_t not_below(double v, double s)
+{
+    constexpr int kUnorderedOrGE = 11;
+    return __builtin_amdgcn_fcmp(v, s, kUnorderedOrGE);
+}
 
 // Per-lane fallback used when the live lanes of a wavefront do not share one
 // turn index (particles reset while others were not) or when that index range
@@ -45,94 +52,95 @@ __device__ __forceinline__ void track_lanes(double &x, double &px, double &y, do
     }
 }
 
-// P particles per lane, n_turns turns in registers. Wavefront w owns the 64*P
-// consecutive entries [64*P*w, 64*P*(w+1)) of the particle list (or of the
-// live-index list `idx_in`), lane l the entries 64*q + l. The particle count is
-// read from device memory (`count_in`) when given, so a launch can be sized
-// from an upper bound without a host round trip.
+// One particle per lane, n_turns turns in registers. Wavefront w owns the 64
+// consecutive entries [64 w, 64 (w + 1)) of the particle list (or of the
+// live-index list `idx_in`). The particle count is read from device memory
+// (`count_in`) when given, so a launch can be sized from an upper bound without a
+// host round trip.
 //
 // The first live lane's turn index s0 is read into a scalar register; when every
 // live particle of the wavefront shares it (the normal case: all particles of a
 // tracker advance together), the table record of turn s0+k is the same for the
-// whole wavefront and is fetched with a scalar load, an iteration ahead, straight
-// into SGPR operands of the VALU ops. Losses are kept as wave-uniform lane masks,
-// so a turn costs the map's VALU ops plus one compare per particle.
+// whole wavefront and is fetched with a scalar load, ahead of its use, straight
+// into SGPR operands of the VALU ops. Losses are kept as wave-uniform lane masks.
 struct TrackArgs {
     double *gx, *gpx, *gy, *gpy;
     uint32_t *gsteps;
     const uint32_t *idx_in, *count_in;
     uint32_t n_arg;
-    uint32_t slots;  // wavefronts launched in mixed mode (0 = one particle per lane everywhere)
     const TabEntry *tab;
     uint32_t tab_len, n_turns;
     double mu, b2;
+    double safe1;  // squared radius below which the next turn cannot lose a point (safe_radius2)
     uint32_t *idx_out, *count_out, *status;
 };
 
-// LDS ring of the staged turn loop, per wavefront: 3 chunks of 8 records.
-constexpr int kTrackRingWave = 3 * 8 * 4;
-constexpr int kTrackRingWaves = 4;  // wavefronts per workgroup (at most 256 threads)
-
-template <int MODE, bool INV, bool OCT, int P, bool RING = false>
-__device__ __forceinline__ void track_wave(const TrackArgs &A, uint32_t base, uint32_t n)
+// How much of a turn's octupole kick is fused (fwd_exact_fused): 0 without
+// octupole, 2 in exact mode when mu is a power of two, else 1.
+inline int octupole_kind(int mode, double mu)
 {
-    double *__restrict__ gx = A.gx, *__restrict__ gpx = A.gpx, *__restrict__ gy = A.gy, *__restrict__ gpy = A.gpy;
-    uint32_t *__restrict__ gsteps = A.gsteps;
-    const uint32_t *__restrict__ idx_in = A.idx_in;
+    if (mu == 0.0) return 0;
+    if (mode != kExact) return 1;
+    int e = 0;
+    const double m = std::frexp(std::fabs(mu), &e);
+    return m == 0.5 && e >= -63 && e <= 65 ? 2 : 1;
+}
+
+// Squared radius R^2 such that a point with r < R is inside the barrier b and stays
+// inside for one turn of the map or of its inverse: the kick moves (px, py) by at
+// most rho^2 + |mu| rho^3, rho = |(x, y)| <= r, and the rotations keep r, so a turn
+// takes r to at most r + r^2 + |mu| r^3; R takes that to b, less a margin far above
+// the roundings. 0 (never inside) where no such radius exists.
+inline double safe_radius2(double barrier, double mu)
+{
+    const double m = std::fabs(mu), b = std::fmin(std::fabs(barrier), 1e100);
+    if (!(b > 0.0) || !(m < 1e100)) return 0.0;
+    double lo = 0.0, hi = b;
+    for (int i = 0; i < 1100; ++i) {
+        const double r = 0.5 * (lo + hi);
+        if (r <= lo || r >= hi) break;
+        (r + r * r + m * r * r * r < b ? lo : hi) = r;
+    }
+    lo *= 1.0 - 1e-6;
+    return lo * lo;
+}
+
+// What a wavefront writes at the end of its turns. Read again then (see
+// track_wave): kept through the turn loop, these pointers would take 14 of its
+// scalar registers.
+struct TrackOut {
+    double *gx, *gpx, *gy, *gpy;
+    uint32_t *gsteps, *idx_out, *count_out;
+};
+
+constexpr uint32_t kBlock = 8;  // turns per pass of the turn loop
+// out(): the TrackOut of this wavefront, called after the turns.
+template <int MODE, bool INV, int OCT, class Out>
+__device__ __forceinline__ void track_wave(const TrackArgs &A, uint32_t base, uint32_t n, Out out)
+{
+    constexpr bool EXACT = MODE == kExact;
     const TabEntry *__restrict__ tab = A.tab;
     const uint32_t tab_len = A.tab_len, n_turns = A.n_turns;
-    const double mu = A.mu, b2 = A.b2;
-    uint32_t *__restrict__ idx_out = A.idx_out;
-    uint32_t *__restrict__ count_out = A.count_out;
-    uint32_t *__restrict__ status = A.status;
-    const uint32_t lane = __lane_id();
-    double x[P], px[P], y[P], py[P];
-    uint32_t j[P], s[P], done[P];
-    bool alive0[P];
-    uint64_t live[P];
+    const double mu = A.mu, b2 = A.b2, m3mu = -3.0 * mu;
+    const uint32_t lane = __lane_id(), i = base + lane;
     const uint64_t my_bit = 1ull << lane;
-    uint64_t any_live = 0;
-#pragma unroll
-    for (int q = 0; q < P; ++q) {
-        const uint32_t i = base + 64u * q + lane;
-        const bool in_range = i < n;
-        j[q] = 0;
-        s[q] = 0;
-        x[q] = px[q] = y[q] = py[q] = __builtin_nan("");
-        if (in_range) {
-            j[q] = idx_in ? idx_in[i] : i;
-            x[q] = gx[j[q]];
-            px[q] = gpx[j[q]];
-            y[q] = gy[j[q]];
-            py[q] = gpy[j[q]];
-            s[q] = gsteps[j[q]];
-        }
-        // henon.cu:431-434: a particle with a NaN coordinate is not stepped
-        alive0[q] = in_range && !any_nan(x[q], px[q], y[q], py[q]);
-        live[q] = __ballot(alive0[q]);
-        any_live |= live[q];
-        done[q] = n_turns;
+    const bool in_range = i < n;
+    uint32_t j = 0, s = 0, done = n_turns;
+    double x = __builtin_nan(""), px = x, y = x, py = x;
+    if (in_range) {
+        j = A.idx_in ? A.idx_in[i] : i;
+        x = A.gx[j];
+        px = A.gpx[j];
+        y = A.gy[j];
+        py = A.gpy[j];
+        s = A.gsteps[j];
     }
-    if (!any_live) return;
-
-    const double m3mu = -3.0 * mu;
-    // turn index of the first live particle (q-major), and whether all share it
-    int qf = 0;
-#pragma unroll
-    for (int q = P - 1; q >= 0; --q)
-        if (live[q]) qf = q;
-    uint32_t sf = 0;
-#pragma unroll
-    for (int q = 0; q < P; ++q)
-        if (q == qf) sf = s[q];
-    uint64_t lf = 0;
-#pragma unroll
-    for (int q = 0; q < P; ++q)
-        if (q == qf) lf = live[q];
-    const uint32_t s0 = __builtin_amdgcn_readlane(sf, __builtin_ctzll(lf));
-    bool same = true;
-#pragma unroll
-    for (int q = 0; q < P; ++q) same = same && __all(!alive0[q] || s[q] == s0);
+    // henon.cu:431-434: a particle with a NaN coordinate is not stepped
+    const bool alive0 = in_range && !any_nan(x, px, y, py);
+    uint64_t live = __ballot(alive0);
+    if (!live) return;
+    const uint32_t s0 = __builtin_amdgcn_readlane(s, __builtin_ctzll(live));
+    const bool same = __all(!alive0 || s == s0);
     // forward reads records s0 .. s0+n_turns-1, inverse s0-1 down to s0-n_turns:
     // both ends must lie inside [0, tab_len), else the per-lane path flags it
     const bool in_table = INV ? (s0 >= n_turns && s0 <= tab_len) : ((uint64_t)s0 + n_turns <= (uint64_t)tab_len);
@@ -146,179 +154,139 @@ __device__ __forceinline__ void track_wave(const TrackArgs &A, uint32_t base, ui
             const ConstPtr<TabEntry> r = INV ? tp - k : tp + k;
             return load_record(r);
         };
-        // exact forward mode carries x*x, y*y from one turn to the next
-        constexpr bool CARRY = MODE == kExact && !INV;
-        double xx[P], yy[P];
-#pragma unroll
-        for (int q = 0; q < P; ++q) {
-            xx[q] = x[q] * x[q];
-            yy[q] = y[q] * y[q];
-        }
+        double xx = x * x, yy = y * y, r2 = 0.0;
         // exact mode screens losses with a fused radius (screen_radius2) and
         // confirms candidates with the reference's expression
-        constexpr bool SCREEN = MODE == kExact;
-        const double b2s = SCREEN ? screen_bound(b2) : b2;
-        double r2[P];
+        const double b2s = EXACT ? screen_bound(b2) : b2;
+        auto radius = [&] {
+            r2 = EXACT ? fma(px, px, xx) + fma(py, py, yy) : radius2<MODE>(x, px, y, py);
+        };
         auto turn = [&](const TabEntry &t) {
-#pragma unroll
-            for (int q = 0; q < P; ++q) {
-                if (CARRY) {
-                    r2[q] = fwd_exact_carry<OCT>(x[q], px[q], y[q], py[q], xx[q], yy[q], mu, t);
+            if (EXACT && INV) inv_exact_fused<OCT>(x, px, y, py, xx, yy, mu, t);
+            else if (EXACT) fwd_exact_fused<OCT>(x, px, y, py, xx, yy, mu, t);
+            else map_step<MODE, INV, OCT != 0>(x, px, y, py, mu, m3mu, t);
+        };
+        // The losses of turn kk (the exact confirmation, the loss turn, the live
+        // mask): the rare path of a checked turn.
+        auto settle = [&](uint32_t kk) {
+            uint64_t lost = live & not_below(r2, b2s);
+            if (EXACT && lost) lost &= not_below(exact_radius2(x * x, px, y * y, py), b2);
+            if (lost & my_bit) done = kk;
+            live &= ~lost;
+        };
+        auto checked = [&](const TabEntry &t, uint32_t kk) {
+            turn(t);
+            radius();
+            if (live & not_below(r2, b2s)) settle(kk);
+        };
+        // The fused forms need every coordinate zero or at least kTinyCoord.
+        bool plain = true;
+        if (EXACT) {
+            auto small = [](double v) { return v != 0.0 && fabs(v) < kTinyCoord; };
+            plain = !__any(alive0 && (small(x) || small(px) || small(y) || small(py)));
+        }
+        if (plain) {
+            // Turns go in pairs with one test: a point below safe1 after the first
+            // turn is inside the barrier after the second, whatever it is. (A record
+            // that is not finite takes every point out at once; if it was the
+            // untested turn's, the loss is that turn's.)
+            // A turn is then 30 to 32 operations and half a test (4 operations and a
+            // branch), where every turn had one: 1e6 particles on the 1000 x 1000
+            // grid, 3e4 turns, mu = 0.5: 22.0 -> 19.3 ms (exact), 15.9 -> 14.5 ms
+            // (fast).
+            uint32_t k = 0;
+            const double safe1 = A.safe1;
+            auto pair = [&](const TabEntry &t0, const TabEntry &t1, uint32_t kk) {
+                turn(t0);
+                radius();
+                if (__builtin_expect((live & not_below(r2, safe1)) == 0, 1)) {
+                    turn(t1);
                 } else {
-                    map_step<MODE, INV, OCT>(x[q], px[q], y[q], py[q], mu, m3mu, t);
-                    r2[q] = SCREEN ? screen_radius2(x[q], px[q], y[q], py[q]) : radius2<MODE>(x[q], px[q], y[q], py[q]);
-                }
-            }
-        };
-        // The common turn costs one compare and one scalar test per particle
-        // slot; everything about a loss (the exact confirmation, the loss turn,
-        // the live masks, the early exit) sits on the rare path `settle`, which
-        // returns false when no particle of the wavefront is left.
-        auto lost_mask = [&]() -> uint64_t {
-            uint64_t any = 0;
-#pragma unroll
-            for (int q = 0; q < P; ++q) any |= live[q] & ~__ballot(r2[q] < b2s);
-            return any;
-        };
-        auto settle = [&](uint32_t kk) -> bool {
-            uint64_t all = 0;
-#pragma unroll
-            for (int q = 0; q < P; ++q) {
-                uint64_t lost = live[q] & ~__ballot(r2[q] < b2s);
-                if (SCREEN && lost) {
-                    const double e = CARRY ? exact_radius2(xx[q], px[q], yy[q], py[q])
-                                           : exact_radius2(x[q] * x[q], px[q], y[q] * y[q], py[q]);
-                    lost &= ~__ballot(e < b2);
-                }
-                if (lost & my_bit) done[q] = kk;
-                live[q] &= ~lost;
-                all |= live[q];
-            }
-            return all != 0;
-        };
-        // Four turns per iteration in two halves: each half's two records are
-        // requested (one 64-byte scalar load, fixed offsets from a pointer that
-        // advances by four records) one half ahead, into the register pair the
-        // half before last used, so no register copies are needed. The last
-        // turns (fewer than four) go one by one. When the last particle is lost,
-        // the rare path ends the loop by shortening its count: the common path
-        // has no exit test of its own.
-        uint32_t k = 0;
-        bool any_live = true;
-        if constexpr (RING) {
-            // With few wavefronts per SIMD nothing hides a scalar load's latency
-            // (an L2 miss the first time a table is read): the wavefront stages
-            // the records of 8-turn chunks into its own LDS ring two chunks
-            // ahead (one vector load and one LDS store per lane and chunk) and
-            // reads each turn's record one turn ahead. Lanes 32..63 repeat
-            // lanes 0..31 (identical stores).
-            __shared__ __align__(16) double ring_all[kTrackRingWaves * kTrackRingWave];
-            double *const ring = ring_all + (threadIdx.x >> 6) * kTrackRingWave;
-            const double *tabd = reinterpret_cast<const double *>(tab);
-            const uint32_t G = (n_turns + 7) / 8;
-            auto clampg = [&](uint32_t g) { return g < G ? g : G - 1; };
-            auto stage_load = [&](uint32_t g) -> double {
-                const uint32_t kk = min(g * 8 + ((lane & 31) >> 2), n_turns - 1);
-                const uint32_t ti = INV ? s0 - 1 - kk : s0 + kk;
-                return tabd[4 * (size_t)ti + (lane & 3)];
-            };
-            auto stage_store = [&](uint32_t g, double e) { ring[(g % 3) * 32 + (lane & 31)] = e; };
-            auto ring_at = [&](uint32_t g, uint32_t m) -> TabEntry {
-                const double *q = ring + (g % 3) * 32 + m * 4;
-                return TabEntry{q[0], q[1], q[2], q[3]};
-            };
-            stage_store(0, stage_load(0));
-            stage_store(clampg(1), stage_load(clampg(1)));
-            double e = stage_load(clampg(2));
-            __builtin_amdgcn_wave_barrier();
-            TabEntry r = ring_at(0, 0);
-            for (uint32_t g = 0; g < G; ++g) {
-                stage_store(clampg(g + 2), e);
-                e = stage_load(clampg(g + 3));
-                __builtin_amdgcn_wave_barrier();  // the stores precede later chunks' reads
-                const uint32_t k0 = g * 8, len = min(8u, n_turns - k0);
-                if (len == 8) {
-#pragma unroll
-                    for (uint32_t m = 0; m < 8; ++m) {
-                        const TabEntry rn = m + 1 < 8 ? ring_at(g, m + 1) : ring_at(g + 1, 0);
-                        turn(r);
-                        if (lost_mask() && !settle(k0 + m)) any_live = false;
-                        r = rn;
+                    if (kk) {
+                        const TabEntry t = rec(kk - 1);
+                        const double z = 0.0 * ((t.sx + t.cx) + (t.sy + t.cy));
+                        settle(z == 0.0 ? kk : kk - 1);
+                    } else {
+                        settle(kk);
                     }
-                } else {
-                    for (uint32_t m = 0; m < len; ++m) {
-                        turn(ring_at(g, m));
-                        if (lost_mask() && !settle(k0 + m)) any_live = false;
+                    checked(t1, kk + 1);
+                }
+            };
+            if (n_turns >= kBlock) {
+                // Two pairs of records: while one pair's turns run, the other is
+                // requested (one 64-byte scalar load), into the registers the pair
+                // before last used.
+                const uint32_t last = n_turns - 2;
+                TabEntry a0 = rec(0), a1 = rec(1), b0, b1;
+                // Each lane touches a record 64 to 128 turns ahead, every 64 turns, so
+                // that scalar loads find the table in L2 also the first time it is
+                // read (64 particles, 1e4 turns: 0.89 ms warm or cold; without the
+                // touches 1.92 ms cold).
+                uint32_t touched = 0;
+                auto touch = [&](uint32_t from) {
+                    const uint32_t kk = min(from + lane, n_turns - 1);
+                    touched = *reinterpret_cast<const uint32_t *>(INV ? tab + (s0 - 1 - kk) : tab + (s0 + kk));
+                };
+                touch(0);
+                for (; k + kBlock <= n_turns && live; k += kBlock) {
+                    if (k % 64 == 0) {
+                        asm volatile("" ::"v"(touched));
+                        touch(k + 64);
+                    }
+#pragma unroll
+                    for (uint32_t q = 0; q < kBlock; q += 4) {
+                        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): a0, a1 are there
+                        __builtin_amdgcn_sched_barrier(0);
+                        b0 = rec(k + q + 2);
+                        b1 = rec(k + q + 3);
+                        __builtin_amdgcn_sched_barrier(0);
+                        pair(a0, a1, k + q);
+                        const uint32_t nx = min(k + q + 4, last);
+                        __builtin_amdgcn_s_waitcnt(0xC07F);
+                        __builtin_amdgcn_sched_barrier(0);
+                        a0 = rec(nx);
+                        a1 = rec(nx + 1);
+                        __builtin_amdgcn_sched_barrier(0);
+                        pair(b0, b1, k + q + 2);
                     }
                 }
-                if (!any_live) break;
+                radius();  // the last turn may have gone untested
+                if (live & not_below(r2, b2s)) settle(k - 1);
             }
-            k = n_turns;
-        } else if (n_turns >= 6) {
-            ConstPtr<TabEntry> p = tp;  // record of turn k (forward) / k-th back (inverse)
-            auto at = [&](int off) -> TabEntry {
-                const ConstPtr<TabEntry> r = INV ? p - off : p + off;
-                return load_record(r);
-            };
-            auto one = [&](const TabEntry &t, uint32_t kk, uint32_t &quads) {
-                turn(t);
-                if (lost_mask() && !settle(kk)) {
-                    any_live = false;
-                    quads = 1;
-                }
-            };
-            TabEntry a0 = at(0), a1 = at(1);
-            // turns k..k+3 use a0, a1, b0, b1; the next quad's a0, a1 (turns k+4,
-            // k+5) must exist, hence (n_turns - 2) / 4 quads
-            for (uint32_t quads = (n_turns - 2) / 4; quads; --quads) {
-                const TabEntry b0 = at(2), b1 = at(3);
-                one(a0, k, quads);
-                one(a1, k + 1, quads);
-                a0 = at(4);
-                a1 = at(5);
-                one(b0, k + 2, quads);
-                one(b1, k + 3, quads);
-                k += 4;
-                p = INV ? p - 4 : p + 4;
+            for (; live && k < n_turns; ++k) checked(rec(k), k);
+        } else {
+            // The reference's operations one by one and a test every turn.
+            TabEntry next = rec(0);
+            for (uint32_t k = 0; k < n_turns && live; ++k) {
+                const TabEntry t = next;
+                next = rec(min(k + 1, n_turns - 1));
+                map_step<MODE, INV, OCT != 0>(x, px, y, py, mu, m3mu, t);
+                r2 = screen_radius2(x, px, y, py);
+                if (live & not_below(r2, b2s)) settle(k);
             }
         }
-        for (; any_live && k < n_turns; ++k) {
-            turn(rec(k));
-            if (lost_mask()) any_live = settle(k);
-        }
-#pragma unroll
-        for (int q = 0; q < P; ++q)
-            if (alive0[q] && !(live[q] & my_bit)) x[q] = px[q] = y[q] = py[q] = __builtin_nan("");
+        if (alive0 && !(live & my_bit)) x = px = y = py = __builtin_nan("");
     } else if (n_turns > 0) {
-#pragma unroll
-        for (int q = 0; q < P; ++q) {
-            bool a = alive0[q];
-            track_lanes<MODE, INV, OCT>(x[q], px[q], y[q], py[q], a, done[q], s[q], tab, tab_len, n_turns, mu, b2,
-                                        status);
-            live[q] = __ballot(a);
-        }
+        bool a = alive0;
+        track_lanes<MODE, INV, OCT != 0>(x, px, y, py, a, done, s, tab, tab_len, n_turns, mu, b2, A.status);
+        live = __ballot(a);
     }
 
-#pragma unroll
-    for (int q = 0; q < P; ++q) {
-        if (alive0[q]) {
-            gx[j[q]] = x[q];
-            gpx[j[q]] = px[q];
-            gy[j[q]] = y[q];
-            gpy[j[q]] = py[q];
-            gsteps[j[q]] = INV ? s[q] - done[q] : s[q] + done[q];
-        }
-        if (idx_out) {
-            // wavefront-aggregated append of the survivors to the next live list
-            const uint64_t m = live[q];
-            if (m) {
-                const int leader = __builtin_ctzll(m);
-                uint32_t slot = 0;
-                if ((int)lane == leader) slot = atomicAdd(count_out, (uint32_t)__popcll(m));
-                slot = __builtin_amdgcn_readlane(slot, leader);
-                if (m & my_bit) idx_out[slot + __popcll(m & (my_bit - 1ull))] = j[q];
-            }
-        }
+    const TrackOut o = out();
+    if (alive0) {
+        o.gx[j] = x;
+        o.gpx[j] = px;
+        o.gy[j] = y;
+        o.gpy[j] = py;
+        o.gsteps[j] = INV ? s - done : s + done;
+    }
+    if (o.idx_out && live) {
+        // wavefront-aggregated append of the survivors to the next live list
+        const int leader = __builtin_ctzll(live);
+        uint32_t slot = 0;
+        if ((int)lane == leader) slot = atomicAdd(o.count_out, (uint32_t)__popcll(live));
+        slot = __builtin_amdgcn_readlane(slot, leader);
+        if (live & my_bit) o.idx_out[slot + __popcll(live & (my_bit - 1ull))] = j;
     }
 }
 

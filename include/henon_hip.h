@@ -14,7 +14,10 @@
  * Layouts in HBM
  *   particles : structure of arrays, x, px, y, py (double[n]) and steps (uint32[n])
  *   table     : one 32-byte record per turn, {sin wx(n), cos wx(n), sin wy(n), cos wy(n)}
- *               (double[turns][4]); built on the host by hm_build_table
+ *               (double[turns][4]); built on the host by hm_build_table. The kernels
+ *               count on each pair being the sine and cosine of one angle (or not
+ *               finite): a point well inside the barrier is not tested for loss
+ *               after a turn that cannot take it out
  *   matrices  : double[n][16], row-major 4x4 per particle (the reference's layout)
  *
  * Each declaration names the reference interface it replaces (paths relative to
@@ -101,18 +104,14 @@ int hm_birkhoff_weights(uint32_t n_weights, double *out);
 /* ---- tracking ------------------------------------------------------------ */
 /* Launch configuration; zero fields take the tuned defaults. */
 typedef struct hm_launch_cfg {
-    int32_t block;              /* threads per workgroup: 64, 128, 192 or 256 (0 = 256) */
+    int32_t block;              /* threads per workgroup: 64, 128, 192 or 256 (0 = 64 up to one
+                                   wavefront per SIMD, 256 beyond) */
     int32_t compact_every;      /* turns between loss compactions (0 = 1000, <0 = never); segments
                                    start at 125 turns and double up to this */
-    int32_t particles_per_lane; /* 1 = one per lane; 2 = one, or two for the leading wavefronts
-                                   when the live particles exceed one round of resident
-                                   wavefronts; 0 = 1 in exact mode, 2 in fast mode */
-    int32_t table_staging;      /* how a wavefront reads the turn's table record: HM_STAGING_SCALAR
-                                   (scalar loads one half-quad ahead), HM_STAGING_RING (8-turn
-                                   chunks staged through a per-wavefront LDS ring), or
-                                   HM_STAGING_AUTO (0): the ring when a launch has at most 2
-                                   wavefronts per SIMD, where nothing else hides a scalar load's
-                                   latency */
+    int32_t particles_per_lane; /* 0, 1 or 2, for callers that set it: every launch takes one
+                                   particle per lane */
+    int32_t table_staging;      /* HM_STAGING_*, for callers that set it: table records always come
+                                   by scalar loads, touched ahead of time by vector loads */
 } hm_launch_cfg;
 enum { HM_STAGING_AUTO = 0, HM_STAGING_SCALAR = 1, HM_STAGING_RING = 2 };
 
@@ -168,10 +167,9 @@ int hm_track_kicked(double *x, double *px, double *y, double *py, uint32_t *step
                     int mode, uint64_t seed, uint64_t draw, void *stream);
 
 /* Autotuner (no reference counterpart). Times hm_track launch configurations
- * (block 64 / 256, compact_every 500 / 1000 / 2000, one or two particles per
- * lane) on a copy of the given particles: first warm_turns turns with the
- * defaults (so that the fast early losses are behind), then trial_turns turns
- * from that state per candidate. Returns the fastest configuration in *best
+ * (block 64 / 256, compact_every 500 / 1000 / 2000) on a copy of the given
+ * particles: first warm_turns turns with the defaults (so that the fast early
+ * losses are behind), then trial_turns turns from that state per candidate. Returns the fastest configuration in *best
  * (its trial time in *best_ms) and remembers it for this device, mode, mu != 0
  * and particle-count class (floor(log2 n)): hm_track with cfg == NULL uses the
  * remembered configuration. The caller's particles are not modified; every
