@@ -15,6 +15,7 @@
 #include <type_traits>
 #include <vector>
 
+#include "hm_angle.h"
 #include "hm_device.h"
 #include "hm_internal.h"
 #include "hm_tangent.h"
@@ -189,6 +190,13 @@ constexpr int ind_state_len(int V) { return V == 2 ? kIndConsState + 5 * kMaxBir
 // the table instead of a ratio's, the loss test by the reference's expression
 // alone and two turns per pass of the loop, a plain turn is 180 instructions
 // (256 before): 131072 particles x 1e5 turns, whole call, 105.7 -> 80.1 ms.
+// A call of few waves is bound by latency. Workgroups of 64 threads spread them over
+// the CUs and a vector load touches the records ahead, 65536 x 3000 without windows
+// 1.75 -> 1.73 ms (exact) and 1.37 -> 1.27 (fast), 4099 x 3000 1.46 -> 1.40. Turns with
+// Birkhoff windows take two angles, which are most of what the windows cost: by the
+// table (hm_angle.h) instead of the library, 4099 x 3000 with two windows 3.40 ->
+// 2.81 ms, 131072 x 5000 8.36 -> 7.37 (both exact). Weights read ahead into lanes or
+// scalar registers cost more instructions than the loads they hide.
 // Variants V: 0 MEGNO/FLI only; 1 with Birkhoff windows; 2 with any of the
 // trajectory window and the construct windows as well. Every variant runs the
 // straight runs of plain turns and loss-compaction segments (its sums kept in
@@ -219,6 +227,8 @@ __global__ void __launch_bounds__(256) k_indicators(IndicatorArgs a)
     constexpr int SL = ind_state_len(V);
     constexpr int MAP = map_mode(MODE), TAN = tangent_mode(MODE);
     __shared__ LogBin log_tab[kLogBins];
+    __shared__ double angle_tab[BW ? kAngleBins : 1];
+    if (BW) fill_angle_table(angle_tab);
     fill_log_bins(log_tab);
     const uint32_t li = blockIdx.x * blockDim.x + threadIdx.x;  // position in the live list
     const uint32_t n_live = a.count_in ? *a.count_in : a.n;
@@ -275,8 +285,8 @@ __global__ void __launch_bounds__(256) k_indicators(IndicatorArgs a)
     bool alive = alive0;
     uint32_t done = k1;  // the turn a particle is lost in (k1: survived the launch)
     if (BW && a.n_birk && a.first) {
-        thx = atan2(px, x);
-        thy = atan2(py, y);
+        thx = angle_of(px, x, angle_tab);
+        thy = angle_of(py, y, angle_tab);
     }
     // construct-form accumulators: megno_birkhoff L2_j, tune_birkhoff
     // (tune1 x, tune2 x, tune1 y, tune2 y)_j and the stored angles
@@ -299,8 +309,8 @@ __global__ void __launch_bounds__(256) k_indicators(IndicatorArgs a)
             ctx = st[5 * kMaxBirk];
             cty = st[5 * kMaxBirk + 1];
         } else if (a.n_tb) {
-            ctx = atan2(px, x);
-            cty = atan2(py, y);
+            ctx = angle_of(px, x, angle_tab);
+            cty = angle_of(py, y, angle_tab);
         }
     }
     if (EXTRA && a.first && in_range && a.hist_len && a.hist_from == 0) {
@@ -354,7 +364,7 @@ __global__ void __launch_bounds__(256) k_indicators(IndicatorArgs a)
     };
     // Birkhoff windows after turn idx - 1 (the sample idx is the state now)
     auto birkhoff_turn = [&](uint32_t idx) {
-        const double nx = atan2(px, x), ny = atan2(py, y);
+        const double nx = angle_of(px, x, angle_tab), ny = angle_of(py, y, angle_tab);
         double dx = nx - thx, dy = ny - thy;
         if (dx < 0.0) dx += 2.0 * M_PI;
         if (dy < 0.0) dy += 2.0 * M_PI;
@@ -371,7 +381,7 @@ __global__ void __launch_bounds__(256) k_indicators(IndicatorArgs a)
     };
     // tune_birkhoff_construct's add after turn idx - 1 (add index idx)
     auto tune_birkhoff_turn = [&](uint32_t idx) {
-        const double nx = atan2(px, x), ny = atan2(py, y);
+        const double nx = angle_of(px, x, angle_tab), ny = angle_of(py, y, angle_tab);
         double dx = nx - ctx, dy = ny - cty;
         dx = dx > 0 ? dx : dx + 2 * M_PI;
         dy = dy > 0 ? dy : dy + 2 * M_PI;
@@ -389,6 +399,17 @@ __global__ void __launch_bounds__(256) k_indicators(IndicatorArgs a)
             a.hist[base + 2 * n + i] = vy; a.hist[base + 3 * n + i] = vpy;
         }
     };
+    // Each lane touches a record 64 to 128 turns ahead, so that the scalar loads
+    // find a table in L2 that was not read before.
+    uint32_t touched = 0;
+    auto touch = [&](uint32_t from) {
+        asm volatile("" ::"v"(touched));
+        touched = *reinterpret_cast<const uint32_t *>(a.tab + s0 + (min(from + __lane_id(), k1 - 1) - k0));
+    };
+    if (uniform) {
+        touch(k0);
+        touch(k0 + 64);
+    }
     for (; k < k1; ++k) {
         if (uniform && pending) {
             // Plain turns up to the next event (an FLI sample at its turn, a
@@ -419,6 +440,7 @@ __global__ void __launch_bounds__(256) k_indicators(IndicatorArgs a)
 #pragma unroll
                     for (uint32_t u = 0; u < U; ++u) {
                         const uint32_t kk = k2 + u;
+                        if (u == 0 && (k2 - k0) % 64 < U) touch(k2 + 64);
                         __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): this turn's entries
                         __builtin_amdgcn_sched_barrier(0);
                         const uint32_t kn = min(kk + 1, k1 - 1);
@@ -469,6 +491,7 @@ __global__ void __launch_bounds__(256) k_indicators(IndicatorArgs a)
         if (pending) megno_update();
         TabEntry t;
         if (uniform) {
+            if ((k - k0) % 64 == 0) touch(k + 64);
             t = load_record(tp + k);
         } else {
             const uint64_t ti = (uint64_t)s + (k - k0);
@@ -595,7 +618,7 @@ __global__ void __launch_bounds__(256) k_indicators(IndicatorArgs a)
         // wavefront may have stopped early; the arrays hold the start)
         x = a.x[i]; px = a.px[i]; y = a.y[i]; py = a.py[i];
         if (a.n_tb) {
-            const double ax = atan2(px, x), ay = atan2(py, y);
+            const double ax = angle_of(px, x, angle_tab), ay = angle_of(py, y, angle_tab);
             double dx = ax - ax, dy = ay - ay;
             dx = dx > 0 ? dx : dx + 2 * M_PI;
             dy = dy > 0 ? dy : dy + 2 * M_PI;
@@ -816,6 +839,12 @@ using namespace hm;
 
 namespace {
 inline uint32_t grid_of(size_t n, uint32_t block = 256) { return (uint32_t)((n + block - 1) / block); }
+// Threads per workgroup of a kernel that runs its turns in registers: one
+// wavefront up to one wavefront per SIMD, so that they spread over all CUs and
+// share no CU's scalar and instruction caches (4099 particles x 3000 turns of
+// indicators 1.46 -> 1.40 ms; with more waves than that the larger group is no slower
+// and has fewer groups to start).
+inline uint32_t turn_block(size_t n) { return (n + 63) / 64 <= device_simds() ? 64 : 256; }
 
 void host_birkhoff_weights(uint32_t n, double *out)
 {
@@ -851,7 +880,8 @@ extern "C" int hm_megno_trace(double *x, double *px, double *y, double *py, uint
         a.m_in = matrix_in; a.m_out = matrix_out;
         hipStream_t s = as_stream(stream);
         LaunchTimer timer("k_megno_trace", s);
-        const dim3 g(grid_of(n)), b(256);
+        const uint32_t block = turn_block(n);
+        const dim3 g(grid_of(n, block)), b(block);
         if (inverse) {
             if (mu != 0.0) hipLaunchKernelGGL((k_megno_trace<true, true>), g, b, 0, s, a);
             else hipLaunchKernelGGL((k_megno_trace<false, true>), g, b, 0, s, a);
@@ -1009,7 +1039,8 @@ extern "C" int hm_track_indicators(double *x, double *px, double *y, double *py,
         a.k0 = 0;
         a.k1 = n_turns;
         if (n_turns <= kIndFirstSegment || n > 0x7fffffffull) {
-            hipLaunchKernelGGL(k, dim3(grid_of(n)), dim3(256), 0, s, a);
+            const uint32_t block = turn_block(n);
+            hipLaunchKernelGGL(k, dim3(grid_of(n, block)), dim3(block), 0, s, a);
             launch_check("k_indicators");
             return;
         }
@@ -1055,7 +1086,8 @@ extern "C" int hm_track_indicators(double *x, double *px, double *y, double *py,
                 a.count_out = last ? nullptr : counts + q + 1;
                 a.state = state;
                 if (bound > 0) {
-                    hipLaunchKernelGGL(k, dim3(grid_of(bound)), dim3(256), 0, s, a);
+                    const uint32_t block = turn_block(bound);
+                    hipLaunchKernelGGL(k, dim3(grid_of(bound, block)), dim3(block), 0, s, a);
                     launch_check("k_indicators");
                 }
                 if (!last) {
