@@ -39,6 +39,7 @@
 #include <complex>
 #include <cstdint>
 #include <cstdlib>
+#include <iterator>
 #include <map>
 #include <mutex>
 #include <vector>
@@ -97,10 +98,18 @@ template <int R>
 __device__ __forceinline__ constexpr double root_cos(int q)
 {
     if constexpr (R == 5) {
-        constexpr double c[3] = {1.0, 0.30901699437494742410, -0.80901699437494742410};
+        constexpr double c[3] = {1.0, 0.30901699437494742408, -0.80901699437494742410};
+        return c[q];
+    } else if constexpr (R == 7) {
+        constexpr double c[4] = {1.0, 0.62348980185873353053, -0.22252093395631440434, -0.90096886790241912632};
+        return c[q];
+    } else if constexpr (R == 11) {
+        constexpr double c[6] = {1.0, 0.84125353283118116886, 0.41541501300188642549, -0.14231483827328514046,
+                                 -0.65486073394528506413, -0.95949297361449738990};
         return c[q];
     } else {
-        constexpr double c[4] = {1.0, 0.62348980185873353053, -0.22252093395631440429, -0.90096886790241912624};
+        constexpr double c[7] = {1.0, 0.88545602565320989587, 0.56806474673115580249, 0.12053668025532305325,
+                                 -0.35460488704253562600, -0.74851074817110109868, -0.97094181742605202719};
         return c[q];
     }
 }
@@ -108,15 +117,23 @@ template <int R>
 __device__ __forceinline__ constexpr double root_sin(int q)
 {
     if constexpr (R == 5) {
-        constexpr double s[3] = {0.0, 0.95105651629515357212, 0.58778525229247312917};
+        constexpr double s[3] = {0.0, 0.95105651629515357211, 0.58778525229247312913};
+        return s[q];
+    } else if constexpr (R == 7) {
+        constexpr double s[4] = {0.0, 0.78183148246802980873, 0.97492791218182360698, 0.43388373911755812029};
+        return s[q];
+    } else if constexpr (R == 11) {
+        constexpr double s[6] = {0.0, 0.54064081745559758210, 0.90963199535451837142, 0.98982144188093273236,
+                                 0.75574957435425828370, 0.28173255684142969765};
         return s[q];
     } else {
-        constexpr double s[4] = {0.0, 0.78183148246802980871, 0.97492791218182360702, 0.43388373911755812048};
+        constexpr double s[7] = {0.0, 0.46472317204376854566, 0.82298386589365639458, 0.99270887409805399284,
+                                 0.93501624268541482345, 0.66312265824079520232, 0.23931566428755776695};
         return s[q];
     }
 }
 
-// Forward DFT of prime size R = 5, 7 from the pairs m, R - m: with
+// Forward DFT of prime size R = 5, 7, 11, 13 from the pairs m, R - m: with
 // a_m = v_m + v_{R-m}, b_m = v_m - v_{R-m} and t = 2 pi m k / R,
 //   X_k = v_0 + sum_m (a_m cos t - i b_m sin t),  X_{R-k} = v_0 + sum_m (a_m cos t + i b_m sin t)
 // (m, k = 1 .. (R-1)/2): (R-1) constants instead of (R-1)^2 products of roots.
@@ -154,10 +171,100 @@ __device__ __forceinline__ void dft_prime(Cplx *v)
 }
 
 template <int R>
+__device__ __forceinline__ void dft_any(Cplx *v);
+
+// 9 = 3 x 3 and 16 = 4 x 4: the inner DFTs over n1 of n = A n1 + n2, the roots
+// W_R^{n2 k1}, the outer DFTs over n2 (k = k1 + A k2).
+__device__ __forceinline__ void dft9(Cplx *v)
+{
+    // W_9^1, W_9^2, W_9^4
+    constexpr Cplx w1{0.76604444311897803519, -0.64278760968653932633}, w2{0.17364817766693034880, -0.98480775301220805940},
+        w4{-0.93969262078590838410, -0.34202014332566873297};
+    Cplx a[3][3];
+#pragma unroll
+    for (int n2 = 0; n2 < 3; ++n2) {
+#pragma unroll
+        for (int n1 = 0; n1 < 3; ++n1) a[n2][n1] = v[3 * n1 + n2];
+        dft3(a[n2]);
+    }
+    a[1][1] = cmul(a[1][1], w1);
+    a[1][2] = cmul(a[1][2], w2);
+    a[2][1] = cmul(a[2][1], w2);
+    a[2][2] = cmul(a[2][2], w4);
+#pragma unroll
+    for (int k1 = 0; k1 < 3; ++k1) {
+        Cplx b[3] = {a[0][k1], a[1][k1], a[2][k1]};
+        dft3(b);
+#pragma unroll
+        for (int k2 = 0; k2 < 3; ++k2) v[k1 + 3 * k2] = b[k2];
+    }
+}
+__device__ __forceinline__ void dft16(Cplx *v)
+{
+    constexpr double c1 = 0.92387953251128675610, s1 = 0.38268343236508977172, h = 0.70710678118654752440;
+    Cplx a[4][4];
+#pragma unroll
+    for (int n2 = 0; n2 < 4; ++n2) {
+#pragma unroll
+        for (int n1 = 0; n1 < 4; ++n1) a[n2][n1] = v[4 * n1 + n2];
+        dft4(a[n2][0], a[n2][1], a[n2][2], a[n2][3]);
+    }
+    // W_16^q: q = 1, 2, 3 (n2 = 1), 2, 4, 6 (n2 = 2), 3, 6, 9 (n2 = 3)
+    a[1][1] = cmul(a[1][1], Cplx{c1, -s1});
+    a[1][2] = Cplx{h * (a[1][2].re + a[1][2].im), h * (a[1][2].im - a[1][2].re)};
+    a[1][3] = cmul(a[1][3], Cplx{s1, -c1});
+    a[2][1] = Cplx{h * (a[2][1].re + a[2][1].im), h * (a[2][1].im - a[2][1].re)};
+    a[2][2] = mul_mi(a[2][2]);
+    a[2][3] = Cplx{h * (a[2][3].im - a[2][3].re), -h * (a[2][3].re + a[2][3].im)};
+    a[3][1] = cmul(a[3][1], Cplx{s1, -c1});
+    a[3][2] = Cplx{h * (a[3][2].im - a[3][2].re), -h * (a[3][2].re + a[3][2].im)};
+    a[3][3] = cmul(a[3][3], Cplx{-c1, s1});
+#pragma unroll
+    for (int k1 = 0; k1 < 4; ++k1) {
+        dft4(a[0][k1], a[1][k1], a[2][k1], a[3][k1]);
+#pragma unroll
+        for (int k2 = 0; k2 < 4; ++k2) v[k1 + 4 * k2] = a[k2][k1];
+    }
+}
+
+// R = A B with coprime factors: n = (B n1 + A n2) mod R, k the number with
+// k mod A = k1 and k mod B = k2; no roots between the two steps.
+template <int A, int B>
+__device__ __forceinline__ void dft_coprime(Cplx *v)
+{
+    constexpr int R = A * B;
+    Cplx t[B][A];
+#pragma unroll
+    for (int n2 = 0; n2 < B; ++n2) {
+#pragma unroll
+        for (int n1 = 0; n1 < A; ++n1) t[n2][n1] = v[(B * n1 + A * n2) % R];
+        dft_any<A>(t[n2]);
+    }
+#pragma unroll
+    for (int k1 = 0; k1 < A; ++k1) {
+        Cplx b[B];
+#pragma unroll
+        for (int n2 = 0; n2 < B; ++n2) b[n2] = t[n2][k1];
+        dft_any<B>(b);
+#pragma unroll
+        for (int k2 = 0; k2 < B; ++k2) {
+            int k = k1;
+            while (k % B != k2) k += A;
+            v[k] = b[k2];
+        }
+    }
+}
+
+template <int R>
 __device__ __forceinline__ void dft_any(Cplx *v)
 {
     if constexpr (R == 2 || R == 4 || R == 8) dft_r<R>(v);
     else if constexpr (R == 3) dft3(v);
+    else if constexpr (R == 6) dft_coprime<2, 3>(v);
+    else if constexpr (R == 9) dft9(v);
+    else if constexpr (R == 10) dft_coprime<2, 5>(v);
+    else if constexpr (R == 12) dft_coprime<4, 3>(v);
+    else if constexpr (R == 16) dft16(v);
     else dft_prime<R>(v);
 }
 
@@ -417,24 +524,41 @@ __global__ void __launch_bounds__(kMrThreads) k_mr_tune(MrArgs a)
 // in 160 KiB) runs in one kernel, one workgroup per signal: the samples are
 // read once, every pass runs in LDS and the tune is found there, with no
 // scratch in HBM and no second launch.
-//   direct : lengths whose prime factors are 2, 3, 5, 7 (the radix passes above)
-//            or other primes up to kWhPrimeMax (one prime-size pass each, below)
+//   direct : lengths whose prime factors are 2 to 13 (passes of radix 2 to 13 and
+//            16 in registers) or other primes up to kWhPrimeMax (one pass each,
+//            on the matrix cores where it fits them)
 //   chirp-z: other lengths N, over a smooth M >= 2N - 1 that fits: the chirped
 //            samples, FFT_M, times B = DFT_M(conj(c)), conjugated, FFT_M again;
 //            |X_k| = |V_k| / M for k < N (the scale does not change the tune)
 // The signal sits in LDS unpadded: the first pass takes an odd radix where the
 // length has an odd factor, so its stores step by an odd number of 16-byte
 // entries, and the later passes store runs of consecutive entries (a power of
-// two, here only as a chirp-z length, pays some bank conflicts in its first
-// pass).
+// two pays some bank conflicts in its first pass).
+// At 10^4 points one workgroup has the CU to itself and runs the phases one after
+// the other, in cycles: the load 15000 (12000 with the chip idle: the CU's own way
+// to L2), a radix-10 pass 6000 (320 KB through LDS 2500, 60 FP64 instructions per
+// point and wavefront 3700), the maximum and the tune 7000. 10000 points as 10^4
+// instead of 5^4 x 2 x 8, twiddles read in order instead of strided through one
+// table (64 cache lines an instruction) and one square root a signal instead of
+// one an entry: 129 -> 86 ns per signal; 500 points (10 x 10 x 5, one wavefront)
+// 7.7 -> 3.1, 501 (chirp-z over 7 x 9 x 16 instead of 3 x 3 x 7 x 2 x 8) 16.3 -> 10.6.
+// The shapes of k_wh_tune: 64, 128 .. kWhThreads threads for up to ten points a
+// thread (a butterfly of the radix-10 passes each, every wavefront at work; 16
+// wavefronts and up to 160 KiB of signals per CU in every shape).
+constexpr uint32_t kWhThreads = 1024, kWhPoints = 10, kWhPmax = kWhPoints * kWhThreads;
 constexpr uint32_t kWhPrimeMax = 257;
 constexpr int kWhMaxPasses = 16;
 
-// One pass: radix R after the radices of product Ns, B = L / R butterflies,
-// twiddle stride step = L / (Ns R); m_* are the multipliers of udiv_m for Ns,
-// H = (R - 1) / 2 and H + 1.
+// One pass: radix R after the radices of product Ns, B = L / R butterflies; tw =
+// where its twiddles start in the plan's table, in the order that the butterflies
+// read them (k = 0 .. Ns - 1 of W_{Ns R}^k, or for a prime pass the rows r = 1 ..
+// R - 1 of W_{Ns R}^{r k}; none if Ns = 1); m_* are the multipliers of udiv_m for
+// Ns, B and (R + 1) / 2; frag = where the root matrix of a matrix pass starts in
+// the plan's (kNoFrag: another pass), root = where W_R^q of another prime pass
+// starts in the table.
+constexpr uint32_t kNoFrag = 0xffffffffu;
 struct WhPass {
-    uint32_t R, Ns, B, step, m_ns, m_h, m_h1;
+    uint32_t R, Ns, B, tw, m_ns, m_b, m_h1, frag, root;
 };
 struct WhPlan {
     uint32_t L, n_pass;
@@ -453,22 +577,25 @@ struct WhArgs {
     uint32_t n, p0, from, N, M;
     WhPlan plan;          // passes of the M-point transform
     const double *hann;   // [N]
-    const Cplx *tw;       // W_M^q, q < M
+    const Cplx *tw;       // the passes' twiddles
+    const Cplx *frag;     // the root matrices of the matrix passes
     const Cplx *chirp;    // chirp-z: [N]
     const Cplx *bhat;     // chirp-z: [M], B in natural order
     double *out;          // [window][plane][n]
     uint32_t window;
+    double cos_n, sin_n;  // of 2 pi / N
 };
 
-
 // One radix-R Stockham pass (as mr_pass) over the whole signal of length L:
-// butterfly j reads x[j + r L/R], twiddles by W_L^{k r L/(Ns R)} (k = j mod
-// Ns), takes the R-point DFT and writes element r to (j - k) R + k + r Ns.
+// butterfly j reads x[j + r L/R], twiddles by W_{Ns R}^{k r} (k = j mod Ns; one
+// load, neighbours from neighbours, the powers by products), takes the R-point
+// DFT and writes element r to (j - k) R + k + r Ns.
 template <int R, uint32_t NT, uint32_t PMAX>
-__device__ __forceinline__ void wh_pass(Cplx *buf, const WhPass &ps, const Cplx *__restrict__ tw)
+__device__ __forceinline__ void wh_pass(Cplx *buf, const WhPass &ps, const Cplx *__restrict__ tws)
 {
     constexpr uint32_t PER = (PMAX / R + NT - 1) / NT;
-    const uint32_t B = ps.B, step = ps.step, Ns = ps.Ns;
+    const uint32_t B = ps.B, Ns = ps.Ns;
+    const Cplx *tw = tws + ps.tw;
     Cplx v[PER][R];
     uint32_t base[PER];
 #pragma unroll
@@ -479,13 +606,13 @@ __device__ __forceinline__ void wh_pass(Cplx *buf, const WhPass &ps, const Cplx 
 #pragma unroll
             for (int r = 0; r < R; ++r) v[q][r] = buf[j + r * B];
             const uint32_t k = j - udiv_m(j, ps.m_ns) * Ns;
-            if (k != 0) {
-                const Cplx w1 = tw[k * step];
-                Cplx w = w1;
+            if (Ns > 1) {
+                Cplx w[R];
+                w[1] = tw[k];
 #pragma unroll
                 for (int r = 1; r < R; ++r) {
-                    v[q][r] = cmul(v[q][r], w);
-                    if (r + 1 < R) w = cmul(w, w1);
+                    if (r > 1) w[r] = r % 2 ? cmul(w[r - 1], w[1]) : cmul(w[r / 2], w[r / 2]);
+                    v[q][r] = cmul(v[q][r], w[r]);
                 }
             }
             dft_any<R>(v[q]);
@@ -501,17 +628,120 @@ __device__ __forceinline__ void wh_pass(Cplx *buf, const WhPass &ps, const Cplx 
     __syncthreads();
 }
 
-// A pass of odd prime radix R (11 .. kWhPrimeMax), the same butterflies with
-// the R-point DFT from the pairs (r, R - r) as in dft_prime:
-//   A: each pair twiddled and replaced in place by a_r = x_r + x_{R-r} (at r)
-//      and b_r = x_r - x_{R-r} (at R - r)
-//   B: one thread per output pair (q, R - q) of a butterfly (q = 0: the sum),
-//      Y_q = x_0 + sum_r (a_r cos t - i b_r sin t), Y_{R-q} with + i, t = 2 pi r q / R;
-//      the lanes of a wavefront share the butterfly (the same a_r, b_r: LDS
-//      broadcasts) and step cos t, sin t by the three-term recurrence
-//      f(r+1) = 2 cos(2 pi q / R) f(r) - f(r-1) (two multiply-adds a step)
-// R(R-1)/2 real multiply-adds per butterfly and plane pair instead of R^2
-// complex products. The recurrence's rounding errors grow at most like
+// A pass of odd prime radix R (11 .. kWhPrimeMax) takes the R-point DFT from the
+// pairs (r, R - r) as in dft_prime, H = (R - 1) / 2:
+//   fold : each pair twiddled and replaced in place by a_r = x_r + x_{R-r} (at r)
+//          and b_r = x_r - x_{R-r} (at R - r)
+//   sums : Y_q = x_0 + sum_r (a_r cos t - i b_r sin t), Y_{R-q} with + i, t = 2 pi r q / R,
+//          for q = 0 .. H (q = 0: the sum alone)
+template <uint32_t NT>
+__device__ __forceinline__ void wh_fold_pairs(Cplx *buf, const WhPass &ps, const Cplx *__restrict__ tws)
+{
+    const uint32_t R = ps.R, Ns = ps.Ns, B = ps.B, H = (R - 1) / 2;
+    const Cplx *tw = tws + ps.tw;
+    for (uint32_t e = threadIdx.x; e < B * H; e += NT) {
+        const uint32_t r0 = udiv_m(e, ps.m_b), r = r0 + 1, j = e - r0 * B, k = j - udiv_m(j, ps.m_ns) * Ns;
+        const uint32_t iu = j + r * B, iv = j + (R - r) * B;
+        Cplx u = buf[iu], v = buf[iv];
+        if (Ns > 1) {
+            u = cmul(u, tw[r0 * Ns + k]);
+            v = cmul(v, tw[(R - 1 - r) * Ns + k]);
+        }
+        buf[iu] = cadd(u, v);
+        buf[iv] = csub(u, v);
+    }
+    __syncthreads();
+}
+
+// The sums as matrix products on the matrix cores: the roots' cosines and sines
+// (rows q, columns r) times the a_r and b_r of 16 butterflies, real and
+// imaginary parts apart, v_mfma_f64_16x16x4 each. A wavefront takes up to
+// kMatrixRounds tiles of 16 outputs by 16 butterflies and keeps their sums in
+// registers until every wavefront has read its terms. The vector form reads both
+// terms for every output (bound by LDS) and computes its roots; here a term serves
+// 16 outputs and the matrix cores set the pace: of 101000 cycles at 10001 = 73 x 137
+// points the two products take 20000 and 36000, where the instructions alone would
+// (padding to 16 included) 16000 and 30000. 10001 points 331 -> 181 ns per signal.
+constexpr uint32_t kMatrixRounds = 2;
+using Quad = double __attribute__((ext_vector_type(4)));
+
+__host__ __device__ constexpr uint32_t matrix_steps(uint32_t R) { return ((R - 1) / 2 + 3) / 4; }
+__host__ __device__ constexpr uint32_t matrix_rows(uint32_t R) { return ((R - 1) / 2 + 16) / 16; }
+__host__ __device__ constexpr uint32_t matrix_tiles(uint32_t R, uint32_t B) { return matrix_rows(R) * ((B + 15) / 16); }
+
+template <uint32_t NT>
+__device__ __forceinline__ void wh_pass_matrix(Cplx *buf, const WhPass &ps, const Cplx *__restrict__ tw,
+                                               const Cplx *__restrict__ frags)
+{
+    wh_fold_pairs<NT>(buf, ps, tw);
+    const uint32_t R = ps.R, Ns = ps.Ns, B = ps.B, H = (R - 1) / 2;
+    const uint32_t steps = matrix_steps(R), rows = matrix_rows(R), tiles = matrix_tiles(R, B);
+    const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t col = lane & 15, sub = lane >> 4;
+    Quad cr[kMatrixRounds], ci[kMatrixRounds], sr[kMatrixRounds], si[kMatrixRounds];
+#pragma unroll
+    for (uint32_t g = 0; g < kMatrixRounds; ++g) {
+        sr[g] = si[g] = Quad{0.0, 0.0, 0.0, 0.0};
+        const uint32_t tile = wave + g * (NT / 64);
+        if (tile >= tiles) continue;
+        const uint32_t ct = tile / rows, rt = tile - ct * rows;
+        const uint32_t j = min(ct * 16 + col, B - 1);
+        const Cplx x0 = buf[j];
+        cr[g] = Quad{x0.re, x0.re, x0.re, x0.re};
+        ci[g] = Quad{x0.im, x0.im, x0.im, x0.im};
+        const Cplx *f = frags + ps.frag + (size_t)rt * steps * 64 + lane;
+        // terms r = 4 t + sub + 1, a_r and b_r of the lane's butterfly (zero beyond
+        // H, which only the last step reaches), requested a step ahead of their use
+        struct Term {
+            Cplx w, a, b;
+        };
+        const Cplx *pa = buf + j + (sub + 1) * B, *pb = buf + j + (R - 1 - sub) * B;
+        auto term = [&](uint32_t t) {
+            Term m{f[t * 64], pa[t * 4 * B], pb[-(int)(t * 4 * B)]};
+            if (t + 1 == steps && t * 4 + sub + 1 > H) m.a = m.b = Cplx{0.0, 0.0};
+            return m;
+        };
+        auto add = [&](const Term &m) {
+            cr[g] = __builtin_amdgcn_mfma_f64_16x16x4f64(m.w.re, m.a.re, cr[g], 0, 0, 0);
+            ci[g] = __builtin_amdgcn_mfma_f64_16x16x4f64(m.w.re, m.a.im, ci[g], 0, 0, 0);
+            sr[g] = __builtin_amdgcn_mfma_f64_16x16x4f64(m.w.im, m.b.re, sr[g], 0, 0, 0);
+            si[g] = __builtin_amdgcn_mfma_f64_16x16x4f64(m.w.im, m.b.im, si[g], 0, 0, 0);
+        };
+        Term even = term(0);
+        uint32_t t = 0;
+        for (; t + 2 <= steps; t += 2) {
+            const Term odd = term(t + 1);
+            add(even);
+            even = term(min(t + 2, steps - 1));
+            add(odd);
+        }
+        if (t < steps) add(even);
+    }
+    __syncthreads();
+#pragma unroll
+    for (uint32_t g = 0; g < kMatrixRounds; ++g) {
+        const uint32_t tile = wave + g * (NT / 64);
+        if (tile >= tiles) continue;
+        const uint32_t ct = tile / rows, rt = tile - ct * rows, j = ct * 16 + col;
+        const uint32_t k = j - udiv_m(j, ps.m_ns) * Ns, ob = (j - k) * R + k;
+#pragma unroll
+        for (uint32_t e = 0; e < 4; ++e) {
+            // the lane's sums: rows 4 e + sub of the tile
+            const uint32_t q = rt * 16 + 4 * e + sub;
+            if (j < B && q <= H) {
+                buf[ob + q * Ns] = Cplx{cr[g][e] + si[g][e], ci[g][e] - sr[g][e]};
+                if (q > 0) buf[ob + (R - q) * Ns] = Cplx{cr[g][e] - si[g][e], ci[g][e] + sr[g][e]};
+            }
+        }
+    }
+    __syncthreads();
+}
+
+// The sums of a pass without a root matrix: one thread per output pair
+// (q, R - q) of a butterfly; the lanes of a wavefront share the butterfly (the
+// same a_r, b_r: LDS broadcasts) and step cos t, sin t by the three-term
+// recurrence f(r+1) = 2 cos(2 pi q / R) f(r) - f(r-1) (two multiply-adds a
+// step). The recurrence's rounding errors grow at most like
 // r min(r, 1 / |sin(2 pi q / R)|) units in the last place: about 1e-12 of the
 // unit roots at most over the (R-1)/2 <= 128 steps, far under what moves a
 // tune (the tests hold the tunes to 1e-12 of the long-double DFT's).
@@ -520,20 +750,8 @@ __device__ __forceinline__ void wh_pass_prime(Cplx *buf, const WhPass &ps, const
 {
     // output pairs per thread: B (H + 1) <= L (R + 1) / (2R) <= 0.55 L for R >= 11
     constexpr uint32_t GP = ((PMAX * 11 / 20 + NT - 1) / NT + 1) / 2 * 2;
-    const uint32_t R = ps.R, Ns = ps.Ns, B = ps.B, H = (R - 1) / 2, step = ps.step;
-    for (uint32_t e = threadIdx.x; e < B * H; e += NT) {
-        const uint32_t j = udiv_m(e, ps.m_h), r = e - j * H + 1, k = j - udiv_m(j, ps.m_ns) * Ns;
-        const uint32_t iu = j + r * B, iv = j + (R - r) * B;
-        Cplx u = buf[iu], v = buf[iv];
-        if (k != 0) {
-            // k r step < L: the exponents need no reduction
-            u = cmul(u, tw[k * r * step]);
-            v = cmul(v, tw[k * (R - r) * step]);
-        }
-        buf[iu] = cadd(u, v);
-        buf[iv] = csub(u, v);
-    }
-    __syncthreads();
+    const uint32_t R = ps.R, Ns = ps.Ns, B = ps.B, H = (R - 1) / 2;
+    wh_fold_pairs<NT>(buf, ps, tw);
     // output positions (< 2^15) of Y_q in the low, of Y_{R-q} in the high half
     static_assert(PMAX < 0xffffu, "output positions are packed in 16 bits");
     static_assert(GP % 2 == 0, "output pairs are taken two at a time");
@@ -552,7 +770,7 @@ __device__ __forceinline__ void wh_pass_prime(Cplx *buf, const WhPass &ps, const
             const uint32_t e = min(threadIdx.x + (g + h) * NT, items - 1);
             ja[h] = udiv_m(e, ps.m_h1);
             qa[h] = e - ja[h] * (H + 1);
-            const Cplx wq = tw[qa[h] * B];  // W_L^{q L / R} = exp(-2 pi i q / R)
+            const Cplx wq = tw[ps.root + qa[h]];  // exp(-2 pi i q / R)
             c[h] = wq.re;
             sn[h] = -wq.im;
             cp[h] = 1.0;
@@ -604,32 +822,44 @@ __device__ __forceinline__ void wh_pass_prime(Cplx *buf, const WhPass &ps, const
 }
 
 // Forward DFT of the whole signal in LDS, in natural order. The plan lists its
-// radices grouped (3s, 5s, 7s, the other primes, then 2s, 4s, 8s: an odd or
-// small first radix keeps the first pass's strided stores off shared banks),
-// so each radix gets a loop of its own: one switch over the inlined passes
-// inside a single loop keeps more registers live than any pass needs.
+// radices grouped as here (an odd or small first radix keeps the first pass's
+// strided stores off shared banks), so each radix gets a loop of its own: one
+// switch over the inlined passes inside a single loop keeps more registers live
+// than any pass needs.
 template <uint32_t NT, uint32_t PMAX>
-__device__ __forceinline__ void wh_fft(Cplx *buf, const WhPlan &p, const Cplx *__restrict__ tw)
+__device__ __forceinline__ void wh_fft(Cplx *buf, const WhPlan &p, const Cplx *__restrict__ tw,
+                                       const Cplx *__restrict__ frags)
 {
     uint32_t s = 0;
     for (; s < p.n_pass && p.pass[s].R == 3; ++s) wh_pass<3, NT, PMAX>(buf, p.pass[s], tw);
     for (; s < p.n_pass && p.pass[s].R == 5; ++s) wh_pass<5, NT, PMAX>(buf, p.pass[s], tw);
     for (; s < p.n_pass && p.pass[s].R == 7; ++s) wh_pass<7, NT, PMAX>(buf, p.pass[s], tw);
-    for (; s < p.n_pass && p.pass[s].R > 8; ++s) wh_pass_prime<NT, PMAX>(buf, p.pass[s], tw);
+    for (; s < p.n_pass && p.pass[s].R == 9; ++s) wh_pass<9, NT, PMAX>(buf, p.pass[s], tw);
+    for (; s < p.n_pass && p.pass[s].R == 11; ++s) wh_pass<11, NT, PMAX>(buf, p.pass[s], tw);
+    for (; s < p.n_pass && p.pass[s].R == 13; ++s) wh_pass<13, NT, PMAX>(buf, p.pass[s], tw);
+    for (; s < p.n_pass && p.pass[s].R > 16; ++s) {
+        if (p.pass[s].frag != kNoFrag) wh_pass_matrix<NT>(buf, p.pass[s], tw, frags);
+        else wh_pass_prime<NT, PMAX>(buf, p.pass[s], tw);
+    }
+    for (; s < p.n_pass && p.pass[s].R == 6; ++s) wh_pass<6, NT, PMAX>(buf, p.pass[s], tw);
+    for (; s < p.n_pass && p.pass[s].R == 10; ++s) wh_pass<10, NT, PMAX>(buf, p.pass[s], tw);
     for (; s < p.n_pass && p.pass[s].R == 2; ++s) wh_pass<2, NT, PMAX>(buf, p.pass[s], tw);
+    for (; s < p.n_pass && p.pass[s].R == 12; ++s) wh_pass<12, NT, PMAX>(buf, p.pass[s], tw);
     for (; s < p.n_pass && p.pass[s].R == 4; ++s) wh_pass<4, NT, PMAX>(buf, p.pass[s], tw);
     for (; s < p.n_pass && p.pass[s].R == 8; ++s) wh_pass<8, NT, PMAX>(buf, p.pass[s], tw);
+    for (; s < p.n_pass && p.pass[s].R == 16; ++s) wh_pass<16, NT, PMAX>(buf, p.pass[s], tw);
 }
 
 // One workgroup per signal (2 per particle: plane x, plane y): load, mean
 // removal and Hanning, the transform(s), the first maximum of |X_k| over
 // k < N and the three-point interpolation (dynamic_indicator.cpp:139-196).
-template <bool CZ, uint32_t NT, uint32_t PMAX>
+template <bool CZ, uint32_t NT>
 __global__ void __launch_bounds__(NT, 4) k_wh_tune(WhArgs a)
 {
+    constexpr uint32_t PMAX = kWhPoints * NT;
     extern __shared__ Cplx buf[];
     __shared__ double sv[NT / 64];
-    __shared__ uint32_t si[NT / 64];
+    __shared__ uint32_t first;
     const uint32_t sig = blockIdx.x;
     const uint32_t particle = a.p0 + sig / 2, plane = sig % 2;
     const size_t nn = a.n;
@@ -648,6 +878,9 @@ __global__ void __launch_bounds__(NT, 4) k_wh_tune(WhArgs a)
     const bool scan_other =
         !a.means || !(isfinite(mc[0]) && isfinite(mc[1]) && isfinite(mc[2]) && isfinite(mc[3]));
     const int cx = 2 * plane, cp = cx + 1, co0 = 2 * (1 - plane), co1 = co0 + 1;
+    // selected once: an index into mc at run time is a chain of compares at each use
+    const double mean_x = plane ? mc[2] : mc[0], mean_p = plane ? mc[3] : mc[1];
+    const double mean_o0 = plane ? mc[0] : mc[2], mean_o1 = plane ? mc[1] : mc[3];
     int nan_seen = 0;
     // every sample load of the thread issued before the first use (a loop
     // that waits for each sample in turn leaves the workgroup idle)
@@ -667,14 +900,14 @@ __global__ void __launch_bounds__(NT, 4) k_wh_tune(WhArgs a)
     if (scan_other)
         for (uint32_t m = threadIdx.x; m < N; m += NT) {
             const uint64_t sm = (uint64_t)a.from + m;
-            nan_seen |= __builtin_isnan(a.hist[hat(a.lay, sm, co0, particle)] - mc[co0]) ||
-                        __builtin_isnan(a.hist[hat(a.lay, sm, co1, particle)] - mc[co1]);
+            nan_seen |= __builtin_isnan(a.hist[hat(a.lay, sm, co0, particle)] - mean_o0) ||
+                        __builtin_isnan(a.hist[hat(a.lay, sm, co1, particle)] - mean_o1);
         }
 #pragma unroll
     for (uint32_t u = 0; u < LP; ++u) {
         const uint32_t m = threadIdx.x + u * NT;
         if (m < N) {
-            const double x = vx[u] - mc[cx], xp = vp[u] - mc[cp];
+            const double x = vx[u] - mean_x, xp = vp[u] - mean_p;
             nan_seen |= __builtin_isnan(x) || __builtin_isnan(xp);
             Cplx z{x * hh[u], xp * hh[u]};
             if constexpr (CZ) z = cmul(z, a.chirp[m]);
@@ -687,7 +920,7 @@ __global__ void __launch_bounds__(NT, 4) k_wh_tune(WhArgs a)
         if (threadIdx.x == 0) *o = __builtin_nan("");
         return;
     }
-    wh_fft<NT, PMAX>(buf, a.plan, a.tw);
+    wh_fft<NT, PMAX>(buf, a.plan, a.tw, a.frag);
     if constexpr (CZ) {
         for (uint32_t k = threadIdx.x; k < M; k += NT) {
             const uint32_t l = k;
@@ -695,33 +928,50 @@ __global__ void __launch_bounds__(NT, 4) k_wh_tune(WhArgs a)
             buf[l] = Cplx{z.re, -z.im};
         }
         __syncthreads();
-        wh_fft<NT, PMAX>(buf, a.plan, a.tw);
+        wh_fft<NT, PMAX>(buf, a.plan, a.tw, a.frag);
     }
-    auto mag = [&](uint32_t k) {
+    // first maximum of |X_k|, k < N: the largest square (one square root of it for
+    // the workgroup instead of one an entry), then the lowest k whose root equals
+    // its root; only squares within a few units of it can
+    auto square = [&](uint32_t k) {
         const Cplx z = buf[k];
-        return sqrt(z.re * z.re + z.im * z.im);
+        return z.re * z.re + z.im * z.im;
     };
-    // first maximum: each thread scans increasing k, ties go to the lower k
-    double v = -1.0;
-    uint32_t i = 0xffffffffu;
-    for (uint32_t k = threadIdx.x; k < N; k += NT) {
-        const double mg = mag(k);
-        if (mg > v || i == 0xffffffffu) { v = mg; i = k; }
+    double sq[LP], top = -1.0;
+#pragma unroll
+    for (uint32_t u = 0; u < LP; ++u) {
+        const uint32_t k = threadIdx.x + u * NT;
+        const double v = square(min(k, N - 1));
+        sq[u] = k < N ? v : -1.0;
+        top = sq[u] > top ? sq[u] : top;
     }
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) {
-        const double ov = __shfl_xor(v, off);
-        const uint32_t oi = __shfl_xor(i, off);
-        if (ov > v || (ov == v && oi < i)) { v = ov; i = oi; }
+        const double o2 = __shfl_xor(top, off);
+        top = o2 > top ? o2 : top;
     }
-    if ((threadIdx.x & 63) == 0) { sv[threadIdx.x >> 6] = v; si[threadIdx.x >> 6] = i; }
+    if (threadIdx.x == 0) first = 0xffffffffu;
+    if ((threadIdx.x & 63) == 0) sv[threadIdx.x >> 6] = top;
+    __syncthreads();
+    top = sv[threadIdx.x % (NT / 64)];
+#pragma unroll
+    for (int off = (int)NT / 128; off > 0; off >>= 1) {
+        const double o2 = __shfl_xor(top, off);
+        top = o2 > top ? o2 : top;
+    }
+    const double near = top * (1.0 - 0x1p-50), root = sqrt(top);
+    uint32_t i = 0xffffffffu;
+#pragma unroll
+    for (int u = (int)LP - 1; u >= 0; --u)
+        if (sq[u] >= near) {
+            asm volatile("" : "+v"(sq[u]));  // no root ahead of the branch
+            if (sqrt(sq[u]) == root) i = threadIdx.x + u * NT;
+        }
+    if (i != 0xffffffffu) atomicMin(&first, i);
     __syncthreads();
     if (threadIdx.x == 0) {
-        double bv = sv[0];
-        uint32_t bi = si[0];
-        for (uint32_t q = 1; q < NT / 64; ++q)
-            if (sv[q] > bv || (sv[q] == bv && si[q] < bi)) { bv = sv[q]; bi = si[q]; }
-        *o = interp_tune_at(mag, N, bi);
+        auto mag = [&](uint32_t k) { return sqrt(square(k)); };
+        *o = interp_tune_at(mag, N, first == 0xffffffffu ? 0u : first, a.cos_n, a.sin_n);
     }
 }
 
@@ -919,51 +1169,76 @@ static void set_lds(K kernel, size_t bytes)
 }
 
 // ---------------------------------------------------------------- whole-signal plans
-// The three shapes of k_wh_tune: up to 2048 points with 256 threads, up to
-// 4096 with 512 (several workgroups per CU at four wavefronts per SIMD), up to
-// kWhPmax with 1024 (one).
-constexpr uint32_t kWhSmallPmax = 2048, kWhSmallThreads = 256;
-constexpr uint32_t kWhMidPmax = 4096, kWhMidThreads = 512;
-constexpr uint32_t kWhPmax = 10240, kWhThreads = 1024;
-
-// Passes of the direct transform of L, grouped as wh_fft runs them: 3s, 5s,
-// 7s, the other primes in increasing order (each at most kWhPrimeMax), then the
-// power of two as 2, 4 and 8s (8 while it divides). `gen` = the sum of the
-// other primes (their passes cost about 2R operations per point against a few
-// tens for a small radix).
+// Passes of the direct transform of L: primes from 17 up to kWhPrimeMax by one
+// pass each, the rest by as few passes as the radices 2 .. 13 and 16 allow (each
+// pass is a trip through LDS behind two barriers, 4000 to 7000 cycles of a
+// workgroup of 1024 threads at 10^4 points whatever its radix), of the fewest the
+// one with the smallest sum of radices; grouped as wh_fft runs them. `gen` = the
+// sum of the primes (their passes cost about 2R operations per point against a
+// few tens for a small radix).
 static uint32_t udiv_magic(uint32_t d) { return d == 1 ? 0u : (uint32_t)((1ull << 32) / d + 1); }
+
+constexpr uint32_t kSmallRadices[] = {16, 13, 12, 11, 10, 9, 8, 7, 6, 5, 4, 3, 2};
+
+// The best list of radices (not increasing, from entry `from` on) with product r:
+// the fewest; then one with a radix whose stores of the first pass share banks
+// least (stride R entries of 16 bytes); then the smallest sum.
+static bool few_radices(uint32_t r, size_t from, std::vector<uint32_t> &best)
+{
+    best.clear();
+    if (r == 1) return true;
+    auto cost = [](const std::vector<uint32_t> &v) {
+        uint32_t sum = 0, shared = 8;
+        for (uint32_t R : v) {
+            sum += R;
+            shared = std::min(shared, R & (0u - R));
+        }
+        return (uint64_t)v.size() << 32 | shared << 16 | sum;
+    };
+    bool found = false;
+    for (size_t q = from; q < std::size(kSmallRadices); ++q) {
+        std::vector<uint32_t> rest;
+        if (r % kSmallRadices[q] || !few_radices(r / kSmallRadices[q], q, rest)) continue;
+        rest.push_back(kSmallRadices[q]);
+        if (!found || cost(rest) < cost(best)) best = rest;
+        found = true;
+    }
+    return found;
+}
 
 static bool wh_radix_plan(uint32_t L, WhPlan &p, uint32_t &gen)
 {
     p = WhPlan{};
     p.L = L;
     gen = 0;
-    uint32_t r = L, Ns = 1;
+    uint32_t r = L, Ns = 1, tw = 0;
     auto push = [&](uint32_t R) {
         if (p.n_pass == (uint32_t)kWhMaxPasses) return false;
         WhPass &q = p.pass[p.n_pass++];
-        q.R = R; q.Ns = Ns; q.B = L / R; q.step = L / (Ns * R);
-        q.m_ns = udiv_magic(Ns); q.m_h = udiv_magic(std::max(1u, (R - 1) / 2)); q.m_h1 = udiv_magic((R - 1) / 2 + 1);
+        q.R = R; q.Ns = Ns; q.B = L / R;
+        q.m_ns = udiv_magic(Ns); q.m_b = udiv_magic(q.B); q.m_h1 = udiv_magic((R - 1) / 2 + 1);
+        q.frag = kNoFrag;
+        q.tw = tw;
+        if (Ns > 1) tw += R > 16 ? (R - 1) * Ns : Ns;
+        q.root = tw;
+        if (R > 16) tw += (R - 1) / 2 + 1;
         Ns *= R;
-        r /= R;
         return true;
     };
-    for (uint32_t R : {3u, 5u, 7u})
-        while (r % R == 0)
-            if (!push(R)) return false;
-    for (uint32_t q = 11; r > 1 && q <= kWhPrimeMax; q += 2)
-        while (r % q == 0) {
-            if (!push(q)) return false;
+    std::vector<uint32_t> primes, small;
+    uint32_t smooth = 1;
+    for (uint32_t q : {2u, 3u, 5u, 7u, 11u, 13u})
+        for (; r % q == 0; r /= q) smooth *= q;
+    for (uint32_t q = 17; r > 1 && q <= kWhPrimeMax; q += 2)
+        for (; r % q == 0; r /= q) {
+            primes.push_back(q);
             gen += q;
         }
-    uint32_t twos = 0;
-    while (r % 2 == 0) { r /= 2; ++twos; }
-    if (r != 1) return false;
-    r = 1u << twos;  // the power of two, taken as 2^(twos mod 3 == 1), 4^(... == 2), then 8s
-    if (twos % 3 == 1 && !push(2)) return false;
-    if (twos % 3 == 2 && !push(4)) return false;
-    while (r > 1)
-        if (!push(8)) return false;
+    if (r != 1 || !few_radices(smooth, 0, small)) return false;
+    for (uint32_t R : {3u, 5u, 7u, 9u, 11u, 13u, 0u, 6u, 10u, 2u, 12u, 4u, 8u, 16u}) {
+        for (uint32_t v : R ? small : primes)
+            if ((!R || v == R) && !push(v)) return false;
+    }
     return true;
 }
 
@@ -971,17 +1246,53 @@ struct WhTables {
     bool ok = false, cz = false;
     uint32_t M = 0, nt = 0;
     WhPlan plan{};
-    Cplx *tw = nullptr, *chirp = nullptr, *bhat = nullptr;
+    Cplx *tw = nullptr, *chirp = nullptr, *bhat = nullptr, *frag = nullptr;
 };
 
+static uint32_t wh_threads(uint32_t M)
+{
+    uint32_t nt = 64;
+    while (nt * kWhPoints < M) nt *= 2;
+    return nt;
+}
 
-// Whole-signal plan of a window length (cached per device): the direct
-// transform when N is {2,3,5,7}-smooth or its other primes are cheap (sum at
-// most kWhCzGen), else chirp-z over the smallest smooth M >= 2N - 1 that
-// fits, else the direct transform with dearer prime passes; none when N does
-// not fit or has a prime above kWhPrimeMax and no chirp-z length fits.
+// A prime pass runs on the matrix cores where its tiles fit the registers of the
+// plan's wavefronts; others (17, 19 and 37 near the most points of a shape, 257,
+// primes above 64 in the shapes of one and two wavefronts) take their sums on the
+// vector units. ns per signal with and without, at 2e8 points in all: 437 points (19 x 23) 4.9 and 6.2, 2491 (47 x 53) 28
+// and 40, 4087 (61 x 67) 58 and 99, 10001 (73 x 137) 184 and 331.
+static bool matrix_pass(const WhPass &ps, uint32_t nt)
+{
+    return ps.R > 16 && matrix_tiles(ps.R, ps.B) <= kMatrixRounds * (nt / 64);
+}
+
+// Whether N's own transform beats chirp-z over more than twice the points: without
+// prime passes always; with them while their sum is at most kWhCzGen or all run
+// on the matrix cores, over enough butterflies to fill a pass (a wavefront's worth
+// of a matrix tile's 16; a matrix pass of few rows always). ns per signal, direct
+// and chirp-z: 323 points (17 x 19) 4.4 and 8.0, 1207 (17 x 71) 18 and 23, 2010
+// (30 x 67) 23 and 47, 2869 (19 x 151) 58 and 90; but 67 points 5.7 and 3.5, 501
+// (3 x 167) 12.8 and 10.7, 755 (5 x 151) 23 and 18, 1799 (7 x 257) 63 and 48.
 constexpr uint32_t kWhCzGen = 128;
+static bool prefer_direct(const WhPlan &p, uint32_t gen)
+{
+    const uint32_t nt = wh_threads(p.L);
+    bool all_matrix = true, filled = true;
+    for (uint32_t q = 0; q < p.n_pass; ++q) {
+        const WhPass &ps = p.pass[q];
+        if (ps.R <= 16) continue;
+        const bool m = matrix_pass(ps, nt);
+        all_matrix &= m;
+        filled &= ps.B >= 16 || (m && gen <= kWhCzGen);
+    }
+    return filled && (gen <= kWhCzGen || all_matrix);
+}
 
+// Whole-signal plan of a window length (cached per device): the direct transform
+// or chirp-z over a smooth M >= 2N - 1 that fits, by the rule above; the direct
+// transform also where no chirp-z length fits; none when N does not fit or has a
+// prime above kWhPrimeMax and no chirp-z length fits. M is the one of the least
+// passes times points: 501 points take 1008 = 7 x 9 x 16.
 static const WhTables *wh_tables(uint32_t N, hipStream_t s)
 {
     static std::mutex mu;
@@ -995,12 +1306,7 @@ static const WhTables *wh_tables(uint32_t N, hipStream_t s)
     hip_check(hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, dev), "hipDeviceGetAttribute");
     // the kernels' own LDS (reductions) comes on top of the signal
     size_t fixed = 0;
-    for (const void *k : {(const void *)k_wh_tune<false, kWhSmallThreads, kWhSmallPmax>,
-                          (const void *)k_wh_tune<true, kWhSmallThreads, kWhSmallPmax>,
-                          (const void *)k_wh_tune<false, kWhMidThreads, kWhMidPmax>,
-                          (const void *)k_wh_tune<true, kWhMidThreads, kWhMidPmax>,
-                          (const void *)k_wh_tune<false, kWhThreads, kWhPmax>,
-                          (const void *)k_wh_tune<true, kWhThreads, kWhPmax>}) {
+    for (const void *k : {(const void *)k_wh_tune<false, kWhThreads>, (const void *)k_wh_tune<true, kWhThreads>}) {
         hipFuncAttributes fa{};
         hip_check(hipFuncGetAttributes(&fa, k), "hipFuncGetAttributes");
         fixed = std::max(fixed, (size_t)fa.sharedSizeBytes);
@@ -1013,13 +1319,19 @@ static const WhTables *wh_tables(uint32_t N, hipStream_t s)
     const bool direct = fits(N) && wh_radix_plan(N, pd, gen);
     uint32_t Mcz = 0;
     WhPlan pc{};
-    if (!(direct && gen <= kWhCzGen)) {
-        for (uint64_t M = 2ull * N - 1; M <= kWhPmax && fits((uint32_t)M); ++M) {
+    const bool own = direct && prefer_direct(pd, gen);
+    if (!own) {
+        uint64_t cost = ~0ull;
+        for (uint64_t M = 2ull * N - 1; M <= 4ull * N && M <= kWhPmax && fits((uint32_t)M); ++M) {
             uint32_t g = 0;
-            if (wh_radix_plan((uint32_t)M, pc, g) && g == 0) { Mcz = (uint32_t)M; break; }
+            WhPlan pm{};
+            if (!wh_radix_plan((uint32_t)M, pm, g) || g || pm.n_pass * M >= cost) continue;
+            cost = pm.n_pass * M;
+            Mcz = (uint32_t)M;
+            pc = pm;
         }
     }
-    if (direct && (gen <= kWhCzGen || !Mcz)) {
+    if (own || (direct && !Mcz)) {
         t.ok = true; t.cz = false; t.M = N; t.plan = pd;
     } else if (Mcz) {
         t.ok = true; t.cz = true; t.M = Mcz; t.plan = pc;
@@ -1029,14 +1341,40 @@ static const WhTables *wh_tables(uint32_t N, hipStream_t s)
         return nullptr;
     }
     const uint32_t M = t.M;
-    t.nt = M <= kWhSmallPmax ? kWhSmallThreads : M <= kWhMidPmax ? kWhMidThreads : kWhThreads;
+    t.nt = wh_threads(M);
     const long double two_pi = 6.283185307179586476925286766559005768L, pi = two_pi / 2;
-    std::vector<Cplx> w(M);
-    for (uint32_t q = 0; q < M; ++q) {
-        const long double ang = two_pi * (long double)q / (long double)M;
-        w[q] = Cplx{(double)cosl(ang), (double)-sinl(ang)};
+    std::vector<Cplx> w;
+    auto root = [&](uint64_t num, uint64_t den) {
+        const long double ang = two_pi * (long double)(num % den) / (long double)den;
+        w.push_back(Cplx{(double)cosl(ang), (double)-sinl(ang)});
+    };
+    for (uint32_t p = 0; p < t.plan.n_pass; ++p) {
+        const WhPass &ps = t.plan.pass[p];
+        if (ps.Ns > 1)
+            for (uint32_t r = 1; r < (ps.R > 16 ? ps.R : 2u); ++r)
+                for (uint32_t k = 0; k < ps.Ns; ++k) root((uint64_t)k * r, (uint64_t)ps.Ns * ps.R);
+        if (ps.R > 16)
+            for (uint32_t q = 0; q <= (ps.R - 1) / 2; ++q) root(q, ps.R);
     }
+    if (w.empty()) w.push_back(Cplx{1.0, 0.0});
     t.tw = upload(w, s, "hipMalloc(whole-signal twiddles)");
+    // Root matrices in the lanes' order of the matrix instruction: lane l of step t
+    // of row tile i holds row q = 16 i + l % 16, column r = 4 t + l / 16 + 1 (zero beyond H).
+    std::vector<Cplx> frag;
+    for (uint32_t p = 0; p < t.plan.n_pass; ++p) {
+        WhPass &ps = t.plan.pass[p];
+        if (!matrix_pass(ps, t.nt)) continue;
+        ps.frag = (uint32_t)frag.size();
+        const uint32_t H = (ps.R - 1) / 2;
+        for (uint32_t i = 0; i < matrix_rows(ps.R); ++i)
+            for (uint32_t st = 0; st < matrix_steps(ps.R); ++st)
+                for (uint32_t l = 0; l < 64; ++l) {
+                    const uint32_t q = 16 * i + l % 16, r = 4 * st + l / 16 + 1;
+                    const long double ang = two_pi * (long double)(q * r % ps.R) / (long double)ps.R;
+                    frag.push_back(q <= H && r <= H ? Cplx{(double)cosl(ang), (double)sinl(ang)} : Cplx{0.0, 0.0});
+                }
+    }
+    if (!frag.empty()) t.frag = upload(frag, s, "hipMalloc(whole-signal root matrices)");
     if (t.cz) {
         // chirp c_m = exp(-i pi (m^2 mod 2N) / N), filter b_j = conj(c_j) for
         // |j| < N (j mod M), B = DFT_M(b) in natural order
@@ -1059,10 +1397,12 @@ static const WhTables *wh_tables(uint32_t N, hipStream_t s)
     return &cache[{dev, N}];
 }
 
-template <bool CZ, uint32_t NT, uint32_t PMAX>
-static void launch_wh(const WhArgs &a0, uint32_t n, size_t lds_bytes, hipStream_t s)
+template <bool CZ, uint32_t NT>
+static void launch_wh(const WhArgs &a0, uint32_t nt, uint32_t n, size_t lds_bytes, hipStream_t s)
 {
-    auto k = k_wh_tune<CZ, NT, PMAX>;
+    if constexpr (NT > 64)
+        if (nt < NT) return launch_wh<CZ, NT / 2>(a0, nt, n, lds_bytes, s);
+    auto k = k_wh_tune<CZ, NT>;
     set_lds(k, lds_bytes);
     WhArgs a = a0;
     // 2 signals per particle, one workgroup each: grids below 2^31 workgroups
@@ -1085,20 +1425,14 @@ static bool fft_tune_whole(const double *hist, HistLayout lay, uint32_t n, const
     if (n == 0) return true;
     WhArgs a{};
     a.hist = hist; a.lay = lay; a.means = means; a.n = n; a.from = from; a.N = N; a.M = t->M;
-    a.plan = t->plan; a.hann = hann; a.tw = t->tw; a.chirp = t->chirp; a.bhat = t->bhat;
+    a.plan = t->plan; a.hann = hann; a.tw = t->tw;
+    a.cos_n = std::cos(2.0 * M_PI / (double)N); a.sin_n = std::sin(2.0 * M_PI / (double)N);
+    a.frag = t->frag; a.chirp = t->chirp; a.bhat = t->bhat;
     a.out = out; a.window = window;
     const size_t lds_bytes = (size_t)t->M * sizeof(Cplx);
     LaunchTimer timer("k_wh_tune", s);
-    if (t->nt == kWhSmallThreads) {
-        if (t->cz) launch_wh<true, kWhSmallThreads, kWhSmallPmax>(a, n, lds_bytes, s);
-        else launch_wh<false, kWhSmallThreads, kWhSmallPmax>(a, n, lds_bytes, s);
-    } else if (t->nt == kWhMidThreads) {
-        if (t->cz) launch_wh<true, kWhMidThreads, kWhMidPmax>(a, n, lds_bytes, s);
-        else launch_wh<false, kWhMidThreads, kWhMidPmax>(a, n, lds_bytes, s);
-    } else {
-        if (t->cz) launch_wh<true, kWhThreads, kWhPmax>(a, n, lds_bytes, s);
-        else launch_wh<false, kWhThreads, kWhPmax>(a, n, lds_bytes, s);
-    }
+    if (t->cz) launch_wh<true, kWhThreads>(a, t->nt, n, lds_bytes, s);
+    else launch_wh<false, kWhThreads>(a, t->nt, n, lds_bytes, s);
     return true;
 }
 

@@ -85,8 +85,9 @@ __device__ __forceinline__ double interp_A(double a, double b, double c)
 
 // dynamic_indicator.cpp:139-176 on magnitudes mag[0..N): first maximum wins
 // `mag(k)` gives the magnitude of spectrum entry k.
+// and cos_n, sin_n are those of 2 pi / N.
 template <class Mag>
-__device__ double interp_tune_at(Mag mag, uint32_t N, uint32_t index)
+__device__ double interp_tune_at(Mag mag, uint32_t N, uint32_t index, double cos_n, double sin_n)
 {
     const double Nd = (double)N;
     if (index == 0) return 1.0;
@@ -98,9 +99,13 @@ __device__ double interp_tune_at(Mag mag, uint32_t N, uint32_t index)
         i1 = index; i2 = index + 1;
     }
     const double value = ((double)index / Nd) +
-                         (1.0 / (2.0 * M_PI)) * asin(interp_A(mag(i1), mag(i2), cos(2.0 * M_PI / Nd)) *
-                                                     sin(2.0 * M_PI / Nd));
+                         (1.0 / (2.0 * M_PI)) * asin(interp_A(mag(i1), mag(i2), cos_n) * sin_n);
     return fabs(1.0 - value);
+}
+template <class Mag>
+__device__ double interp_tune_at(Mag mag, uint32_t N, uint32_t index)
+{
+    return interp_tune_at(mag, N, index, cos(2.0 * M_PI / (double)N), sin(2.0 * M_PI / (double)N));
 }
 
 // FFT tunes of one window of any length N >= 2 (hm_chirpz.hip): Bluestein's
