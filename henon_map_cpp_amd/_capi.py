@@ -71,6 +71,8 @@ SIGNATURES = {
     "hm_mem_info": (I, [ctypes.POINTER(SZ), ctypes.POINTER(SZ)]),
     "hm_malloc": (I, [ctypes.POINTER(P), SZ]),
     "hm_free": (I, [P]),
+    "hm_buffer_take": (I, [ctypes.POINTER(P), SZ]),
+    "hm_buffer_give": (I, [P]),
     "hm_memcpy": (I, [P, P, SZ, I, P]),
     "hm_memset": (I, [P, I, SZ, P]),
     "hm_stream_synchronize": (I, [P]),

@@ -54,7 +54,8 @@ void require_device()
 }
 
 // A device allocation owned through the C ABI; move-only (the reference's
-// classes owned raw device pointers with implicit copies).
+// classes owned raw device pointers with implicit copies). Its contents start
+// undefined, and all work on it is on the null stream.
 class DevBuf {
   public:
     DevBuf() = default;
@@ -76,7 +77,7 @@ class DevBuf {
     void alloc(size_t bytes)
     {
         release();
-        check(hm_malloc(&p_, bytes ? bytes : 8));
+        check(hm_buffer_take(&p_, bytes));
         bytes_ = bytes;
     }
     template <class T> void upload(const std::vector<T> &v)
@@ -98,7 +99,7 @@ class DevBuf {
   private:
     void release()
     {
-        if (p_) (void)hm_free(p_);
+        if (p_) (void)hm_buffer_give(p_);
         p_ = nullptr;
         bytes_ = 0;
     }
@@ -670,12 +671,16 @@ class HenonTracker {
         // the FFT reads each particle's samples in place
         const size_t row_len = ((size_t)L + 15) / 16 * 16;
         const size_t per = row_len * 32;
-        // as many particles per chunk as half the free device memory holds
-        // (at least 8 GiB): tracking the rows needs many wavefronts
+        // Even chunks of at most 8 GiB of rows, which the next call finds again
+        // (device memory costs 24 ms a GiB the first time), but of 16384 particles
+        // at least where half the free memory holds them: a chunk's tracking takes
+        // about as long as one wavefront per SIMD would, however few it has.
         size_t free_b = 0, total_b = 0;
         check(hm_mem_info(&free_b, &total_b));
-        const size_t budget = std::max<size_t>((size_t)8 << 30, free_b / 2);
-        const size_t chunk = std::max<size_t>(1, std::min<size_t>(p.n_particles, budget / per));
+        const size_t budget = std::max<size_t>((size_t)8 << 30, std::min(free_b / 2, 16384 * per));
+        const size_t most = std::max<size_t>(1, std::min<size_t>(p.n_particles, budget / per));
+        const size_t n_chunks = std::max<size_t>(1, (p.n_particles + most - 1) / most);
+        const size_t chunk = std::max<size_t>(1, (p.n_particles + n_chunks - 1) / n_chunks);
         std::vector<double> birk(p.n_particles * 2 * NW), fft(all ? p.n_particles * 2 * NW : 0);
         DevBuf hist(chunk * per), means(all ? chunk * 32 : 8), ob(chunk * 2 * NW * 8), of(chunk * 2 * NW * 8);
         {
@@ -754,15 +759,13 @@ class HenonTracker {
              chunks(TB, HM_MAX_BIRKHOFF)});
         DevBuf mg(n * S * 8), fl(n * S * 8), mat(n * 128), ls(n * 8), bo(n * 2 * B * 8),
             hi(n * 32 * (size_t)history.second), mbo(n * MB * 8), tbo(n * 4 * TB * 8);
-        std::vector<double> eye(16 * n, 0.0);
-        for (size_t i = 0; i < n; i++) eye[16 * i] = eye[16 * i + 5] = eye[16 * i + 10] = eye[16 * i + 15] = 1.0;
         DevBuf sx(passes > 1 ? n * 8 : 8), spx(passes > 1 ? n * 8 : 8), sy(passes > 1 ? n * 8 : 8),
             spy(passes > 1 ? n * 8 : 8), ss(passes > 1 ? n * 4 : 8);
         if (passes > 1) snapshot(p, sx, spx, sy, spy, ss);
         for (size_t pass = 0; pass < passes; ++pass) {
             if (pass) restore(p, sx, spx, sy, spy, ss);
-            mat.upload(eye);
-            ls.upload(std::vector<double>(n, 0.0));
+            check(hm_matrix_identity(mat.as<double>(), n, nullptr));
+            check(hm_memset(ls.as<void>(), 0, n * 8, nullptr));
             hm_indicator_spec spec{};
             spec.renorm_every = renorm_every;
             for (int q = 0; q < 4; q++) spec.fli_dir[q] = fli_direction[q];

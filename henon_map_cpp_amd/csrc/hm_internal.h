@@ -78,6 +78,9 @@ uint32_t *status_word();
 void *workspace(size_t bytes, int slot);
 // SIMDs of the current device (CUs x 4), cached per device.
 uint32_t device_simds();
+// Device blocks kept between owners (hm_buffer_take, hm_buffer_give).
+void *buffer_take(size_t bytes);
+void buffer_give(void *p);
 
 constexpr size_t kTableRecord = 4;  // doubles per turn in the interleaved table
 
