@@ -255,7 +255,15 @@ extern "C" int hm_track(double *x, double *px, double *y, double *py, uint32_t *
         hipStream_t s = as_stream(stream);
         const uint32_t N = (uint32_t)n;
 
-        if (every < 0 || (uint32_t)every >= n_turns) {
+        // Up to one wavefront per SIMD, compaction frees nothing that another wavefront
+        // waits for: all turns go in one launch (up to about 0.1 s of them) unless the
+        // caller chose. 1e4 particles x 1e4 turns, mu = 0.5, r < 0.4: 0.89 -> 0.81 ms;
+        // 32768 x 1e5: 9.4 -> 8.5; 65536 x 1e5, r < 0.7, two thirds lost: 9.5 -> 8.5
+        // (r < 0.4, 2 % lost: 10.6 -> 10.9). With two wavefronts per SIMD it depends on
+        // the losses (131072 x 1e4: 1.82 -> 1.61 ms with few, 0.99 -> 1.01 with most).
+        const bool chosen = cfg && cfg->compact_every;
+        const bool one_launch = !chosen && (N + 63u) / 64u <= device_simds() && n_turns <= (1u << 20);
+        if (one_launch || every < 0 || (uint32_t)every >= n_turns) {
             a.n_arg = a.grid_bound = N;
             a.n_turns = n_turns;
             pick_track(mode, inverse != 0, mu)(a, s);

@@ -202,12 +202,16 @@ __device__ __forceinline__ void track_wave(const TrackArgs &A, uint32_t base, ui
                 if (__builtin_expect((live & not_below(r2, safe1)) == 0, 1)) {
                     turn(t1);
                 } else {
-                    if (kk) {
-                        const TabEntry t = rec(kk - 1);
-                        const double z = 0.0 * ((t.sx + t.cx) + (t.sy + t.cy));
-                        settle(z == 0.0 ? kk : kk - 1);
-                    } else {
-                        settle(kk);
+                    if (live & not_below(r2, b2s)) {
+                        // (read for a loss alone: a chaotic orbit can stay beyond
+                        // safe1 for thousands of turns)
+                        if (kk) {
+                            const TabEntry t = rec(kk - 1);
+                            const double z = 0.0 * ((t.sx + t.cx) + (t.sy + t.cy));
+                            settle(z == 0.0 ? kk : kk - 1);
+                        } else {
+                            settle(kk);
+                        }
                     }
                     checked(t1, kk + 1);
                 }

@@ -112,7 +112,8 @@ int hm_birkhoff_weights(uint32_t n_weights, double *out);
 typedef struct hm_launch_cfg {
     int32_t block;              /* threads per workgroup: 64, 128, 192 or 256 (0 = 64 up to one
                                    wavefront per SIMD, 256 beyond) */
-    int32_t compact_every;      /* turns between loss compactions (0 = 1000, <0 = never); segments
+    int32_t compact_every;      /* turns between loss compactions (<0 = never; 0 = 1000, or never where
+                                   the particles leave a SIMD no more than one wavefront); segments
                                    start at 125 turns and double up to this */
     int32_t particles_per_lane; /* 0, 1 or 2, for callers that set it: every launch takes one
                                    particle per lane */
