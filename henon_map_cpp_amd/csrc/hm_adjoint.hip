@@ -25,6 +25,7 @@
 
 #include "hm_device.h"
 #include "hm_internal.h"
+#include "hm_wave.h"
 
 namespace hm {
 
@@ -37,7 +38,7 @@ struct AdjointFwdArgs {
     uint32_t n;
     const TabEntry *tab;
     uint32_t n_turns, every;  // T, K
-    double mu, b2;
+    double mu, b2, safe1;     // safe1: see safe_radius2
     const double *weights;    // [T] birkhoff_weights(T)
     double *ckpt;             // [T/K + 1][4][n]
     double *final_state;      // [4][n]
@@ -45,24 +46,22 @@ struct AdjointFwdArgs {
     uint8_t *alive;           // [n]
 };
 
-// LDS ring of the aligned forward sweep, one per wavefront: three 8-turn
-// chunks, per turn sx cx sy cy | weight, pad.
-constexpr int kFwdTurn = 6;
-constexpr int kFwdChunk = 8 * kFwdTurn;
-constexpr int kFwdWave = 3 * kFwdChunk;
 constexpr int kFwdBlock = 256;
 
 // Every lane runs every turn (a lost particle's lane carries on with values
 // that are discarded), so the table record and the weight of a turn are
 // wave-uniform. A lost particle is parked at the origin, a fixed point of the
 // map, so that its lane never again takes the loss test's rare path.
-// With every % 8 == 0 (ALIGNED) the turns run in 8-turn chunks whose table
-// records and weights the wavefront stages into its LDS ring two chunks ahead
-// (one vector load and one LDS store per lane and chunk); a turn reads its
-// entries from LDS one turn ahead, so neither scalar-cache misses nor LDS
-// latency sit on the dependency chain. Otherwise the turns run four at a time
-// with scalar loads of two alternating prefetched pairs of records.
-template <int MODE, bool OCT, bool ALIGNED>
+// With every % 8 == 0 (ALIGNED) the turns run eight to a pass of the loop, in pairs
+// with one loss test as the tracking kernel's (a point below safe1 after the first
+// turn is inside the barrier after the second), records and weights requested a pair
+// ahead by scalar loads and touched 64 to 128 turns ahead by a vector load. Otherwise
+// the turns run four at a time with scalar loads of two alternating prefetched pairs
+// of records and a test each.
+// With a test a turn and the records in an LDS ring before: 1e4 turns, mu = 0.5, exact, 1000 particles 1.17 -> 0.82 ms, 32768 1.20 ->
+// 0.98, 65536 1.36 -> 1.20, and 200000 x 4000 1.49 -> 1.20. At full load the chip's
+// power sets the pace: 34 FP64 operations a turn.
+template <int MODE, int OCT, bool ALIGNED>
 __global__ void __launch_bounds__(kFwdBlock) k_adjoint_forward(AdjointFwdArgs a)
 {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -95,9 +94,9 @@ __global__ void __launch_bounds__(kFwdBlock) k_adjoint_forward(AdjointFwdArgs a)
     auto turn = [&](const TabEntry &t, double w) {
         bool cand;
         if (MODE == kExact) {
-            cand = !(fwd_exact_carry<OCT>(x, px, y, py, xx, yy, mu, t) < b2s);
+            cand = !(fwd_exact_carry<OCT != 0>(x, px, y, py, xx, yy, mu, t) < b2s);
         } else {
-            map_step<kFast, false, OCT>(x, px, y, py, mu, m3mu, t);
+            map_step<kFast, false, OCT != 0>(x, px, y, py, mu, m3mu, t);
             cand = !(radius2<kFast>(x, px, y, py) < b2);
         }
         if (__builtin_expect(__any(cand), 0)) {
@@ -116,66 +115,98 @@ __global__ void __launch_bounds__(kFwdBlock) k_adjoint_forward(AdjointFwdArgs a)
     };
     const uint32_t T = a.n_turns, K = a.every;
     if constexpr (ALIGNED) {
-        __shared__ __align__(16) double ring_all[(kFwdBlock / 64) * kFwdWave];
-        double *ring = ring_all + (threadIdx.x >> 6) * kFwdWave;
-        const uint32_t lane = threadIdx.x & 63;
-        const int G = (int)((T + 7) / 8);
-        const double *tabd = reinterpret_cast<const double *>(a.tab);
-        // chunk g: lane l < 32 carries table double l (turn l/4), the others the
-        // weight of turn l % 8 (identical writes); turns past T read turn T-1
-        auto stage_load = [&](int g) -> double {
-            const uint32_t t0 = (uint32_t)g * 8;
-            return lane < 32 ? tabd[4 * (size_t)umin(t0 + (lane >> 2), T - 1) + (lane & 3)]
-                             : a.weights[umin(t0 + (lane & 7), T - 1)];
+        double r2 = 0.0;
+        auto plain_turn = [&](const TabEntry &t) {
+            if (MODE == kExact) fwd_exact_fused<OCT>(x, px, y, py, xx, yy, mu, t);
+            else map_step<kFast, false, OCT != 0>(x, px, y, py, mu, m3mu, t);
         };
-        auto stage_store = [&](int g, double e) {
-            double *slot = ring + ((uint32_t)g % 3) * kFwdChunk;
-            slot[lane < 32 ? (lane >> 2) * kFwdTurn + (lane & 3) : (lane & 7) * kFwdTurn + 4] = e;
+        auto radius = [&] {
+            r2 = MODE == kExact ? fma(px, px, xx) + fma(py, py, yy) : radius2<kFast>(x, px, y, py);
         };
-        auto ring_at = [&](int g, int m, TabEntry &t, double &w) {
-            const double *q = ring + ((uint32_t)g % 3) * kFwdChunk + m * kFwdTurn;
-            t = TabEntry{q[0], q[1], q[2], q[3]};
-            w = q[4];
+        auto park = [&] {
+            const bool lost =
+                !(r2 < (MODE == kExact ? b2s : b2)) && (MODE != kExact || !(exact_radius2(xx, px, yy, py) < b2));
+            if (lost) {
+                alive = false;
+                x = px = y = py = xx = yy = 0.0;
+            }
         };
-        auto clampg = [&](int g) { return g < G ? g : G - 1; };
-        stage_store(0, stage_load(0));
-        stage_store(clampg(1), stage_load(clampg(1)));
-        double e = stage_load(clampg(2));
-        __builtin_amdgcn_wave_barrier();
-        const uint32_t K8 = K / 8;
+        auto sum = [&](double w) { bsum = fma(w, MODE == kExact ? xx : x * x, bsum); };
+        const double safe1 = a.safe1;
+        auto pair = [&](const TabEntry &t0, const TabEntry &t1, double w0, double w1) {
+            plain_turn(t0);
+            radius();
+            if (__builtin_expect(not_below(r2, safe1) == 0, 1)) {
+                sum(w0);
+                plain_turn(t1);
+            } else {
+                park();
+                sum(w0);
+                plain_turn(t1);
+                radius();
+                park();
+            }
+            sum(w1);
+        };
+        // the fused forms need every coordinate zero or at least kTinyCoord
+        auto small = [](double v) { return v != 0.0 && fabs(v) < kTinyCoord; };
+        const bool fused = MODE != kExact || !__any(small(x) || small(px) || small(y) || small(py));
+        const uint32_t pairs_end = fused ? T / 8 * 8 : 0, lane = threadIdx.x & 63;
         double *ck = a.ckpt;
-        uint32_t to_ck = 0;  // chunks until the next checkpoint
-        TabEntry r;
-        double w;
-        ring_at(0, 0, r, w);
-        for (int g = 0; g < G; ++g) {
+        uint32_t to_ck = 0;  // turns until the next checkpoint
+        uint32_t k = 0;
+        if (pairs_end) {
+            const uint32_t last = pairs_end - 2;
+            TabEntry a0 = load_record(tab), a1 = load_record(tab + 1), b0, b1;
+            double wa0 = weights[0], wa1 = weights[1], wb0, wb1;
+            uint32_t touched = 0, touched_w = 0;
+            auto touch = [&](uint32_t from) {
+                const uint32_t kk = umin(from + lane, T - 1);
+                asm volatile("" ::"v"(touched), "v"(touched_w));
+                touched = *reinterpret_cast<const uint32_t *>(a.tab + kk);
+                touched_w = *reinterpret_cast<const uint32_t *>(a.weights + kk);
+            };
+            touch(0);
+            for (; k < pairs_end; k += 8) {
+                if (to_ck == 0) {
+                    checkpoint(ck);
+                    ck += 4 * n;
+                    to_ck = K;
+                }
+                to_ck -= 8;
+                if (k % 64 == 0) touch(k + 64);
+#pragma unroll
+                for (uint32_t q = 0; q < 8; q += 4) {
+                    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): this pair's entries
+                    __builtin_amdgcn_sched_barrier(0);
+                    b0 = load_record(tab + (k + q + 2));
+                    b1 = load_record(tab + (k + q + 3));
+                    wb0 = weights[k + q + 2];
+                    wb1 = weights[k + q + 3];
+                    __builtin_amdgcn_sched_barrier(0);
+                    pair(a0, a1, wa0, wa1);
+                    const uint32_t nx = umin(k + q + 4, last);
+                    __builtin_amdgcn_s_waitcnt(0xC07F);
+                    __builtin_amdgcn_sched_barrier(0);
+                    a0 = load_record(tab + nx);
+                    a1 = load_record(tab + nx + 1);
+                    wa0 = weights[nx];
+                    wa1 = weights[nx + 1];
+                    __builtin_amdgcn_sched_barrier(0);
+                    pair(b0, b1, wb0, wb1);
+                }
+            }
+            radius();  // the last turn may have gone untested
+            park();
+        }
+        for (; k < T; ++k) {
             if (to_ck == 0) {
                 checkpoint(ck);
                 ck += 4 * n;
-                to_ck = K8;
+                to_ck = K;
             }
             --to_ck;
-            stage_store(clampg(g + 2), e);
-            e = stage_load(clampg(g + 3));
-            __builtin_amdgcn_wave_barrier();  // the stores precede later chunks' reads
-            const uint32_t len = umin(8, T - (uint32_t)g * 8);
-            if (len == 8) {
-#pragma unroll
-                for (int m = 0; m < 8; ++m) {
-                    TabEntry rn;
-                    double wn;
-                    if (m + 1 < 8) ring_at(g, m + 1, rn, wn);
-                    else ring_at(g + 1, 0, rn, wn);  // the next chunk's (its slot is staged)
-                    turn(r, w);
-                    r = rn;
-                    w = wn;
-                }
-            } else {
-                for (uint32_t m = 0; m < len; ++m) {
-                    ring_at(g, (int)m, r, w);
-                    turn(r, w);
-                }
-            }
+            turn(load_record(tab + k), weights[k]);
         }
     } else {
         double *ck = a.ckpt;
@@ -226,7 +257,7 @@ struct AdjAcc {
 
 template <bool OCT>
 __device__ __forceinline__ void adjoint_turn(const double (&pre)[4], const double (&post)[4], const TabEntry &t,
-                                             double bw, const double4 &dt, double mu3, double mu6, AdjAcc &a)
+                                             double bw, const double4 &dt, double mu3, AdjAcc &a)
 {
     // Birkhoff seed of sample k+1: d/dx_{k+1} of c w_k x_{k+1}^2 (bw = 2 c w_k)
     a.lx = fma(bw, post[0], a.lx);
@@ -237,15 +268,25 @@ __device__ __forceinline__ void adjoint_turn(const double (&pre)[4], const doubl
     a.g_wy = fma(dwy, dt.z, a.g_wy);
     a.g_eps = fma(dwx, dt.y, fma(dwy, dt.w, a.g_eps));
     // through the rotations
-    const double lxt = fma(t.cx, a.lx, -t.sx * a.lpx), lpt = fma(t.sx, a.lx, t.cx * a.lpx);
-    const double lyt = fma(t.cy, a.ly, -t.sy * a.lpy), lqt = fma(t.sy, a.ly, t.cy * a.lpy);
-    // through the kicks, at the pre-step point
-    const double x = pre[0], y = pre[2], xx = x * x, yy = y * y;
-    if (OCT) a.g_mu = fma(lpt, x * fma(-3.0, yy, xx), fma(lqt, y * fma(-3.0, xx, yy), a.g_mu));
-    const double ja = fma(mu3, xx - yy, 2.0 * x);
-    const double jb = fma(-mu6 * x, y, -2.0 * y);
-    a.lx = fma(ja, lpt, fma(jb, lqt, lxt));
-    a.ly = fma(jb, lpt, fma(-ja, lqt, lyt));
+    double lxt = fma(t.cx, a.lx, -t.sx * a.lpx), lyt = fma(t.cy, a.ly, -t.sy * a.lpy);
+    const double lpt = fma(t.sx, a.lx, t.cx * a.lpx), lqt = fma(t.sy, a.ly, t.cy * a.lpy);
+    // Through the kicks, at the pre-step point: with z = x + i y they are z^2 + mu z^3,
+    // the real part on p_x, minus the imaginary part on p_y, so with l = l_px + i l_py
+    // the adjoint takes 2 z l + 3 mu z^2 l and the derivative by mu is Re z^3 l. The
+    // three products z l, z^2 l, z^3 l share their factors: 14 operations for the 18
+    // of the partial derivatives one by one.
+    const double x = pre[0], y = pre[2];
+    const double ar = fma(x, lpt, -(y * lqt)), ai = fma(y, lpt, x * lqt);
+    lxt = fma(2.0, ar, lxt);
+    lyt = fma(-2.0, ai, lyt);
+    if (OCT) {
+        const double br = fma(x, ar, -(y * ai)), bi = fma(x, ai, y * ar);
+        a.g_mu = fma(x, br, fma(-y, bi, a.g_mu));
+        lxt = fma(mu3, br, lxt);
+        lyt = fma(-mu3, bi, lyt);
+    }
+    a.lx = lxt;
+    a.ly = lyt;
     a.lpx = lpt;
     a.lpy = lqt;
 }
@@ -275,8 +316,8 @@ struct AdjRec {
 //    checkpoint, one thread per (particle, segment), and writes the state at the
 //    start of each 8-turn chunk after the first (sub-checkpoints). The segments
 //    are independent, so this part runs at full occupancy even for few particles.
-//  - the sweep (k_adjoint_sweep_fused for every % 8 == 0, else k_adjoint_sweep),
-//    one thread per particle, walks the window's chunks in reverse: the chunk's
+//  - the sweep (for every % 8 == 0 k_adjoint_sweep_split up to half a wavefront per
+//    SIMD and k_adjoint_sweep_fused beyond, else k_adjoint_sweep), a lane per particle, walks the window's chunks in reverse: the chunk's
 //    nine states S0..S8 (S8 = the next chunk's S0) come from its sub-checkpoint
 //    (the segment's checkpoint for a first chunk), and the adjoint runs back
 //    through its turns. The states of the chunk before it are recomputed in the
@@ -364,7 +405,7 @@ __global__ void __launch_bounds__(256) k_adjoint_sweep(AdjointSweepArgs a)
                      a.grad_p[i],  a.grad_p[n + i],  a.grad_p[2 * n + i],  a.grad_p[3 * n + i]};
     }
     const double bseed = 2.0 * (a.seed_b ? a.seed_b[i] : 0.0);
-    const double mu = a.mu, m3mu = -3.0 * mu, mu3 = 3.0 * mu, mu6 = 6.0 * mu;
+    const double mu = a.mu, m3mu = -3.0 * mu, mu3 = 3.0 * mu;
     const uint32_t T = a.n_turns, K = a.every;
     const uint32_t n_seg = (T + K - 1) / K;
     const ConstPtr<TabEntry> tab = as_const(a.tab);
@@ -375,7 +416,7 @@ __global__ void __launch_bounds__(256) k_adjoint_sweep(AdjointSweepArgs a)
     auto adjoint_at = [&](uint32_t k, const double (&pre)[4], const double (&post)[4]) {
         const ConstPtr<double> d = dtab + 4 * (size_t)k;
         const double4 dt{d[0], d[1], d[2], d[3]};
-        adjoint_turn<OCT>(pre, post, load_record(tab + k), bseed * weights[k], dt, mu3, mu6, acc);
+        adjoint_turn<OCT>(pre, post, load_record(tab + k), bseed * weights[k], dt, mu3, acc);
     };
     auto fill = [&](double (&S)[kChunk][4], uint32_t c0, uint32_t len) {
 #pragma unroll
@@ -484,7 +525,7 @@ __global__ void __launch_bounds__(kFusedBlock) k_adjoint_sweep_fused(AdjointSwee
         for (int c = 0; c < 4; c++) { a.grad_x0[c * n + i] = 0.0; a.grad_p[c * n + i] = 0.0; }
     if (!__any(live)) return;  // the whole wavefront
 
-    const double mu = a.mu, m3mu = -3.0 * mu, mu3 = 3.0 * mu, mu6 = 6.0 * mu;
+    const double mu = a.mu, m3mu = -3.0 * mu, mu3 = 3.0 * mu;
     const uint32_t T = a.n_turns, K = a.every;
     const uint32_t n_seg = (T + K - 1) / K;
     const uint32_t K8 = K / kChunk;
@@ -607,10 +648,10 @@ __global__ void __launch_bounds__(kFusedBlock) k_adjoint_sweep_fused(AdjointSwee
             const ConstPtr<double> d = dtab + 4 * (size_t)k;
             const double4 dt{d[0], d[1], d[2], d[3]};
             if ((uint32_t)m + 1 == lent)
-                adjoint_turn<OCT>(S[m], nxt, load_record(tab + k), bseed * weights[k], dt, mu3, mu6, acc);
+                adjoint_turn<OCT>(S[m], nxt, load_record(tab + k), bseed * weights[k], dt, mu3, acc);
             else
                 adjoint_turn<OCT>(S[m], S[m + 1 < kChunk ? m + 1 : m], load_record(tab + k), bseed * weights[k], dt,
-                                  mu3, mu6, acc);
+                                  mu3, acc);
         }
         copy4(nxt, S[0]);
     }
@@ -637,7 +678,7 @@ __global__ void __launch_bounds__(kFusedBlock) k_adjoint_sweep_fused(AdjointSwee
             TabEntry rpn{};
             if (m > 0) rcn = rec_c(g, m - 1);
             if (j + 2 < kChunk) rpn = rec_p(gp, j + 1);
-            adjoint_turn<OCT>(X[m], post, rc.t, bseed * rc.w, rc.dt, mu3, mu6, acc);
+            adjoint_turn<OCT>(X[m], post, rc.t, bseed * rc.w, rc.dt, mu3, acc);
             copy4(post, X[m]);
             if (j + 1 < kChunk) {
                 copy4(Y[j + 1], Y[j]);
@@ -662,17 +703,225 @@ __global__ void __launch_bounds__(kFusedBlock) k_adjoint_sweep_fused(AdjointSwee
     a.grad_p[i] = acc.g_eps; a.grad_p[n + i] = acc.g_mu; a.grad_p[2 * n + i] = acc.g_wx; a.grad_p[3 * n + i] = acc.g_wy;
 }
 
+// The same sweep for at most half as many wavefronts as SIMDs: the two chains go to
+// two wavefronts of one workgroup on SIMDs of their own. The producer recomputes the
+// states of a chunk from its sub-checkpoint and stores them in LDS, the consumer runs
+// the adjoint back through the chunk above it, with one workgroup barrier a chunk and
+// two chunks of states per pair of wavefronts (32 KiB). Table records, derivatives
+// and weights are uniform and come by scalar loads a pair of turns ahead; the
+// consumer's lanes touch those of 64 to 128 turns ahead. Same operations in the same
+// order, so the same results. Two pairs a workgroup, one wavefront on each SIMD of a
+// CU. Backward pass of 1e4 turns: 8192 particles 1.70 -> 1.15 ms, 32768 2.03 -> 1.57;
+// with more wavefronts than that the chip's power sets the pace, not the issue of
+// single wavefronts (65536: 2.74 ms in one wavefront, 2.87 in two).
+// Wavefronts w < pairs (pairs = half the workgroup's) are consumers, w + pairs their
+// producers.
+constexpr int kSplitChunk = kChunk * 2 * 64;  // double2 entries: [turn][x px | y py][lane]
+
 template <int MODE, bool OCT>
-static void launch_forward(bool aligned, uint32_t grid, hipStream_t s, const AdjointFwdArgs &a)
+__global__ void __launch_bounds__(256) k_adjoint_sweep_split(AdjointSweepArgs a)
 {
-    if (aligned) hipLaunchKernelGGL((k_adjoint_forward<MODE, OCT, true>), dim3(grid), dim3(kFwdBlock), 0, s, a);
-    else hipLaunchKernelGGL((k_adjoint_forward<MODE, OCT, false>), dim3(grid), dim3(kFwdBlock), 0, s, a);
+    extern __shared__ double2 states_all[];
+    const uint32_t pairs = blockDim.x / 128;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const bool consumer = wave < pairs;
+    const uint32_t pair = consumer ? wave : wave - pairs;
+    double2 *const states = states_all + (size_t)pair * 2 * kSplitChunk + lane;
+    const uint32_t i = (blockIdx.x * pairs + pair) * 64 + lane;
+    const size_t n = a.n;
+    // lanes past n read particle n-1; lost particles compute on parked or stale
+    // states; only live lanes store
+    const uint32_t ic = i < a.n ? i : a.n - 1;
+    const bool live = i < a.n && a.alive[ic];
+    if (consumer && !live && i < a.n && a.last_window)
+        for (int c = 0; c < 4; c++) { a.grad_x0[c * n + i] = 0.0; a.grad_p[c * n + i] = 0.0; }
+    if (!__syncthreads_or(live)) return;  // the whole workgroup
+
+    const double mu = a.mu, m3mu = -3.0 * mu, mu3 = 3.0 * mu;
+    const uint32_t T = a.n_turns, K = a.every;
+    const uint32_t n_seg = (T + K - 1) / K;
+    const uint32_t K8 = K / kChunk;
+    const uint32_t G = (T + kChunk - 1) / kChunk;
+    const int g_lo = (int)(a.seg_first * K8);
+    const int gt = (int)umin(a.seg_end * K8, G) - 1;
+    const int steps = gt - g_lo;  // full chunks below the top one
+    const double *sub_base = a.sub ? a.sub : a.ckpt;
+    auto load4 = [&](const double *p, double (&v)[4]) {
+        v[0] = p[ic]; v[1] = p[n + ic]; v[2] = p[2 * n + ic]; v[3] = p[3 * n + ic];
+    };
+    auto start_of = [&](int g) -> const double * {
+        const uint32_t seg = (uint32_t)g / K8, j = (uint32_t)g - seg * K8;
+        return j == 0 ? a.ckpt + (size_t)seg * 4 * n
+                      : sub_base + ((size_t)(seg - a.seg_first) * (K8 - 1) + j - 1) * 4 * n;
+    };
+    const ConstPtr<TabEntry> tab = as_const(a.tab);
+
+    if (!consumer) {
+        // chunk gt - c goes to half c % 2 while the consumer reads the other
+        double P[4];
+        if (steps > 0) load4(start_of(gt - 1), P);
+        TabEntry t0 = load_record(tab + (size_t)(steps > 0 ? gt - 1 : gt) * kChunk), t1{};
+        for (int c = 1; c <= steps; ++c) {
+            const int g = gt - c;
+            const uint32_t k = (uint32_t)g * kChunk, kn = (uint32_t)(g > g_lo ? g - 1 : g) * kChunk;
+            double v[4], Q[4];
+            copy4(v, P);
+            load4(start_of(g > g_lo ? g - 1 : g), Q);  // used by the next chunk
+            double2 *out = states + (size_t)(c & 1) * kSplitChunk;
+#pragma unroll
+            for (int m = 0; m < kChunk; ++m) {
+                __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): this turn's record
+                __builtin_amdgcn_sched_barrier(0);
+                t1 = load_record(tab + (m + 1 < kChunk - 1 ? k + m + 1 : kn));
+                out[(2 * m) * 64] = double2{v[0], v[1]};
+                out[(2 * m + 1) * 64] = double2{v[2], v[3]};
+                __builtin_amdgcn_sched_barrier(0);
+                if (m + 1 < kChunk) step4<MODE, OCT>(v, mu, m3mu, t0);
+                if (m + 1 < kChunk) t0 = t1;
+            }
+            copy4(P, Q);
+            __syncthreads();
+        }
+        return;
+    }
+
+    AdjAcc acc;
+    if (a.last_window) {
+        acc = AdjAcc{a.seed_s[ic], a.seed_s[n + ic], a.seed_s[2 * n + ic], a.seed_s[3 * n + ic], 0.0, 0.0, 0.0, 0.0};
+    } else {
+        acc = AdjAcc{a.grad_x0[ic], a.grad_x0[n + ic], a.grad_x0[2 * n + ic], a.grad_x0[3 * n + ic],
+                     a.grad_p[ic],  a.grad_p[n + ic],  a.grad_p[2 * n + ic],  a.grad_p[3 * n + ic]};
+    }
+    const double bseed = 2.0 * (a.seed_b ? a.seed_b[ic] : 0.0);
+    const ConstPtr<double> dtab = as_const(a.dtab), weights = as_const(a.weights);
+    auto record = [&](uint32_t k) -> AdjRec {
+        const ConstPtr<double> d = dtab + 4 * (size_t)k;
+        return AdjRec{load_record(tab + k), double4{d[0], d[1], d[2], d[3]}, weights[k]};
+    };
+    uint32_t touched[3] = {};
+    auto touch = [&](uint32_t k) {  // the records of the 64 turns below turn k
+        asm volatile("" ::"v"(touched[0]), "v"(touched[1]), "v"(touched[2]));
+        const uint32_t q = k > lane ? k - 1 - lane : 0;
+        touched[0] = *reinterpret_cast<const uint32_t *>(a.tab + q);
+        touched[1] = *reinterpret_cast<const uint32_t *>(a.dtab + 4 * (size_t)q);
+        touched[2] = *reinterpret_cast<const uint32_t *>(a.weights + q);
+    };
+    double nxt[4];
+    {
+        // the top chunk, possibly short, from its own start
+        const uint32_t ct = (uint32_t)gt * kChunk, lent = umin(kChunk, T - ct);
+        touch(ct);
+        double S[kChunk][4];
+        load4(start_of(gt), S[0]);
+#pragma unroll
+        for (int m = 1; m < kChunk; ++m) {
+            copy4(S[m], S[m - 1]);
+            if ((uint32_t)m < lent) step4<MODE, OCT>(S[m], mu, m3mu, load_record(tab + ct + m - 1));
+        }
+        if (a.seg_end < n_seg) {
+            load4(a.ckpt + (size_t)a.seg_end * 4 * n, nxt);  // the state after the window
+        } else {
+            double v[4];
+#pragma unroll
+            for (int m = 0; m < kChunk; ++m)
+                if ((uint32_t)m + 1 == lent) copy4(v, S[m]);
+            step4<MODE, OCT>(v, mu, m3mu, load_record(tab + T - 1));
+            copy4(nxt, v);
+        }
+#pragma unroll
+        for (int m = kChunk - 1; m >= 0; --m) {
+            if ((uint32_t)m >= lent) continue;
+            const AdjRec r = record(ct + m);
+            adjoint_turn<OCT>(S[m], nxt, r.t, bseed * r.w, r.dt, mu3, acc);
+            copy4(nxt, S[m]);
+        }
+    }
+    // Two turns' records and states; the next two are requested before these are
+    // used, all at once, as scalar and LDS loads are waited for together. The states
+    // of a chunk's last two turns read, the next chunk may be waited for and the
+    // producer may write over this one.
+    struct Two {
+        AdjRec r1, r0;
+        double2 s[4];
+    };
+    uint32_t k = (uint32_t)gt * kChunk;  // turns from here on are requested
+    auto fetch = [&](int c, int m) {
+        const double2 *in = states + (size_t)(c & 1) * kSplitChunk;
+        Two t{record(k - 1), record(k - 2), {}};
+#pragma unroll
+        for (int q = 0; q < 4; ++q) t.s[q] = in[(2 * (m - 1) + q) * 64];
+        k -= 2;
+        return t;
+    };
+    auto back = [&](const Two &t) {
+        const double post1[4] = {t.s[2].x, t.s[2].y, t.s[3].x, t.s[3].y};
+        const double post0[4] = {t.s[0].x, t.s[0].y, t.s[1].x, t.s[1].y};
+        adjoint_turn<OCT>(post1, nxt, t.r1.t, bseed * t.r1.w, t.r1.dt, mu3, acc);
+        adjoint_turn<OCT>(post0, post1, t.r0.t, bseed * t.r0.w, t.r0.dt, mu3, acc);
+        copy4(nxt, post0);
+    };
+    auto arrived = [] {
+        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    if (steps > 0) {
+        __syncthreads();
+        Two A = fetch(1, kChunk - 1), B;
+        for (int c = 1;; ++c) {
+            arrived();
+            if (c % 8 == 1) touch(k > 64 ? k - 64 : 0);
+            B = fetch(c, kChunk - 3);
+            __builtin_amdgcn_sched_barrier(0);
+            back(A);
+            arrived();
+            A = fetch(c, kChunk - 5);
+            __builtin_amdgcn_sched_barrier(0);
+            back(B);
+            arrived();
+            B = fetch(c, kChunk - 7);
+            __builtin_amdgcn_sched_barrier(0);
+            back(A);
+            arrived();
+            if (c == steps) break;
+            __syncthreads();
+            A = fetch(c + 1, kChunk - 1);
+            __builtin_amdgcn_sched_barrier(0);
+            back(B);
+        }
+        back(B);
+    }
+    if (!live) return;
+    a.grad_x0[i] = acc.lx; a.grad_x0[n + i] = acc.lpx; a.grad_x0[2 * n + i] = acc.ly; a.grad_x0[3 * n + i] = acc.lpy;
+    a.grad_p[i] = acc.g_eps; a.grad_p[n + i] = acc.g_mu; a.grad_p[2 * n + i] = acc.g_wx; a.grad_p[3 * n + i] = acc.g_wy;
+}
+
+// Threads per workgroup: one wavefront up to two per CU, so that they spread over
+// the CUs (forward sweep, 1e4 turns, 16384 particles: 0.83 ms against 1.06); beyond
+// that single wavefronts can come to share a SIMD while another has none (40000
+// particles 1.0 to 1.4 ms, 57344 1.49, against 1.10 and 1.12).
+static uint32_t adjoint_block(size_t n) { return (n + 63) / 64 <= device_simds() / 2 ? 64 : 256; }
+
+template <int MODE, int OCT>
+static void launch_forward(bool aligned, hipStream_t s, const AdjointFwdArgs &a)
+{
+    const uint32_t block = adjoint_block(a.n);
+    const dim3 grid((a.n + block - 1) / block);
+    if (aligned) hipLaunchKernelGGL((k_adjoint_forward<MODE, OCT, true>), grid, dim3(block), 0, s, a);
+    else hipLaunchKernelGGL((k_adjoint_forward<MODE, OCT, false>), grid, dim3(block), 0, s, a);
 }
 
 template <int MODE, bool OCT>
 static void launch_sweep(bool aligned, size_t n, hipStream_t s, const AdjointSweepArgs &w)
 {
-    if (aligned)
+    const uint32_t waves = (uint32_t)((n + 63) / 64);
+    if (aligned && waves <= device_simds() / 2) {
+        const uint32_t pairs = 2;
+        const size_t lds = (size_t)pairs * 2 * kSplitChunk * sizeof(double2);
+        const auto k = k_adjoint_sweep_split<MODE, OCT>;
+        hip_check(hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds),
+                  "hipFuncSetAttribute");
+        hipLaunchKernelGGL(k, dim3((waves + pairs - 1) / pairs), dim3(128 * pairs), lds, s, w);
+    } else if (aligned)
         hipLaunchKernelGGL((k_adjoint_sweep_fused<MODE, OCT>), dim3((uint32_t)((n + kFusedBlock - 1) / kFusedBlock)),
                            dim3(kFusedBlock), 0, s, w);
     else hipLaunchKernelGGL((k_adjoint_sweep<MODE, OCT>), dim3((uint32_t)((n + 255) / 256)), dim3(256), 0, s, w);
@@ -719,18 +968,18 @@ extern "C" int hm_adjoint_forward(const double *x0, const double *px0, const dou
         if (n > UINT32_MAX) throw Error(HM_ERR_RANGE, "adjoint: too many particles");
         every = std::min(every, n_turns);  // one segment either way
         AdjointFwdArgs a{x0, px0, y0, py0, (uint32_t)n, reinterpret_cast<const TabEntry *>(table), n_turns, every,
-                         mu, barrier * barrier, weights, checkpoints, final_state, birk, alive};
+                         mu, barrier * barrier, safe_radius2(barrier, mu), weights, checkpoints, final_state, birk, alive};
         hipStream_t s = as_stream(stream);
-        const uint32_t grid = (uint32_t)((n + kFwdBlock - 1) / kFwdBlock);
-        const bool oct = mu != 0.0;
+        const int oct = octupole_kind(mode, mu);
         const bool aligned = every % 8 == 0;
         LaunchTimer timer("k_adjoint_forward", s);
         if (mode == HM_MODE_EXACT) {
-            if (oct) launch_forward<kExact, true>(aligned, grid, s, a);
-            else launch_forward<kExact, false>(aligned, grid, s, a);
+            if (oct == 2) launch_forward<kExact, 2>(aligned, s, a);
+            else if (oct) launch_forward<kExact, 1>(aligned, s, a);
+            else launch_forward<kExact, 0>(aligned, s, a);
         } else {
-            if (oct) launch_forward<kFast, true>(aligned, grid, s, a);
-            else launch_forward<kFast, false>(aligned, grid, s, a);
+            if (oct) launch_forward<kFast, 1>(aligned, s, a);
+            else launch_forward<kFast, 0>(aligned, s, a);
         }
         launch_check("k_adjoint_forward");
     });
