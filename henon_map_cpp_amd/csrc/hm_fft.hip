@@ -21,9 +21,11 @@
 #include <mutex>
 #include <vector>
 
+#include "hm_angle.h"
 #include "hm_device.h"
 #include "hm_internal.h"
 #include "hm_tune.h"
+#include "hm_wave.h"
 
 namespace hm {
 
@@ -76,6 +78,12 @@ k_history(double *__restrict__ gx, double *__restrict__ gpx, double *__restrict_
 // samples) instead of touching 64 lines (one per particle). With MEANS each
 // coordinate's samples are also summed in sample order from 0.0 and divided by
 // n_turns + 1: k_means' result on the same rows, without reading them again.
+// Bound by the stores (90000 particles x 1e4 turns are 28.8 GB, 4.3 ms at the rate of
+// a large fill) and, with fewer wavefronts, by the turns' latency: records by scalar
+// loads ahead of their use and losses as a mask instead of a load and three branches
+// per lane and turn, and one wavefront per workgroup: 22500 particles 3.96 -> 2.12 ms,
+// 45000 5.09 -> 2.81, 90000 7.40 -> 6.38. (A test every turn: samples are NaN from
+// the turn of the loss on.)
 template <bool INV, bool OCT, bool MEANS>
 __global__ void __launch_bounds__(256)
 k_history_rows(double *__restrict__ gx, double *__restrict__ gpx, double *__restrict__ gy, double *__restrict__ gpy,
@@ -102,31 +110,15 @@ k_history_rows(double *__restrict__ gx, double *__restrict__ gpx, double *__rest
     const double m3mu = -3.0 * mu;
     const uint32_t samples = n_turns + 1;
     double sum[4] = {0.0, 0.0, 0.0, 0.0};
-    for (uint32_t m0 = 0; m0 < samples; m0 += 16) {
-        double buf[4][16];
-#pragma unroll
-        for (int q = 0; q < 16; ++q) {
-            const uint32_t m = m0 + q;
-            if (m > 0 && m < samples && alive) {
-                const int64_t ti = INV ? (int64_t)s - 1 : (int64_t)s;
-                if (ti < 0 || ti >= (int64_t)tab_len) {
-                    atomicOr(status, 1u);
-                    alive = false;
-                } else {
-                    map_step<kExact, INV, OCT>(x, px, y, py, mu, m3mu, tab[ti]);
-                    if (radius2<kExact>(x, px, y, py) < b2) {
-                        s = INV ? s - 1 : s + 1;
-                    } else {
-                        x = px = y = py = __builtin_nan("");
-                        alive = false;
-                    }
-                }
-            }
-            buf[0][q] = x; buf[1][q] = px; buf[2][q] = y; buf[3][q] = py;
-            if (MEANS && m < samples) {
-                sum[0] = sum[0] + x; sum[1] = sum[1] + px; sum[2] = sum[2] + y; sum[3] = sum[3] + py;
-            }
+    double buf[4][16];
+    auto keep = [&](int q) {
+        buf[0][q] = x; buf[1][q] = px; buf[2][q] = y; buf[3][q] = py;
+        if (MEANS) {
+            sum[0] = sum[0] + x; sum[1] = sum[1] + px; sum[2] = sum[2] + y; sum[3] = sum[3] + py;
         }
+    };
+    // the 16 samples from m0 on
+    auto store = [&](uint32_t m0) {
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
             double2 *mine = reinterpret_cast<double2 *>(tr + lane * kPad);
@@ -143,6 +135,120 @@ k_history_rows(double *__restrict__ gx, double *__restrict__ gpx, double *__rest
                     reinterpret_cast<double2 *>(rows + (size_t)(wave0 + pw) * 4 * L + c * L + m0)[part] = v;
             }
             __builtin_amdgcn_wave_barrier();  // the reads precede the next coordinate's writes
+        }
+    };
+    // All live lanes at one turn index inside the table, and no lane that holds
+    // coordinates without being stepped: the records come by scalar loads, a pair of
+    // turns ahead, and losses are kept as a mask.
+    uint64_t live = __ballot(alive);
+    const uint32_t s0 = live ? __builtin_amdgcn_readlane(s, __builtin_ctzll(live)) : 0;
+    const bool held = !alive && !(__builtin_isnan(x) && __builtin_isnan(px) && __builtin_isnan(y) && __builtin_isnan(py));
+    const bool uniform = live && __all(!alive || s == s0) && !__any(held) &&
+                         (INV ? s0 >= n_turns && s0 <= tab_len : (uint64_t)s0 + n_turns <= (uint64_t)tab_len);
+    if (uniform) {
+        const ConstPtr<TabEntry> tp = as_const(INV ? tab + s0 - 1 : tab + s0);
+        auto rec = [&](uint32_t k) -> TabEntry { return load_record(INV ? tp - k : tp + k); };
+        const double b2s = screen_bound(b2);
+        double xx = x * x, yy = y * y;
+        uint32_t done = n_turns;  // the turn the lane's particle is lost in
+        auto turn = [&](const TabEntry &t, uint32_t k) {
+            double r2;
+            if constexpr (INV) {
+                map_step<kExact, true, OCT>(x, px, y, py, mu, m3mu, t);
+                r2 = screen_radius2(x, px, y, py);
+            } else {
+                r2 = fwd_exact_carry<OCT>(x, px, y, py, xx, yy, mu, t);
+            }
+            if (__builtin_expect((live & not_below(r2, b2s)) != 0, 0)) {
+                const uint64_t lost = live & not_below(exact_radius2(x * x, px, y * y, py), b2);
+                if (lost >> lane & 1) {
+                    done = k;
+                    x = px = y = py = xx = yy = __builtin_nan("");
+                }
+                live &= ~lost;
+            }
+        };
+        uint32_t touched = 0;
+        auto touch = [&](uint32_t from) {
+            const uint32_t k = min(from + lane, n_turns - 1);
+            asm volatile("" ::"v"(touched));
+            touched = *reinterpret_cast<const uint32_t *>(INV ? tab + (s0 - 1 - k) : tab + (s0 + k));
+        };
+        if (n_turns) touch(0);
+        TabEntry a0{}, a1{}, b0{}, b1{};
+        for (uint32_t m0 = 0; m0 < samples; m0 += 16) {
+            if (m0 % 64 == 0 && n_turns) touch(m0 + 64);
+            if (m0 && m0 + 16 <= samples) {
+                // turns m0 - 1 .. m0 + 14 give samples m0 .. m0 + 15
+                const uint32_t k0 = m0 - 1, last = n_turns - 2;
+                if (m0 == 16) {
+                    a0 = rec(k0);
+                    a1 = rec(k0 + 1);
+                }
+#pragma unroll
+                for (int q = 0; q < 16; q += 4) {
+                    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): a0, a1 are there
+                    __builtin_amdgcn_sched_barrier(0);
+                    b0 = rec(k0 + q + 2);
+                    b1 = rec(k0 + q + 3);
+                    __builtin_amdgcn_sched_barrier(0);
+                    turn(a0, k0 + q);
+                    keep(q);
+                    turn(a1, k0 + q + 1);
+                    keep(q + 1);
+                    const uint32_t nx = min(k0 + q + 4, last);
+                    __builtin_amdgcn_s_waitcnt(0xC07F);
+                    __builtin_amdgcn_sched_barrier(0);
+                    a0 = rec(nx);
+                    a1 = rec(nx + 1);
+                    __builtin_amdgcn_sched_barrier(0);
+                    turn(b0, k0 + q + 2);
+                    keep(q + 2);
+                    turn(b1, k0 + q + 3);
+                    keep(q + 3);
+                }
+            } else {
+#pragma unroll
+                for (int q = 0; q < 16; ++q) {
+                    const uint32_t m = m0 + q;
+                    if (m > 0 && m < samples) turn(rec(m - 1), m - 1);
+                    if (m < samples) {
+                        keep(q);
+                    } else {
+                        buf[0][q] = x; buf[1][q] = px; buf[2][q] = y; buf[3][q] = py;
+                    }
+                }
+            }
+            store(m0);
+        }
+        if (alive) s = INV ? s - done : s + done;
+    } else {
+        for (uint32_t m0 = 0; m0 < samples; m0 += 16) {
+#pragma unroll
+            for (int q = 0; q < 16; ++q) {
+                const uint32_t m = m0 + q;
+                if (m > 0 && m < samples && alive) {
+                    const int64_t ti = INV ? (int64_t)s - 1 : (int64_t)s;
+                    if (ti < 0 || ti >= (int64_t)tab_len) {
+                        atomicOr(status, 1u);
+                        alive = false;
+                    } else {
+                        map_step<kExact, INV, OCT>(x, px, y, py, mu, m3mu, tab[ti]);
+                        if (radius2<kExact>(x, px, y, py) < b2) {
+                            s = INV ? s - 1 : s + 1;
+                        } else {
+                            x = px = y = py = __builtin_nan("");
+                            alive = false;
+                        }
+                    }
+                }
+                if (m < samples) {
+                    keep(q);
+                } else {
+                    buf[0][q] = x; buf[1][q] = px; buf[2][q] = y; buf[3][q] = py;
+                }
+            }
+            store(m0);
         }
     }
     if (!in) return;
@@ -225,12 +331,19 @@ __global__ void k_birkhoff_hist(const double *__restrict__ hist, HistLayout h, u
 // differences are summed per lane and then across the wavefront in a fixed
 // order. Same terms as k_birkhoff_hist, summed in that order instead of
 // sample order (within rounding of it).
+// Bound by the angles, two thirds of what the rows' reading would take at full rate:
+// by the table (hm_angle.h) instead of the library 20000 rows of 10001 samples 2.04 ->
+// 1.70 ms (6.4 GB), 40000 of 501 0.235 -> 0.199. The sums' error against long double
+// is the same (rms 1.1e-15 at 2000 samples), that of adding them up.
 __global__ void __launch_bounds__(256) k_birkhoff_rows(const double *__restrict__ rows, uint64_t L, uint32_t n,
                                                        uint32_t p0, uint32_t nb, const double *__restrict__ means,
                                                        WindowSet ws, const double *__restrict__ w_flat,
                                                        double *__restrict__ out)
 {
     // particles p0 .. p0 + nb - 1 of n
+    __shared__ double angle_tab[kAngleBins];
+    fill_angle_table(angle_tab);
+    __syncthreads();
     const uint64_t wave = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
     const uint32_t lane = threadIdx.x & 63;
     const uint32_t i = p0 + (uint32_t)(wave % nb);
@@ -279,7 +392,7 @@ __global__ void __launch_bounds__(256) k_birkhoff_rows(const double *__restrict_
             double th = 0.0;
             if (valid) {
                 bad |= any_nan(a0[u] - mx, a1[u] - mp, 0.0, 0.0);
-                th = atan2(a1[u] - mp, a0[u] - mx);
+                th = angle_of(a1[u] - mp, a0[u] - mx, angle_tab);
             }
             double prev = __shfl_up(th, 1);
             if (lane == 0) prev = carry;
@@ -883,7 +996,9 @@ extern "C" int hm_track_rows(double *x, double *px, double *y, double *py, uint3
         if (reinterpret_cast<uintptr_t>(rows) % 16 != 0) throw Error(HM_ERR_ARG, "history rows: rows not 16-byte aligned");
         if (n > UINT32_MAX) throw Error(HM_ERR_RANGE, "history rows: too many particles");
         hipStream_t s = as_stream(stream);
-        const uint32_t grid = (uint32_t)((n + 255) / 256);
+        // one wavefront per workgroup up to one per SIMD: they spread over all CUs
+        const uint32_t block = (n + 63) / 64 <= device_simds() ? 64 : 256;
+        const uint32_t grid = (uint32_t)((n + block - 1) / block);
         const double b2 = barrier * barrier;
         const TabEntry *tab = reinterpret_cast<const TabEntry *>(table);
         LaunchTimer timer("k_history_rows", s);
@@ -898,7 +1013,7 @@ extern "C" int hm_track_rows(double *x, double *px, double *y, double *py, uint3
             if (oct) k = with_means ? k_history_rows<false, true, true> : k_history_rows<false, true, false>;
             else k = with_means ? k_history_rows<false, false, true> : k_history_rows<false, false, false>;
         }
-        hipLaunchKernelGGL(k, dim3(grid), dim3(256), 0, s, x, px, y, py, steps, (uint32_t)n, tab, (uint32_t)table_len,
+        hipLaunchKernelGGL(k, dim3(grid), dim3(block), 0, s, x, px, y, py, steps, (uint32_t)n, tab, (uint32_t)table_len,
                            n_turns, mu, b2, rows, (uint64_t)row_len, means, status_word());
         launch_check("k_history_rows");
     });
