@@ -133,8 +133,9 @@ __global__ void k_megno_init(double *__restrict__ state, uint64_t n_particles)
     st[18] = 0.0;  // formed from the matrix in the first segment
 }
 
+// Takes chunks of the tracking jobs until the queue holds no more.
 template <int MODE>
-__global__ void __launch_bounds__(256, 8) k_batch_track(BatchSeg S)
+__device__ __forceinline__ void track_chunks(const BatchSeg &S)
 {
     const uint32_t lane = __lane_id();
     // written by the plan launch, read-only here: scalar loads
@@ -177,6 +178,12 @@ __global__ void __launch_bounds__(256, 8) k_batch_track(BatchSeg S)
         else if (MODE == kExact && oct == 2) track_wave<MODE, false, 2>(A, base, n, out);
         else track_wave<MODE, false, 1>(A, base, n, out);
     }
+}
+
+template <int MODE>
+__global__ void __launch_bounds__(256, 8) k_batch_track(BatchSeg S)
+{
+    track_chunks<MODE>(S);
 }
 
 // One chunk of a MEGNO job for the segment's turns: the fused tangent map and
@@ -361,6 +368,10 @@ __device__ __forceinline__ void megno_chunk(const BatchSeg &S, ConstPtr<JobDesc>
     }
 }
 
+// The MEGNO jobs' chunks, the longer ones, then the tracking jobs': in a segment of
+// few chunks both kinds are bound by their turns' latency and run side by side, and in
+// a full one the tracking chunks fill the end of the MEGNO's. 192 jobs, 30 % of them
+// with the MEGNO: two launches a segment 48.9 ms, one 40.6; 2 % of them 43.4, 32.1.
 template <int MODE>
 __global__ void __launch_bounds__(256) k_batch_megno(BatchSeg S)
 {
@@ -389,6 +400,7 @@ __global__ void __launch_bounds__(256) k_batch_megno(BatchSeg S)
         if (J->mu != 0.0) megno_chunk<MODE, true>(S, J, job, base, n, log_tab);
         else megno_chunk<MODE, false>(S, J, job, base, n, log_tab);
     }
+    track_chunks<MODE>(S);
 }
 
 static uint32_t batch_resident_waves()
@@ -568,12 +580,13 @@ void batch_run(const hm_job *jobs, size_t n_jobs, int mode, int block, int every
                 else
                     hipLaunchKernelGGL(k_batch_megno<kFast>, dim3(grid), dim3(block), 0, q, S);
                 launch_check("k_batch_megno");
+            } else {
+                if (mode == HM_MODE_EXACT)
+                    hipLaunchKernelGGL(k_batch_track<kExact>, dim3(grid), dim3(block), 0, q, S);
+                else
+                    hipLaunchKernelGGL(k_batch_track<kFast>, dim3(grid), dim3(block), 0, q, S);
+                launch_check("k_batch_track");
             }
-            if (mode == HM_MODE_EXACT)
-                hipLaunchKernelGGL(k_batch_track<kExact>, dim3(grid), dim3(block), 0, q, S);
-            else
-                hipLaunchKernelGGL(k_batch_track<kFast>, dim3(grid), dim3(block), 0, q, S);
-            launch_check("k_batch_track");
         }
     };
     if (!graph) {
