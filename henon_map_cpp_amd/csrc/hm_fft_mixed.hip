@@ -540,8 +540,10 @@ __global__ void __launch_bounds__(kMrThreads) k_mr_tune(MrArgs a)
 // point and wavefront 3700), the maximum and the tune 7000. 10000 points as 10^4
 // instead of 5^4 x 2 x 8, twiddles read in order instead of strided through one
 // table (64 cache lines an instruction) and one square root a signal instead of
-// one an entry: 129 -> 86 ns per signal; 500 points (10 x 10 x 5, one wavefront)
-// 7.7 -> 3.1, 501 (chirp-z over 7 x 9 x 16 instead of 3 x 3 x 7 x 2 x 8) 16.3 -> 10.6.
+// one an entry: 129 -> 91 ns per signal; 500 points (10 x 10 x 5, one wavefront)
+// 7.7 -> 3.1, 501 (chirp-z over 7 x 9 x 16 instead of 3 x 3 x 7 x 2 x 8) 16.3 -> 11.
+// Samples by stepped pointers instead of an address formed of three products each:
+// 91 -> 84 ns, 500 points 3.1 -> 2.8.
 // The shapes of k_wh_tune: 64, 128 .. kWhThreads threads for up to ten points a
 // thread (a butterfly of the radix-10 passes each, every wavefront at work; 16
 // wavefronts and up to 160 KiB of signals per CU in every shape).
@@ -661,7 +663,8 @@ __device__ __forceinline__ void wh_fold_pairs(Cplx *buf, const WhPass &ps, const
 // terms for every output (bound by LDS) and computes its roots; here a term serves
 // 16 outputs and the matrix cores set the pace: of 101000 cycles at 10001 = 73 x 137
 // points the two products take 20000 and 36000, where the instructions alone would
-// (padding to 16 included) 16000 and 30000. 10001 points 331 -> 181 ns per signal.
+// (padding to 16 included) 16000 and 30000. 10001 points 331 -> 184 ns per signal
+// (171 with the load's pointers stepped).
 constexpr uint32_t kMatrixRounds = 2;
 using Quad = double __attribute__((ext_vector_type(4)));
 
@@ -886,16 +889,18 @@ __global__ void __launch_bounds__(NT, 4) k_wh_tune(WhArgs a)
     // that waits for each sample in turn leaves the workgroup idle)
     constexpr uint32_t LP = (CZ ? PMAX / 2 : PMAX + NT - 1) / NT + (CZ ? 1 : 0);
     double vx[LP], vp[LP], hh[LP];
+    const double *px = a.hist + hat(a.lay, (uint64_t)a.from + threadIdx.x, cx, particle);
+    const size_t to_p = a.lay.cs, ahead = (size_t)NT * a.lay.ms;
 #pragma unroll
     for (uint32_t u = 0; u < LP; ++u) {
         const uint32_t m = threadIdx.x + u * NT;
         vx[u] = vp[u] = hh[u] = 0.0;
         if (m < N) {
-            const uint64_t sm = (uint64_t)a.from + m;
-            vx[u] = a.hist[hat(a.lay, sm, cx, particle)];
-            vp[u] = a.hist[hat(a.lay, sm, cp, particle)];
+            vx[u] = px[0];
+            vp[u] = px[to_p];
             hh[u] = a.hann[m];
         }
+        px += ahead;
     }
     if (scan_other)
         for (uint32_t m = threadIdx.x; m < N; m += NT) {
