@@ -1,4 +1,5 @@
-// log10 for the per-turn MEGNO sums, by the method of fdlibm's e_log.c and
+// log10 in one straight block (the MEGNO sums take norms' logarithms from a table
+// instead, hm_lognorm.h; no kernel calls this one), by the method of fdlibm's e_log.c and
 // e_log10.c (Sun Microsystems, 1993; freely distributable): x = 2^k m with m in
 // [sqrt(2)/2, sqrt(2)), f = m - 1, s = f / (2 + f),
 //   ln m = 2 atanh(s) = f - s (f - R(s^2))            (or, for m near sqrt(2),
@@ -12,7 +13,7 @@
 // At most 2 units in the last place from the C library's log10, 88 % of
 // arguments correctly rounded (tests/log10_check.cpp). The library's
 // double-double log10 takes about 90 instructions on gfx950 and a branch, this
-// one about 50 in the same straight block of the indicator kernel's turn.
+// one about 50.
 // Compiles as host code too (no HIP types), so a host check can build it with
 // g++ alone; device and host differ only in the reciprocal's first estimate.
 #pragma once
