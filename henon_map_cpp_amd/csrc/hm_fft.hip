@@ -324,6 +324,22 @@ __global__ void k_birkhoff_hist(const double *__restrict__ hist, HistLayout h, u
     out[((size_t)w * 2 + p) * nn + i] = bad ? __builtin_nan("") : 1 - acc / (2 * M_PI);
 }
 
+// The neighbouring lower lane's value (`first` in lane 0), and lane 63's in every
+// lane: moves between lanes on the vector unit, where __shfl takes two trips through
+// the LDS unit per double. Every lane active.
+__device__ __forceinline__ double lane_before(double v, double first)
+{
+    constexpr int kWaveShiftRight = 0x138;  // DPP wave_shr:1
+    const int hi = __builtin_amdgcn_update_dpp(__double2hiint(first), __double2hiint(v), kWaveShiftRight, 0xf, 0xf, false);
+    const int lo = __builtin_amdgcn_update_dpp(__double2loint(first), __double2loint(v), kWaveShiftRight, 0xf, 0xf, false);
+    return __hiloint2double(hi, lo);
+}
+__device__ __forceinline__ double last_lane(double v)
+{
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), 63),
+                            __builtin_amdgcn_readlane(__double2loint(v), 63));
+}
+
 // Birkhoff tunes of particle rows: one wavefront per (particle, plane,
 // window); lane l takes samples m0 + l of each 64-sample step (coalesced along
 // the row), the angle of the sample before comes from the neighbouring lane
@@ -333,7 +349,8 @@ __global__ void k_birkhoff_hist(const double *__restrict__ hist, HistLayout h, u
 // sample order (within rounding of it).
 // Bound by the angles, two thirds of what the rows' reading would take at full rate:
 // by the table (hm_angle.h) instead of the library 20000 rows of 10001 samples 2.04 ->
-// 1.70 ms (6.4 GB), 40000 of 501 0.235 -> 0.199. The sums' error against long double
+// 1.70 ms (6.4 GB), 40000 of 501 0.235 -> 0.199; the neighbours' angles by lane moves
+// instead of four trips through LDS a sample 1.72 -> 1.57 and 0.200 -> 0.190. The sums' error against long double
 // is the same (rms 1.1e-15 at 2000 samples), that of adding them up.
 __global__ void __launch_bounds__(256) k_birkhoff_rows(const double *__restrict__ rows, uint64_t L, uint32_t n,
                                                        uint32_t p0, uint32_t nb, const double *__restrict__ means,
@@ -394,9 +411,8 @@ __global__ void __launch_bounds__(256) k_birkhoff_rows(const double *__restrict_
                 bad |= any_nan(a0[u] - mx, a1[u] - mp, 0.0, 0.0);
                 th = angle_of(a1[u] - mp, a0[u] - mx, angle_tab);
             }
-            double prev = __shfl_up(th, 1);
-            if (lane == 0) prev = carry;
-            carry = __shfl(th, 63);
+            const double prev = lane_before(th, carry);
+            carry = last_lane(th);
             if (valid && m > 0) {
                 double d = th - prev;
                 if (d < 0.0) d += 2.0 * M_PI;
