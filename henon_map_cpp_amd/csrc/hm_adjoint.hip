@@ -257,7 +257,7 @@ struct AdjAcc {
 
 template <bool OCT>
 __device__ __forceinline__ void adjoint_turn(const double (&pre)[4], const double (&post)[4], const TabEntry &t,
-                                             double bw, const double4 &dt, double mu3, AdjAcc &a)
+                                             double bw, const double4 &dt, double mu3, double mu6, AdjAcc &a)
 {
     // Birkhoff seed of sample k+1: d/dx_{k+1} of c w_k x_{k+1}^2 (bw = 2 c w_k)
     a.lx = fma(bw, post[0], a.lx);
@@ -268,25 +268,15 @@ __device__ __forceinline__ void adjoint_turn(const double (&pre)[4], const doubl
     a.g_wy = fma(dwy, dt.z, a.g_wy);
     a.g_eps = fma(dwx, dt.y, fma(dwy, dt.w, a.g_eps));
     // through the rotations
-    double lxt = fma(t.cx, a.lx, -t.sx * a.lpx), lyt = fma(t.cy, a.ly, -t.sy * a.lpy);
-    const double lpt = fma(t.sx, a.lx, t.cx * a.lpx), lqt = fma(t.sy, a.ly, t.cy * a.lpy);
-    // Through the kicks, at the pre-step point: with z = x + i y they are z^2 + mu z^3,
-    // the real part on p_x, minus the imaginary part on p_y, so with l = l_px + i l_py
-    // the adjoint takes 2 z l + 3 mu z^2 l and the derivative by mu is Re z^3 l. The
-    // three products z l, z^2 l, z^3 l share their factors: 14 operations for the 18
-    // of the partial derivatives one by one.
-    const double x = pre[0], y = pre[2];
-    const double ar = fma(x, lpt, -(y * lqt)), ai = fma(y, lpt, x * lqt);
-    lxt = fma(2.0, ar, lxt);
-    lyt = fma(-2.0, ai, lyt);
-    if (OCT) {
-        const double br = fma(x, ar, -(y * ai)), bi = fma(x, ai, y * ar);
-        a.g_mu = fma(x, br, fma(-y, bi, a.g_mu));
-        lxt = fma(mu3, br, lxt);
-        lyt = fma(-mu3, bi, lyt);
-    }
-    a.lx = lxt;
-    a.ly = lyt;
+    const double lxt = fma(t.cx, a.lx, -t.sx * a.lpx), lpt = fma(t.sx, a.lx, t.cx * a.lpx);
+    const double lyt = fma(t.cy, a.ly, -t.sy * a.lpy), lqt = fma(t.sy, a.ly, t.cy * a.lpy);
+    // through the kicks, at the pre-step point
+    const double x = pre[0], y = pre[2], xx = x * x, yy = y * y;
+    if (OCT) a.g_mu = fma(lpt, x * fma(-3.0, yy, xx), fma(lqt, y * fma(-3.0, xx, yy), a.g_mu));
+    const double ja = fma(mu3, xx - yy, 2.0 * x);
+    const double jb = fma(-mu6 * x, y, -2.0 * y);
+    a.lx = fma(ja, lpt, fma(jb, lqt, lxt));
+    a.ly = fma(jb, lpt, fma(-ja, lqt, lyt));
     a.lpx = lpt;
     a.lpy = lqt;
 }
@@ -405,7 +395,7 @@ __global__ void __launch_bounds__(256) k_adjoint_sweep(AdjointSweepArgs a)
                      a.grad_p[i],  a.grad_p[n + i],  a.grad_p[2 * n + i],  a.grad_p[3 * n + i]};
     }
     const double bseed = 2.0 * (a.seed_b ? a.seed_b[i] : 0.0);
-    const double mu = a.mu, m3mu = -3.0 * mu, mu3 = 3.0 * mu;
+    const double mu = a.mu, m3mu = -3.0 * mu, mu3 = 3.0 * mu, mu6 = 6.0 * mu;
     const uint32_t T = a.n_turns, K = a.every;
     const uint32_t n_seg = (T + K - 1) / K;
     const ConstPtr<TabEntry> tab = as_const(a.tab);
@@ -416,7 +406,7 @@ __global__ void __launch_bounds__(256) k_adjoint_sweep(AdjointSweepArgs a)
     auto adjoint_at = [&](uint32_t k, const double (&pre)[4], const double (&post)[4]) {
         const ConstPtr<double> d = dtab + 4 * (size_t)k;
         const double4 dt{d[0], d[1], d[2], d[3]};
-        adjoint_turn<OCT>(pre, post, load_record(tab + k), bseed * weights[k], dt, mu3, acc);
+        adjoint_turn<OCT>(pre, post, load_record(tab + k), bseed * weights[k], dt, mu3, mu6, acc);
     };
     auto fill = [&](double (&S)[kChunk][4], uint32_t c0, uint32_t len) {
 #pragma unroll
@@ -525,7 +515,7 @@ __global__ void __launch_bounds__(kFusedBlock) k_adjoint_sweep_fused(AdjointSwee
         for (int c = 0; c < 4; c++) { a.grad_x0[c * n + i] = 0.0; a.grad_p[c * n + i] = 0.0; }
     if (!__any(live)) return;  // the whole wavefront
 
-    const double mu = a.mu, m3mu = -3.0 * mu, mu3 = 3.0 * mu;
+    const double mu = a.mu, m3mu = -3.0 * mu, mu3 = 3.0 * mu, mu6 = 6.0 * mu;
     const uint32_t T = a.n_turns, K = a.every;
     const uint32_t n_seg = (T + K - 1) / K;
     const uint32_t K8 = K / kChunk;
@@ -648,10 +638,10 @@ __global__ void __launch_bounds__(kFusedBlock) k_adjoint_sweep_fused(AdjointSwee
             const ConstPtr<double> d = dtab + 4 * (size_t)k;
             const double4 dt{d[0], d[1], d[2], d[3]};
             if ((uint32_t)m + 1 == lent)
-                adjoint_turn<OCT>(S[m], nxt, load_record(tab + k), bseed * weights[k], dt, mu3, acc);
+                adjoint_turn<OCT>(S[m], nxt, load_record(tab + k), bseed * weights[k], dt, mu3, mu6, acc);
             else
                 adjoint_turn<OCT>(S[m], S[m + 1 < kChunk ? m + 1 : m], load_record(tab + k), bseed * weights[k], dt,
-                                  mu3, acc);
+                                  mu3, mu6, acc);
         }
         copy4(nxt, S[0]);
     }
@@ -678,7 +668,7 @@ __global__ void __launch_bounds__(kFusedBlock) k_adjoint_sweep_fused(AdjointSwee
             TabEntry rpn{};
             if (m > 0) rcn = rec_c(g, m - 1);
             if (j + 2 < kChunk) rpn = rec_p(gp, j + 1);
-            adjoint_turn<OCT>(X[m], post, rc.t, bseed * rc.w, rc.dt, mu3, acc);
+            adjoint_turn<OCT>(X[m], post, rc.t, bseed * rc.w, rc.dt, mu3, mu6, acc);
             copy4(post, X[m]);
             if (j + 1 < kChunk) {
                 copy4(Y[j + 1], Y[j]);
@@ -737,7 +727,7 @@ __global__ void __launch_bounds__(256) k_adjoint_sweep_split(AdjointSweepArgs a)
         for (int c = 0; c < 4; c++) { a.grad_x0[c * n + i] = 0.0; a.grad_p[c * n + i] = 0.0; }
     if (!__syncthreads_or(live)) return;  // the whole workgroup
 
-    const double mu = a.mu, m3mu = -3.0 * mu, mu3 = 3.0 * mu;
+    const double mu = a.mu, m3mu = -3.0 * mu, mu3 = 3.0 * mu, mu6 = 6.0 * mu;
     const uint32_t T = a.n_turns, K = a.every;
     const uint32_t n_seg = (T + K - 1) / K;
     const uint32_t K8 = K / kChunk;
@@ -832,7 +822,7 @@ __global__ void __launch_bounds__(256) k_adjoint_sweep_split(AdjointSweepArgs a)
         for (int m = kChunk - 1; m >= 0; --m) {
             if ((uint32_t)m >= lent) continue;
             const AdjRec r = record(ct + m);
-            adjoint_turn<OCT>(S[m], nxt, r.t, bseed * r.w, r.dt, mu3, acc);
+            adjoint_turn<OCT>(S[m], nxt, r.t, bseed * r.w, r.dt, mu3, mu6, acc);
             copy4(nxt, S[m]);
         }
     }
@@ -856,8 +846,8 @@ __global__ void __launch_bounds__(256) k_adjoint_sweep_split(AdjointSweepArgs a)
     auto back = [&](const Two &t) {
         const double post1[4] = {t.s[2].x, t.s[2].y, t.s[3].x, t.s[3].y};
         const double post0[4] = {t.s[0].x, t.s[0].y, t.s[1].x, t.s[1].y};
-        adjoint_turn<OCT>(post1, nxt, t.r1.t, bseed * t.r1.w, t.r1.dt, mu3, acc);
-        adjoint_turn<OCT>(post0, post1, t.r0.t, bseed * t.r0.w, t.r0.dt, mu3, acc);
+        adjoint_turn<OCT>(post1, nxt, t.r1.t, bseed * t.r1.w, t.r1.dt, mu3, mu6, acc);
+        adjoint_turn<OCT>(post0, post1, t.r0.t, bseed * t.r0.w, t.r0.dt, mu3, mu6, acc);
         copy4(nxt, post0);
     };
     auto arrived = [] {
