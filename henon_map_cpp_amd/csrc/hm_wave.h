@@ -90,11 +90,13 @@ inline int octupole_kind(int mode, double mu)
 // inside for one turn of the map or of its inverse: the kick moves (px, py) by at
 // most rho^2 + |mu| rho^3, rho = |(x, y)| <= r, and the rotations keep r, so a turn
 // takes r to at most r + r^2 + |mu| r^3; R takes that to b, less a margin far above
-// the roundings. 0 (never inside) where no such radius exists.
+// the roundings. 0 (never inside) where no such radius exists: a barrier or a mu that
+// is NaN (no point is inside the one, the other has no bound), a mu beyond 1e100.
 inline double safe_radius2(double barrier, double mu)
 {
-    const double m = std::fabs(mu), b = std::fmin(std::fabs(barrier), 1e100);
-    if (!(b > 0.0) || !(m < 1e100)) return 0.0;
+    const double m = std::fabs(mu);
+    if (!(std::fabs(barrier) > 0.0) || !(m < 1e100)) return 0.0;
+    const double b = std::fmin(std::fabs(barrier), 1e100);
     double lo = 0.0, hi = b;
     for (int i = 0; i < 1100; ++i) {
         const double r = 0.5 * (lo + hi);
