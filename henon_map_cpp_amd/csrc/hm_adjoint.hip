@@ -159,46 +159,50 @@ __global__ void __launch_bounds__(kFwdBlock) k_adjoint_forward(AdjointFwdArgs a)
             const uint32_t last = pairs_end - 2;
             TabEntry a0 = load_record(tab), a1 = load_record(tab + 1), b0, b1;
             double wa0 = weights[0], wa1 = weights[1], wb0, wb1;
-            uint32_t touched = 0, touched_w = 0;
-            auto touch = [&](uint32_t from) {
-                const uint32_t kk = umin(from + lane, T - 1);
-                asm volatile("" ::"v"(touched), "v"(touched_w));
-                touched = *reinterpret_cast<const uint32_t *>(a.tab + kk);
-                touched_w = *reinterpret_cast<const uint32_t *>(a.weights + kk);
-            };
-            touch(0);
-            for (; k < pairs_end; k += 8) {
-                if (to_ck == 0) {
-                    checkpoint(ck);
-                    ck += 4 * n;
-                    to_ck = K;
-                }
-                to_ck -= 8;
-                if (k % 64 == 0) touch(k + 64);
+            // records and weights from 64 turns ahead on, as in the tracking kernel
+            auto ahead = [&](uint32_t from) { return a.tab[umin(from + lane, T - 1)]; };
+            uint32_t touched = 0;
+            bool rotating = !__any(!rotates(ahead(0)));
+            while (rotating && k != pairs_end) {
+                const TabEntry later = ahead(k + 64);
+                asm volatile("" ::"v"(touched));
+                touched = *reinterpret_cast<const uint32_t *>(a.weights + umin(k + 64 + lane, T - 1));
+                const uint32_t end = k + umin(pairs_end - k, 64);
+                do {
+                    if (to_ck == 0) {
+                        checkpoint(ck);
+                        ck += 4 * n;
+                        to_ck = K;
+                    }
+                    to_ck -= 8;
+                    const ConstPtr<TabEntry> p = tab + k;
+                    const ConstPtr<double> w = weights + k;
 #pragma unroll
-                for (uint32_t q = 0; q < 8; q += 4) {
-                    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): this pair's entries
-                    __builtin_amdgcn_sched_barrier(0);
-                    b0 = load_record(tab + (k + q + 2));
-                    b1 = load_record(tab + (k + q + 3));
-                    wb0 = weights[k + q + 2];
-                    wb1 = weights[k + q + 3];
-                    __builtin_amdgcn_sched_barrier(0);
-                    pair(a0, a1, wa0, wa1);
-                    const uint32_t nx = umin(k + q + 4, last);
-                    __builtin_amdgcn_s_waitcnt(0xC07F);
-                    __builtin_amdgcn_sched_barrier(0);
-                    a0 = load_record(tab + nx);
-                    a1 = load_record(tab + nx + 1);
-                    wa0 = weights[nx];
-                    wa1 = weights[nx + 1];
-                    __builtin_amdgcn_sched_barrier(0);
-                    pair(b0, b1, wb0, wb1);
-                }
+                    for (uint32_t q = 0; q < 8; q += 4) {
+                        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): this pair's entries
+                        __builtin_amdgcn_sched_barrier(0);
+                        b0 = load_record(p + q + 2);
+                        b1 = load_record(p + q + 3);
+                        wb0 = w[q + 2];
+                        wb1 = w[q + 3];
+                        __builtin_amdgcn_sched_barrier(0);
+                        pair(a0, a1, wa0, wa1);
+                        const uint32_t nx = umin(k + q + 4, last);
+                        __builtin_amdgcn_s_waitcnt(0xC07F);
+                        __builtin_amdgcn_sched_barrier(0);
+                        a0 = load_record(tab + nx);
+                        a1 = load_record(tab + nx + 1);
+                        wa0 = weights[nx];
+                        wa1 = weights[nx + 1];
+                        __builtin_amdgcn_sched_barrier(0);
+                        pair(b0, b1, wb0, wb1);
+                    }
+                    k += 8;
+                } while (k != end);
+                rotating = !__any(!rotates(later));
             }
-            radius();  // the last turn may have gone untested
-            park();
         }
+        // what is left, all of it from a window of records on that do not all rotate
         for (; k < T; ++k) {
             if (to_ck == 0) {
                 checkpoint(ck);

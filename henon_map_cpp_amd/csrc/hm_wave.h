@@ -21,6 +21,16 @@ __device__ __forceinline__ uint64_t not_below(double v, double s)
     return __builtin_amdgcn_fcmp(v, s, kUnorderedOrGE);
 }
 
+// Whether both pairs of a record are the sine and cosine of one angle, to 2^-40 (a
+// table of hm_build_table keeps to about 2^-52; records that are not finite do not).
+// Turns that do not rotate may take a point out from anywhere, or bring it down to
+// where products leave the normal range.
+__device__ __forceinline__ bool rotates(const TabEntry &t)
+{
+    return fabs(fma(t.sx, t.sx, fma(t.cx, t.cx, -1.0))) < 0x1p-40 &&
+           fabs(fma(t.sy, t.sy, fma(t.cy, t.cy, -1.0))) < 0x1p-40;
+}
+
 // Per-lane fallback used when the live lanes of a wavefront do not share one
 // turn index (particles reset while others were not) or when that index range
 // leaves the table: each lane reads its own table record, and a lane whose
@@ -176,27 +186,20 @@ __device__ __forceinline__ void track_wave(const TrackArgs &A, uint32_t base, ui
             if (lost & my_bit) done = kk;
             live &= ~lost;
         };
-        auto checked = [&](const TabEntry &t, uint32_t kk) {
-            turn(t);
-            radius();
-            if (live & not_below(r2, b2s)) settle(kk);
-        };
         // The fused forms need every coordinate zero or at least kTinyCoord.
         bool plain = true;
         if (EXACT) {
             auto small = [](double v) { return v != 0.0 && fabs(v) < kTinyCoord; };
             plain = !__any(alive0 && (small(x) || small(px) || small(y) || small(py)));
         }
-        if (plain) {
+        uint32_t k = 0;
+        if (plain && n_turns >= kBlock) {
             // Turns go in pairs with one test: a point below safe1 after the first
-            // turn is inside the barrier after the second, whatever it is. (A record
-            // that is not finite takes every point out at once; if it was the
-            // untested turn's, the loss is that turn's.)
-            // A turn is then 30 to 32 operations and half a test (4 operations and a
-            // branch), where every turn had one: 1e6 particles on the 1000 x 1000
-            // grid, 3e4 turns, mu = 0.5: 22.0 -> 19.3 ms (exact), 15.9 -> 14.5 ms
-            // (fast).
-            uint32_t k = 0;
+            // turn is inside the barrier after the second, whatever it is, as far as
+            // the records rotate. A turn is then 30 to 32 operations and half a test
+            // (4 operations and a branch), where every turn had one: 1e6 particles on
+            // the 1000 x 1000 grid, 3e4 turns, mu = 0.5: 22.0 -> 19.3 ms (exact), 15.9
+            // -> 14.5 ms (fast).
             const double safe1 = A.safe1;
             auto pair = [&](const TabEntry &t0, const TabEntry &t1, uint32_t kk) {
                 turn(t0);
@@ -204,72 +207,68 @@ __device__ __forceinline__ void track_wave(const TrackArgs &A, uint32_t base, ui
                 if (__builtin_expect((live & not_below(r2, safe1)) == 0, 1)) {
                     turn(t1);
                 } else {
-                    if (live & not_below(r2, b2s)) {
-                        // (read for a loss alone: a chaotic orbit can stay beyond
-                        // safe1 for thousands of turns)
-                        if (kk) {
-                            const TabEntry t = rec(kk - 1);
-                            const double z = 0.0 * ((t.sx + t.cx) + (t.sy + t.cy));
-                            settle(z == 0.0 ? kk : kk - 1);
-                        } else {
-                            settle(kk);
-                        }
-                    }
-                    checked(t1, kk + 1);
+                    if (live & not_below(r2, b2s)) settle(kk);
+                    turn(t1);
+                    radius();
+                    if (live & not_below(r2, b2s)) settle(kk + 1);
                 }
             };
-            if (n_turns >= kBlock) {
-                // Two pairs of records: while one pair's turns run, the other is
-                // requested (one 64-byte scalar load), into the registers the pair
-                // before last used.
-                const uint32_t last = n_turns - 2;
-                TabEntry a0 = rec(0), a1 = rec(1), b0, b1;
-                // Each lane touches a record 64 to 128 turns ahead, every 64 turns, so
-                // that scalar loads find the table in L2 also the first time it is
-                // read (64 particles, 1e4 turns: 0.89 ms warm or cold; without the
-                // touches 1.92 ms cold).
-                uint32_t touched = 0;
-                auto touch = [&](uint32_t from) {
-                    const uint32_t kk = min(from + lane, n_turns - 1);
-                    touched = *reinterpret_cast<const uint32_t *>(INV ? tab + (s0 - 1 - kk) : tab + (s0 + kk));
-                };
-                touch(0);
-                for (; k + kBlock <= n_turns && live; k += kBlock) {
-                    if (k % 64 == 0) {
-                        asm volatile("" ::"v"(touched));
-                        touch(k + 64);
-                    }
+            // Two pairs of records: while one pair's turns run, the other is
+            // requested (one 64-byte scalar load), into the registers the pair
+            // before last used.
+            const uint32_t last = n_turns - 2;
+            TabEntry a0 = rec(0), a1 = rec(1), b0, b1;
+            // At every 64th turn each lane takes one of the 64 records from 64 turns
+            // ahead on: to see that all rotate before the turns get there, and so that
+            // the scalar loads find the table in L2 also the first time it is read (64
+            // particles, 1e4 turns: 0.89 ms warm or cold; without 1.92 ms cold).
+            auto ahead = [&](uint32_t from) {
+                const uint32_t kk = min(from + lane, n_turns - 1);
+                return INV ? tab[s0 - 1 - kk] : tab[s0 + kk];
+            };
+            uint32_t blocks = n_turns / kBlock;
+            bool rotating = !__any(!rotates(ahead(0)));
+            while (rotating && blocks && live) {
+                const TabEntry later = ahead(k + 64);
+                uint32_t m = min(blocks, 64 / kBlock);
+                blocks -= m;
+                do {
+                    const ConstPtr<TabEntry> p = INV ? tp - k : tp + k;
 #pragma unroll
                     for (uint32_t q = 0; q < kBlock; q += 4) {
                         __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): a0, a1 are there
                         __builtin_amdgcn_sched_barrier(0);
-                        b0 = rec(k + q + 2);
-                        b1 = rec(k + q + 3);
+                        b0 = load_record(INV ? p - (q + 2) : p + (q + 2));
+                        b1 = load_record(INV ? p - (q + 3) : p + (q + 3));
+                        // (keeps the loads ahead of the first turn)
+                        asm volatile("" ::: "memory");
                         __builtin_amdgcn_sched_barrier(0);
                         pair(a0, a1, k + q);
                         const uint32_t nx = min(k + q + 4, last);
                         __builtin_amdgcn_s_waitcnt(0xC07F);
                         __builtin_amdgcn_sched_barrier(0);
-                        a0 = rec(nx);
-                        a1 = rec(nx + 1);
+                        const ConstPtr<TabEntry> pn = INV ? tp - nx : tp + nx;
+                        a0 = load_record(pn);
+                        a1 = load_record(INV ? pn - 1 : pn + 1);
                         __builtin_amdgcn_sched_barrier(0);
                         pair(b0, b1, k + q + 2);
                     }
-                }
-                radius();  // the last turn may have gone untested
-                if (live & not_below(r2, b2s)) settle(k - 1);
+                    k += kBlock;
+                    m = __builtin_amdgcn_readfirstlane(m - 1);  // (kept in a scalar register)
+                } while (m && live);
+                rotating = !__any(!rotates(later));
             }
-            for (; live && k < n_turns; ++k) checked(rec(k), k);
-        } else {
-            // The reference's operations one by one and a test every turn.
-            TabEntry next = rec(0);
-            for (uint32_t k = 0; k < n_turns && live; ++k) {
-                const TabEntry t = next;
-                next = rec(min(k + 1, n_turns - 1));
-                map_step<MODE, INV, OCT != 0>(x, px, y, py, mu, m3mu, t);
-                r2 = screen_radius2(x, px, y, py);
-                if (live & not_below(r2, b2s)) settle(k);
-            }
+        }
+        // What is left (fewer than kBlock turns, all of them for tiny coordinates, all
+        // from a window of records on that do not all rotate): the map's own
+        // operations and a test every turn.
+        TabEntry next = rec(min(k, n_turns - 1));
+        for (; k < n_turns && live; ++k) {
+            const TabEntry t = next;
+            next = rec(min(k + 1, n_turns - 1));
+            map_step<MODE, INV, OCT != 0>(x, px, y, py, mu, m3mu, t);
+            r2 = EXACT ? screen_radius2(x, px, y, py) : radius2<MODE>(x, px, y, py);
+            if (live & not_below(r2, b2s)) settle(k);
         }
         if (alive0 && !(live & my_bit)) x = px = y = py = __builtin_nan("");
     } else if (n_turns > 0) {

@@ -14,10 +14,7 @@
  * Layouts in HBM
  *   particles : structure of arrays, x, px, y, py (double[n]) and steps (uint32[n])
  *   table     : one 32-byte record per turn, {sin wx(n), cos wx(n), sin wy(n), cos wy(n)}
- *               (double[turns][4]); built on the host by hm_build_table. The kernels
- *               count on each pair being the sine and cosine of one angle (or not
- *               finite): a point well inside the barrier is not tested for loss
- *               after a turn that cannot take it out
+ *               (double[turns][4]); built on the host by hm_build_table
  *   matrices  : double[n][16], row-major 4x4 per particle (the reference's layout)
  *
  * Each declaration names the reference interface it replaces (paths relative to
