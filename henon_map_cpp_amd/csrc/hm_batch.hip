@@ -698,7 +698,7 @@ extern "C" int hm_autotune_batch(const hm_job *jobs, size_t n_jobs, int mode, ui
                 t.n_turns = std::min(jobs[k].n_turns, trial_turns);
                 if (!n) continue;
                 void *b = nullptr;
-                hip_check(hipMalloc(&b, n * (4 * sizeof(double) + sizeof(uint32_t)) + (jobs[k].megno ? 8 * n + 8 : 0)),
+                hip_check(device_malloc(&b, n * (4 * sizeof(double) + sizeof(uint32_t)) + (jobs[k].megno ? 8 * n + 8 : 0)),
                           "hipMalloc(autotune_batch)");
                 bufs.push_back(b);
                 double *d = static_cast<double *>(b);

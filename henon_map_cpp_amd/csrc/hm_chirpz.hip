@@ -373,11 +373,11 @@ static CzPlan cz_plan(uint32_t N, hipStream_t s)
     std::vector<Cplx> twm(M);
     for (size_t k1 = 0; k1 < M1; ++k1)
         for (size_t n2 = 0; n2 < M2; ++n2) twm[k1 * M2 + n2] = tw[(k1 * n2) & (M - 1)];
-    hip_check(hipMalloc(&p.twm, M * sizeof(Cplx)), "hipMalloc(chirp-z step twiddles)");
+    hip_check(device_malloc(&p.twm, M * sizeof(Cplx)), "hipMalloc(chirp-z step twiddles)");
     hip_check(hipMemcpyAsync(p.twm, twm.data(), M * sizeof(Cplx), hipMemcpyHostToDevice, s), "hipMemcpyAsync");
-    hip_check(hipMalloc(&p.tw, M * sizeof(Cplx)), "hipMalloc(chirp-z twiddles)");
-    hip_check(hipMalloc(&p.bhat, M * sizeof(Cplx)), "hipMalloc(chirp-z filter)");
-    hip_check(hipMalloc(&p.chirp, N * sizeof(Cplx)), "hipMalloc(chirp)");
+    hip_check(device_malloc(&p.tw, M * sizeof(Cplx)), "hipMalloc(chirp-z twiddles)");
+    hip_check(device_malloc(&p.bhat, M * sizeof(Cplx)), "hipMalloc(chirp-z filter)");
+    hip_check(device_malloc(&p.chirp, N * sizeof(Cplx)), "hipMalloc(chirp)");
     hip_check(hipMemcpyAsync(p.tw, tw.data(), M * sizeof(Cplx), hipMemcpyHostToDevice, s), "hipMemcpyAsync");
     hip_check(hipMemcpyAsync(p.bhat, bhat.data(), M * sizeof(Cplx), hipMemcpyHostToDevice, s), "hipMemcpyAsync");
     hip_check(hipMemcpyAsync(p.chirp, chirp.data(), N * sizeof(Cplx), hipMemcpyHostToDevice, s), "hipMemcpyAsync");

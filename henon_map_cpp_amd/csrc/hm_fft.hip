@@ -937,17 +937,17 @@ static FftTables fft_tables(uint32_t N, hipStream_t s)
         tw[2 * q + 1] = (double)-sinl(ang);
     }
     FftTables t;
-    hip_check(hipMalloc(&t.hann, N * sizeof(double)), "hipMalloc(hann)");
+    hip_check(device_malloc(&t.hann, N * sizeof(double)), "hipMalloc(hann)");
     hip_check(hipMemcpyAsync(t.hann, h.data(), N * sizeof(double), hipMemcpyHostToDevice, s), "hipMemcpyAsync");
     if (pow2) {
-        hip_check(hipMalloc(&t.tw, 2 * (size_t)N * sizeof(double)), "hipMalloc(twiddles)");
+        hip_check(device_malloc(&t.tw, 2 * (size_t)N * sizeof(double)), "hipMalloc(twiddles)");
         hip_check(hipMemcpyAsync(t.tw, tw.data(), 2 * (size_t)N * sizeof(double), hipMemcpyHostToDevice, s),
                   "hipMemcpyAsync");
     }
     if (pow2 && N >= 8 && N <= 2048) {
         std::vector<double> bw(N - 1);
         host_birkhoff_weights(N - 1, bw.data());
-        hip_check(hipMalloc(&t.bw, (N - 1) * sizeof(double)), "hipMalloc(Birkhoff weights)");
+        hip_check(device_malloc(&t.bw, (N - 1) * sizeof(double)), "hipMalloc(Birkhoff weights)");
         hip_check(hipMemcpyAsync(t.bw, bw.data(), (N - 1) * sizeof(double), hipMemcpyHostToDevice, s),
                   "hipMemcpyAsync");
     }

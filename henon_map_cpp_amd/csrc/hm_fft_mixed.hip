@@ -1037,7 +1037,7 @@ template <class T>
 static T *upload(const std::vector<T> &v, hipStream_t s, const char *what)
 {
     T *d = nullptr;
-    hip_check(hipMalloc(&d, v.size() * sizeof(T)), what);
+    hip_check(device_malloc(&d, v.size() * sizeof(T)), what);
     hip_check(hipMemcpyAsync(d, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice, s), "hipMemcpyAsync");
     return d;
 }

@@ -78,6 +78,17 @@ uint32_t *status_word();
 void *workspace(size_t bytes, int slot);
 // SIMDs of the current device (CUs x 4), cached per device.
 uint32_t device_simds();
+// hipMalloc, every device allocation of the library: tried again without the idle
+// blocks below if the device has no room for it.
+hipError_t device_malloc(void **p, size_t bytes);
+template <class T>
+hipError_t device_malloc(T **p, size_t bytes)
+{
+    void *v = nullptr;
+    const hipError_t e = device_malloc(&v, bytes);
+    *p = static_cast<T *>(v);
+    return e;
+}
 // Device blocks kept between owners (hm_buffer_take, hm_buffer_give).
 void *buffer_take(size_t bytes);
 void buffer_give(void *p);

@@ -120,36 +120,15 @@ uint32_t device_simds()
     return simds[dev] = (uint32_t)cus * 4u;
 }
 
-void *workspace(size_t bytes, int slot)
-{
-    if (slot < 0 || slot >= kWorkspaceSlots) throw Error(HM_ERR_ARG, "workspace slot out of range");
-    int dev = 0;
-    hip_check(hipGetDevice(&dev), "hipGetDevice");
-    std::lock_guard<std::mutex> lk(g_ws_mu);
-    auto &d = g_scratch[dev];
-    if (d.sizes[slot] < bytes) {
-        if (d.slots[slot]) {
-            hip_check(hipDeviceSynchronize(), "hipDeviceSynchronize");
-            hip_check(hipFree(d.slots[slot]), "hipFree(workspace)");
-            d.slots[slot] = nullptr;
-            d.sizes[slot] = 0;
-        }
-        size_t sz = bytes < 4096 ? 4096 : bytes;
-        hip_check(hipMalloc(&d.slots[slot], sz), "hipMalloc(workspace)");
-        d.sizes[slot] = sz;
-    }
-    return d.slots[slot];
-}
-
 // ---------------------------------------------------------------- buffers
 // hipMalloc and hipFree of a call's buffers took longer than its kernels: 24 ms a
 // GiB (tunes of 90000 particles x 1e4 turns: 28.8 GB of rows, 700 ms beside 105 ms
 // of work), 5 of 7.5 ms for 3001 particles x 2090 turns, half of a 64-particle call.
 // Given blocks therefore wait for the next taker: at most kIdleBytes a device, none
-// larger, all freed with the last taken one and whenever an allocation fails. A
-// block is given to one taker at a time, under a lock, and only used in the order
-// of the null stream, which all host threads share: a new owner's work runs after
-// the old one's.
+// larger, all freed with the last taken one and when the library finds no room for
+// an allocation (device_malloc). A block is given to one taker at a time, under a
+// lock, and only used in the order of the null stream, which all host threads share:
+// a new owner's work runs after the old one's.
 namespace {
 constexpr size_t kIdleBytes = 16ull << 30;
 struct Buffers {
@@ -177,6 +156,22 @@ Buffers &buffers()
 }
 }  // namespace
 
+hipError_t device_malloc(void **p, size_t bytes)
+{
+    const hipError_t e = hipMalloc(p, bytes);
+    if (e != hipErrorOutOfMemory) return e;
+    (void)hipGetLastError();
+    int dev = 0;
+    hip_check(hipGetDevice(&dev), "hipGetDevice");
+    {
+        Buffers &b = buffers();
+        std::lock_guard<std::mutex> lk(b.mu);
+        if (b.idle[dev].empty()) return e;
+        b.free_idle(dev);
+    }
+    return hipMalloc(p, bytes);
+}
+
 void *buffer_take(size_t bytes)
 {
     int dev = 0;
@@ -185,28 +180,26 @@ void *buffer_take(size_t bytes)
     if (bytes > SIZE_MAX - unit) throw Error(HM_ERR_ALLOC, "hipMalloc: out of memory");
     const size_t size = std::max<size_t>(1, (bytes + unit - 1) / unit) * unit;
     Buffers &b = buffers();
-    std::lock_guard<std::mutex> lk(b.mu);
-    auto &idle = b.idle[dev];
-    const auto it = idle.lower_bound(size);
-    if (it != idle.end() && it->first - size <= size / 4) {
-        void *p = it->second;
-        const size_t have = it->first;
-        b.taken[p] = {dev, have};
-        b.idle_bytes[dev] -= have;
-        idle.erase(it);
-        return p;
+    {
+        std::lock_guard<std::mutex> lk(b.mu);
+        auto &idle = b.idle[dev];
+        const auto it = idle.lower_bound(size);
+        if (it != idle.end() && it->first - size <= size / 4) {
+            void *p = it->second;
+            const size_t have = it->first;
+            b.taken[p] = {dev, have};
+            b.idle_bytes[dev] -= have;
+            idle.erase(it);
+            return p;
+        }
     }
     void *p = nullptr;
-    hipError_t e = hipMalloc(&p, size);
-    if (e != hipSuccess && !idle.empty()) {
-        (void)hipGetLastError();
-        b.free_idle(dev);
-        e = hipMalloc(&p, size);
-    }
+    const hipError_t e = device_malloc(&p, size);
     if (e != hipSuccess) {
         (void)hipGetLastError();
         throw Error(HM_ERR_ALLOC, std::string("hipMalloc: ") + hipGetErrorString(e));
     }
+    std::lock_guard<std::mutex> lk(b.mu);
     b.taken[p] = {dev, size};
     return p;
 }
@@ -228,6 +221,27 @@ void buffer_give(void *p)
     }
     b.idle[blk.dev].emplace(blk.size, p);
     b.idle_bytes[blk.dev] += blk.size;
+}
+
+void *workspace(size_t bytes, int slot)
+{
+    if (slot < 0 || slot >= kWorkspaceSlots) throw Error(HM_ERR_ARG, "workspace slot out of range");
+    int dev = 0;
+    hip_check(hipGetDevice(&dev), "hipGetDevice");
+    std::lock_guard<std::mutex> lk(g_ws_mu);
+    auto &d = g_scratch[dev];
+    if (d.sizes[slot] < bytes) {
+        if (d.slots[slot]) {
+            hip_check(hipDeviceSynchronize(), "hipDeviceSynchronize");
+            hip_check(hipFree(d.slots[slot]), "hipFree(workspace)");
+            d.slots[slot] = nullptr;
+            d.sizes[slot] = 0;
+        }
+        size_t sz = bytes < 4096 ? 4096 : bytes;
+        hip_check(device_malloc(&d.slots[slot], sz), "hipMalloc(workspace)");
+        d.sizes[slot] = sz;
+    }
+    return d.slots[slot];
 }
 
 // ---------------------------------------------------------------- modulation
@@ -303,7 +317,7 @@ int hm_malloc(void **ptr, size_t bytes)
         if (!ptr) throw Error(HM_ERR_ARG, "ptr is NULL");
         *ptr = nullptr;
         if (bytes == 0) return;
-        hipError_t e = hipMalloc(ptr, bytes);
+        hipError_t e = device_malloc(ptr, bytes);
         if (e != hipSuccess) throw Error(HM_ERR_ALLOC, std::string("hipMalloc: ") + hipGetErrorString(e));
     });
 }

@@ -67,7 +67,8 @@ int hm_free(void *ptr);
 /* Device memory of objects whose work is all on the null stream (the engine's
  * classes): at least `bytes` bytes, contents undefined. A given block may wait for
  * the next taker instead of going back to the device: at most 16 GiB of them per
- * device, freed when an allocation fails and when no block is taken any more. */
+ * device, freed when any call of the library finds no room for an allocation, and
+ * when no block is taken any more. */
 int hm_buffer_take(void **ptr, size_t bytes);
 int hm_buffer_give(void *ptr);
 /* kind: 0 host->device, 1 device->host, 2 device->device. Asynchronous on
