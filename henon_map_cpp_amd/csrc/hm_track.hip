@@ -40,7 +40,8 @@ struct TrackLaunch {
     uint32_t tab_len, n_turns;
     double mu, b2, safe1;
     uint32_t *idx_out, *count_out;
-    int block;  // 0: chosen per launch
+    int block;       // 0: chosen per launch
+    bool segmented;  // the caller or the autotuner set compact_every
 };
 
 static constexpr int kDefaultBlock = 256;
@@ -210,7 +211,8 @@ static bool prepare_track(double *x, double *px, double *y, double *py, uint32_t
     if (!cfg && tuned_config(mode, mu != 0.0, n, &tuned)) cfg = &tuned;
     const int block = cfg ? cfg->block : 0;
     if (block && (block < 64 || block > 256 || block % 64)) throw Error(HM_ERR_ARG, w + ": block must be 64, 128, 192 or 256");
-    every = cfg && cfg->compact_every ? cfg->compact_every : kDefaultCompactEvery;
+    const bool segmented = cfg && cfg->compact_every;
+    every = segmented ? cfg->compact_every : kDefaultCompactEvery;
     // particles_per_lane and table_staging are accepted for callers that set them:
     // there is one way now, a particle per lane and records by scalar loads
     const int per_lane = cfg ? cfg->particles_per_lane : 0;
@@ -223,6 +225,7 @@ static bool prepare_track(double *x, double *px, double *y, double *py, uint32_t
     a.b2 = barrier * barrier;  // henon.cu:2717, :3173
     a.safe1 = safe_radius2(barrier, mu);
     a.block = block;
+    a.segmented = segmented;
     const int staging = cfg ? cfg->table_staging : HM_STAGING_AUTO;
     if (staging < HM_STAGING_AUTO || staging > HM_STAGING_RING)
         throw Error(HM_ERR_ARG, w + ": table_staging must be 0 (auto), 1 (scalar) or 2 (ring)");
@@ -257,12 +260,11 @@ extern "C" int hm_track(double *x, double *px, double *y, double *py, uint32_t *
 
         // Up to one wavefront per SIMD, compaction frees nothing that another wavefront
         // waits for: all turns go in one launch (up to about 0.1 s of them) unless the
-        // caller chose. 1e4 particles x 1e4 turns, mu = 0.5, r < 0.4: 0.89 -> 0.81 ms;
+        // caller or the autotuner chose. 1e4 particles x 1e4 turns, mu = 0.5, r < 0.4: 0.89 -> 0.81 ms;
         // 32768 x 1e5: 9.4 -> 8.5; 65536 x 1e5, r < 0.7, two thirds lost: 9.5 -> 8.5
         // (r < 0.4, 2 % lost: 10.6 -> 10.9). With two wavefronts per SIMD it depends on
         // the losses (131072 x 1e4: 1.82 -> 1.61 ms with few, 0.99 -> 1.01 with most).
-        const bool chosen = cfg && cfg->compact_every;
-        const bool one_launch = !chosen && (N + 63u) / 64u <= device_simds() && n_turns <= (1u << 20);
+        const bool one_launch = !a.segmented && (N + 63u) / 64u <= device_simds() && n_turns <= (1u << 20);
         if (one_launch || every < 0 || (uint32_t)every >= n_turns) {
             a.n_arg = a.grid_bound = N;
             a.n_turns = n_turns;
@@ -454,8 +456,7 @@ extern "C" int hm_autotune_track(const double *x, const double *px, const double
         hm_launch_cfg best_c = base;
         try {
             for (int block : {64, 256})
-                for (int every : {500, 1000, 2000})
-                {
+                for (int every : {500, 1000, 2000}) {
                     hm_launch_cfg c{block, every, 1, 0};
                     hip_check(hipMemcpyAsync(work, warm, state, hipMemcpyDeviceToDevice, s), "hipMemcpyAsync");
                     hip_check(hipEventRecord(e0, s), "hipEventRecord");
@@ -470,7 +471,7 @@ extern "C" int hm_autotune_track(const double *x, const double *px, const double
                         best_t = ms;
                         best_c = c;
                     }
-                    }
+                }
         } catch (...) {
             (void)hipEventDestroy(e0);
             (void)hipEventDestroy(e1);
