@@ -1293,11 +1293,33 @@ static bool prefer_direct(const WhPlan &p, uint32_t gen)
     return filled && (gen <= kWhCzGen || all_matrix);
 }
 
+// The time of chirp-z over a plan's points, in about 5e-5 ns. A pass takes its
+// butterflies a wavefront of 64 at a time, whole or not, at 18 to 26 units a point by its
+// radix; a point takes 120 beside the passes (samples, filter, maximum), more in a small
+// length whose radices are all multiples of 4, which share banks; a thread takes 400 and
+// 60 a pass (start, barriers). Half as much again where one workgroup of 512 threads
+// leaves no room on the CU for a second. ns per signal: 1779 points over 4096 = 16^3 46.3,
+// over 3564 = 4 x 9 x 9 x 11 44.2, over 3584 = 7 x 8 x 8 x 8 40.3; 281 over 560 = 7 x 8 x 10
+// 4.9, over 567 = 7 x 9 x 9 (63 butterflies of radix 9) 4.3; 2520 over 5120 87, over 5040 58.
+static uint64_t chirp_cost(const WhPlan &p, bool alone)
+{
+    static constexpr uint32_t per_point[17] = {0, 0, 26, 26, 24, 20, 18, 20, 19, 20, 19, 24, 18, 26, 0, 0, 22};
+    uint64_t c = (400ull + 60 * p.n_pass) * wh_threads(p.L) + 120ull * p.L;
+    uint32_t shared = 8;
+    for (uint32_t q = 0; q < p.n_pass; ++q) {
+        const WhPass &ps = p.pass[q];
+        c += (uint64_t)per_point[ps.R] * ps.R * ((ps.B + 63) / 64 * 64);
+        shared = std::min(shared, ps.R & (0u - ps.R));
+    }
+    if (p.L <= 256 * kWhPoints) c += (shared == 8 ? 80ull : shared == 4 ? 12ull : 0ull) * p.L;
+    return alone ? c + c / 2 : c;
+}
+
 // Whole-signal plan of a window length (cached per device): the direct transform
 // or chirp-z over a smooth M >= 2N - 1 that fits, by the rule above; the direct
 // transform also where no chirp-z length fits; none when N does not fit or has a
-// prime above kWhPrimeMax and no chirp-z length fits. M is the one of the least
-// passes times points: 501 points take 1008 = 7 x 9 x 16.
+// prime above kWhPrimeMax and no chirp-z length fits. M is the one of the least cost:
+// 501 points take 1008 = 7 x 12 x 12.
 static const WhTables *wh_tables(uint32_t N, hipStream_t s)
 {
     static std::mutex mu;
@@ -1326,12 +1348,17 @@ static const WhTables *wh_tables(uint32_t N, hipStream_t s)
     WhPlan pc{};
     const bool own = direct && prefer_direct(pd, gen);
     if (!own) {
+        hipFuncAttributes fa512{};
+        hip_check(hipFuncGetAttributes(&fa512, (const void *)k_wh_tune<true, 512>), "hipFuncGetAttributes");
         uint64_t cost = ~0ull;
         for (uint64_t M = 2ull * N - 1; M <= 4ull * N && M <= kWhPmax && fits((uint32_t)M); ++M) {
             uint32_t g = 0;
             WhPlan pm{};
-            if (!wh_radix_plan((uint32_t)M, pm, g) || g || pm.n_pass * M >= cost) continue;
-            cost = pm.n_pass * M;
+            if (!wh_radix_plan((uint32_t)M, pm, g) || g) continue;
+            const bool alone = wh_threads((uint32_t)M) == 512 && 2 * (M * sizeof(Cplx) + fa512.sharedSizeBytes) > (size_t)v;
+            const uint64_t c = chirp_cost(pm, alone);
+            if (c >= cost) continue;
+            cost = c;
             Mcz = (uint32_t)M;
             pc = pm;
         }
