@@ -49,8 +49,8 @@ struct JobDesc {
 };
 
 // Per-particle state a MEGNO job carries from one segment to the next: the
-// tangent matrix (16), L1, L2 and log10|M|_F of the last turn.
-constexpr int kMegnoState = 19;
+// tangent matrix (16), L1 and L2.
+constexpr int kMegnoState = 18;
 
 struct BatchQueue {
     uint32_t total;   // chunks of the current segment
@@ -130,7 +130,6 @@ __global__ void k_megno_init(double *__restrict__ state, uint64_t n_particles)
     for (int q = 0; q < 16; q++) st[q] = (q % 5 == 0) ? 1.0 : 0.0;
     st[16] = 0.0;
     st[17] = 0.0;
-    st[18] = 0.0;  // formed from the matrix in the first segment
 }
 
 // Takes chunks of the tracking jobs until the queue holds no more.
@@ -203,7 +202,7 @@ __device__ __forceinline__ void megno_chunk(const BatchSeg &S, ConstPtr<JobDesc>
     uint32_t j = 0, s = 0;
     double x = __builtin_nan(""), px = x, y = x, py = x;
     double m[16];
-    MegnoSums sums{0.0, 0.0, 0.0};
+    MegnoSums sums{0.0, 0.0, {0.0, 0}};
     double *st = nullptr;
     if (in) {
         j = S.first ? i : S.lists_cur[list_off + i];
@@ -212,8 +211,7 @@ __device__ __forceinline__ void megno_chunk(const BatchSeg &S, ConstPtr<JobDesc>
         st = J->state + (size_t)j * kMegnoState;
 #pragma unroll
         for (int q = 0; q < 16; q++) m[q] = st[q];
-        sums = MegnoSums{st[16], st[17], st[18]};
-        if (S.first) sums.lh = half_log10(frob2_fused(m), log_tab);
+        sums = MegnoSums{st[16], st[17], log_norm_or_inf(frob2_fused(m), log_tab)};
     } else {
 #pragma unroll
         for (int q = 0; q < 16; q++) m[q] = 0.0;
@@ -245,7 +243,7 @@ __device__ __forceinline__ void megno_chunk(const BatchSeg &S, ConstPtr<JobDesc>
     bool pending = false;
     double w_prev = 0.0, inv_prev = 0.0;
     auto megno_update = [&]() {
-        sums.add(half_log10_or_inf(frob2_fused(m), log_tab), w_prev, inv_prev);
+        sums.add(log_norm_or_inf(frob2_fused(m), log_tab), w_prev, inv_prev);
         pending = false;
     };
     double xx = x * x, yy = y * y;  // carried between turns in exact mode
@@ -277,7 +275,7 @@ __device__ __forceinline__ void megno_chunk(const BatchSeg &S, ConstPtr<JobDesc>
                         const double inv_n = inv_idx[S.seg_start + kn];
                         const double f2 = frob2_fused(m);
                         zero_m = zero_m | (f2 == 0.0);
-                        sums.add(half_log10(f2, log_tab), w_prev, inv_prev);
+                        sums.add(log_norm(f2, log_tab), w_prev, inv_prev);
                         const Jac jc = jac_coeffs<MODE>(x, y, mu3, mu6);
                         mat_mul_structured<MODE>(jc, t, m);
                         const bool out = forward_turn_out<MODE, OCT>(x, px, y, py, xx, yy, mu, m3mu, t, b2);
@@ -290,7 +288,7 @@ __device__ __forceinline__ void megno_chunk(const BatchSeg &S, ConstPtr<JobDesc>
                     }
                 }
                 stop = k2;
-                if (zero_m) sums = MegnoSums{__builtin_nan(""), __builtin_nan(""), -HUGE_VAL};
+                if (zero_m) sums.lose();
                 if (alive_start && !alive) {
                     x = px = y = py = xx = yy = __builtin_nan("");
 #pragma unroll
@@ -335,7 +333,7 @@ __device__ __forceinline__ void megno_chunk(const BatchSeg &S, ConstPtr<JobDesc>
                 const double inv = 1.0 / fa;
 #pragma unroll
                 for (int q = 0; q < 16; q++) m[q] = m[q] * inv;
-                sums.lh = half_log10_or_inf(frob2_fused(m), log_tab);
+                sums.norm = log_norm_or_inf(frob2_fused(m), log_tab);
             }
         }
         if (!__any(alive || held)) break;
@@ -348,7 +346,7 @@ __device__ __forceinline__ void megno_chunk(const BatchSeg &S, ConstPtr<JobDesc>
     if (alive0 || held) {
 #pragma unroll
         for (int q = 0; q < 16; q++) st[q] = m[q];
-        st[16] = sums.l1; st[17] = sums.l2; st[18] = sums.lh;
+        st[16] = sums.l1; st[17] = sums.l2;
     }
     // a particle leaves the live list when lost (or all NaN from the start):
     // its MEGNO is final then; survivors and held particles get theirs after

@@ -16,24 +16,27 @@ __device__ __forceinline__ void fill_log_bins(LogBin *tab)
     __syncthreads();
 }
 
-// The MEGNO recursion of one add (src/henon.cu:2259-2283) in the form of norms'
-// logarithms: L1 += (log10|M_{k+1}| - log10|M_k|) idx, L2 += L1 / idx.
-struct MegnoSums {
-    double l1, l2, lh;  // lh = log10|M| before the add
-    __device__ __forceinline__ void add(double lh_new, double idx, double inv_idx)
-    {
-        l1 = fma(lh_new - lh, idx, l1);
-        l2 = fma(inv_idx, l1, l2);
-        lh = lh_new;
-    }
-};
-
-// half_log10 with log10(0) = -inf.
-__device__ __forceinline__ double half_log10_or_inf(double F, const LogBin *tab)
+// log_norm with log10(0) = -inf.
+__device__ __forceinline__ LogNorm log_norm_or_inf(double F, const LogBin *tab)
 {
-    const double v = half_log10(F, tab);
-    return F == 0.0 ? -HUGE_VAL : v;
+    const LogNorm v = log_norm(F, tab);
+    return LogNorm{F == 0.0 ? -HUGE_VAL : v.f, v.e};
 }
+
+// The MEGNO recursion of one add (src/henon.cu:2259-2283) in the form of norms'
+// logarithms: L1 += log10(|M_{k+1}| / |M_k|) idx, L2 += L1 / idx.
+struct MegnoSums {
+    double l1, l2;
+    LogNorm norm;  // of M before the add
+    __device__ __forceinline__ void add(const LogNorm &now, double idx, double inv_idx)
+    {
+        l1 = fma(log_ratio(now, norm), idx, l1);
+        l2 = fma(inv_idx, l1, l2);
+        norm = now;
+    }
+    // The logarithm of a zero matrix has been taken: no MEGNO from here on.
+    __device__ __forceinline__ void lose() { l1 = l2 = __builtin_nan(""); }
+};
 
 // M <- J M with J's structure: rows 0-1 touch M rows 0,1,2; rows 2-3 M rows 0,2,3.
 template <int MODE>

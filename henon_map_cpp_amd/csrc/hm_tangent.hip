@@ -160,11 +160,11 @@ struct IndicatorArgs {
     uint32_t first, last;
 };
 
-// Per-particle state between segments: M (16), log10 scale, L1, L2, log10|M|_F;
+// Per-particle state between segments: M (16), log10 scale, L1, L2;
 // with Birkhoff windows the last angles (2) and the window sums (2 per window);
 // with construct windows the megno_birkhoff sums (1 per window), the
 // tune_birkhoff sums (4 per window) and their last angles (2).
-constexpr int kIndBirkState = 20;                          // offset of the Birkhoff part
+constexpr int kIndBirkState = 19;                          // offset of the Birkhoff part
 constexpr int kIndConsState = kIndBirkState + 2 + 2 * kMaxBirk;  // offset of the construct part
 // doubles of state per particle in variant V (below)
 constexpr int ind_state_len(int V) { return V == 2 ? kIndConsState + 5 * kMaxBirk + 2 : V == 1 ? kIndConsState : kIndBirkState; }
@@ -243,7 +243,7 @@ __global__ void __launch_bounds__(256) k_indicators(IndicatorArgs a)
     }
     double m[16];
     double lscale = 0.0;
-    MegnoSums sums{0.0, 0.0, 0.0};
+    MegnoSums sums{0.0, 0.0, {0.0, 0}};
     double bacc[kMaxBirk][2];
 #pragma unroll
     for (int w = 0; w < kMaxBirk; w++) bacc[w][0] = bacc[w][1] = 0.0;
@@ -252,7 +252,7 @@ __global__ void __launch_bounds__(256) k_indicators(IndicatorArgs a)
         const double *st = a.state + (size_t)i * SL;
 #pragma unroll
         for (int q = 0; q < 16; q++) m[q] = st[q];
-        lscale = st[16]; sums = MegnoSums{st[17], st[18], st[19]};
+        lscale = st[16]; sums.l1 = st[17]; sums.l2 = st[18];
         if (BW && a.n_birk) {
             thx = st[kIndBirkState]; thy = st[kIndBirkState + 1];
 #pragma unroll
@@ -270,8 +270,8 @@ __global__ void __launch_bounds__(256) k_indicators(IndicatorArgs a)
             for (int q = 0; q < 16; q++) m[q] = (q % 5 == 0) ? 1.0 : 0.0;
         }
         lscale = (a.log_scale && in_range) ? a.log_scale[i] : 0.0;
-        sums.lh = half_log10_or_inf(frob2_fused(m), log_tab);
     }
+    sums.norm = log_norm_or_inf(frob2_fused(m), log_tab);
     const double mu3 = a.mu * 3, mu6 = a.mu * 6, m3mu = -3.0 * a.mu;
     const bool alive0 = in_range && !any_nan(x, px, y, py);
     // held: some but not all coordinates NaN. The particle is not tracked (its
@@ -353,7 +353,7 @@ __global__ void __launch_bounds__(256) k_indicators(IndicatorArgs a)
                 mbacc[w] = mbacc[w] + (sums.l1 * a.birk_w[a.mb_off[w] + idx - 1]) * inv;
     };
     auto megno_update = [&]() {
-        sums.add(half_log10_or_inf(frob2_fused(m), log_tab), w_prev, inv_prev);
+        sums.add(log_norm_or_inf(frob2_fused(m), log_tab), w_prev, inv_prev);
         if (EXTRA && a.n_mb) megno_birkhoff_turn(idx_prev, inv_prev);
         if (idx_prev == next_megno) {
             if (in_range && a.megno) a.megno[(size_t)sample_m * a.n + i] = inv_prev * sums.l2;
@@ -451,7 +451,7 @@ __global__ void __launch_bounds__(256) k_indicators(IndicatorArgs a)
                         // the construct windows take the sums turn by turn
                         const double f2 = frob2_fused(m);
                         zero_m = zero_m | (f2 == 0.0);
-                        sums.add(EXTRA ? half_log10_or_inf(f2, log_tab) : half_log10(f2, log_tab), w_prev, inv_prev);
+                        sums.add(EXTRA ? log_norm_or_inf(f2, log_tab) : log_norm(f2, log_tab), w_prev, inv_prev);
                         if (EXTRA && a.n_mb) megno_birkhoff_turn(idx_prev, inv_prev);
                         const Jac jc = jac_coeffs<TAN>(x, y, mu3, mu6);
                         mat_mul_structured<TAN>(jc, t, m);
@@ -469,7 +469,7 @@ __global__ void __launch_bounds__(256) k_indicators(IndicatorArgs a)
                     }
                 }
                 stop = k2;
-                if (!EXTRA && zero_m) sums = MegnoSums{__builtin_nan(""), __builtin_nan(""), -HUGE_VAL};
+                if (!EXTRA && zero_m) sums.lose();
                 if (alive_start && !alive) {
                     x = px = y = py = xx = yy = __builtin_nan("");
 #pragma unroll
@@ -545,7 +545,7 @@ __global__ void __launch_bounds__(256) k_indicators(IndicatorArgs a)
 #pragma unroll
                 for (int q = 0; q < 16; q++) m[q] = m[q] * inv;
                 lscale = lscale + log10(fa);
-                sums.lh = half_log10_or_inf(frob2_fused(m), log_tab);
+                sums.norm = log_norm_or_inf(frob2_fused(m), log_tab);
             }
         }
         if (BW && a.n_birk) birkhoff_turn(idx);
@@ -578,7 +578,7 @@ __global__ void __launch_bounds__(256) k_indicators(IndicatorArgs a)
         double *st = a.state + (size_t)i * SL;
 #pragma unroll
         for (int q = 0; q < 16; q++) st[q] = m[q];
-        st[16] = lscale; st[17] = sums.l1; st[18] = sums.l2; st[19] = sums.lh;
+        st[16] = lscale; st[17] = sums.l1; st[18] = sums.l2;
         if (BW && a.n_birk) {
             st[kIndBirkState] = thx; st[kIndBirkState + 1] = thy;
 #pragma unroll
