@@ -358,7 +358,7 @@ __global__ void __launch_bounds__(256) k_birkhoff_rows(const double *__restrict_
                                                        double *__restrict__ out)
 {
     // particles p0 .. p0 + nb - 1 of n
-    __shared__ double angle_tab[kAngleBins];
+    __shared__ AngleEntry angle_tab[kAngleEntries];
     fill_angle_table(angle_tab);
     __syncthreads();
     const uint64_t wave = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;

@@ -227,7 +227,7 @@ __global__ void __launch_bounds__(256) k_indicators(IndicatorArgs a)
     constexpr int SL = ind_state_len(V);
     constexpr int MAP = map_mode(MODE), TAN = tangent_mode(MODE);
     __shared__ LogBin log_tab[kLogBins];
-    __shared__ double angle_tab[BW ? kAngleBins : 1];
+    __shared__ AngleEntry angle_tab[BW ? kAngleEntries : 1];
     if (BW) fill_angle_table(angle_tab);
     fill_log_bins(log_tab);
     const uint32_t li = blockIdx.x * blockDim.x + threadIdx.x;  // position in the live list
