@@ -406,7 +406,9 @@ static uint32_t batch_resident_waves()
     int dev = 0, cus = 0;
     hip_check(hipGetDevice(&dev), "hipGetDevice");
     hip_check(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev), "hipDeviceGetAttribute");
-    return (uint32_t)cus * 32u;  // 4 SIMDs x 8 wavefronts (the kernel stays within 64 VGPRs)
+    // 4 SIMDs x 8 wavefronts (k_batch_track stays within 64 VGPRs; workgroups of
+    // k_batch_megno that find no room at first start on what the queue still holds)
+    return (uint32_t)cus * 32u;
 }
 
 }  // namespace hm
@@ -478,7 +480,7 @@ std::vector<std::pair<GraphKey, hipGraphExec_t>> g_graphs;  // oldest first
 void batch_run(const hm_job *jobs, size_t n_jobs, int mode, int block, int every, uint32_t waves, bool graph,
                hipStream_t s)
 {
-    // tracking-only jobs first, then the MEGNO jobs (each kernel takes one range)
+    // tracking-only jobs first, then the MEGNO jobs (two ranges with a queue head each)
     std::vector<size_t> order;
     order.reserve(n_jobs);
     for (size_t k = 0; k < n_jobs; ++k)

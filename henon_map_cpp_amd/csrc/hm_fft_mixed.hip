@@ -630,7 +630,7 @@ __device__ __forceinline__ void wh_pass(Cplx *buf, const WhPass &ps, const Cplx 
     __syncthreads();
 }
 
-// A pass of odd prime radix R (11 .. kWhPrimeMax) takes the R-point DFT from the
+// A pass of odd prime radix R (17 .. kWhPrimeMax) takes the R-point DFT from the
 // pairs (r, R - r) as in dft_prime, H = (R - 1) / 2:
 //   fold : each pair twiddled and replaced in place by a_r = x_r + x_{R-r} (at r)
 //          and b_r = x_r - x_{R-r} (at R - r)

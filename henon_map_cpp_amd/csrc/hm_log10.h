@@ -1,7 +1,8 @@
-// log10 in one straight block (the MEGNO sums take norms' logarithms from a table
-// instead, hm_lognorm.h; no kernel calls this one), by the method of fdlibm's e_log.c and
-// e_log10.c (Sun Microsystems, 1993; freely distributable): x = 2^k m with m in
-// [sqrt(2)/2, sqrt(2)), f = m - 1, s = f / (2 + f),
+// log10 in one straight block. Kept for the host check that holds it
+// (tests/log10_check.cpp); no kernel includes it, the MEGNO sums take norms' logarithms
+// from a table (hm_lognorm.h). By the method of fdlibm's e_log.c and e_log10.c (Sun
+// Microsystems, 1993; freely distributable): x = 2^k m with m in [sqrt(2)/2, sqrt(2)),
+// f = m - 1, s = f / (2 + f),
 //   ln m = 2 atanh(s) = f - s (f - R(s^2))            (or, for m near sqrt(2),
 //        = f - (f^2/2 - s (f^2/2 + R(s^2))))           the form with f^2/2)
 // with R the degree-7 minimax polynomial of fdlibm's log (Lg1..Lg7), and
@@ -10,10 +11,9 @@
 // reciprocal refined by Newton steps (2 + f lies in [1.7, 2.5]); zero,
 // negative, infinite and NaN arguments selected at the end (-inf, NaN, +inf,
 // NaN); subnormal arguments are not handled (the MEGNO norm ratio is never one).
-// At most 2 units in the last place from the C library's log10, 88 % of
-// arguments correctly rounded (tests/log10_check.cpp). The library's
-// double-double log10 takes about 90 instructions on gfx950 and a branch, this
-// one about 50.
+// At most 2 units in the last place from the C library's log10, 88 % of arguments
+// correctly rounded. The library's double-double log10 takes about 90 instructions on
+// gfx950 and a branch, this one about 50.
 // Compiles as host code too (no HIP types), so a host check can build it with
 // g++ alone; device and host differ only in the reciprocal's first estimate.
 #pragma once

@@ -260,10 +260,11 @@ extern "C" int hm_track(double *x, double *px, double *y, double *py, uint32_t *
 
         // Up to one wavefront per SIMD, compaction frees nothing that another wavefront
         // waits for: all turns go in one launch (up to about 0.1 s of them) unless the
-        // caller or the autotuner chose. 1e4 particles x 1e4 turns, mu = 0.5, r < 0.4: 0.89 -> 0.81 ms;
-        // 32768 x 1e5: 9.4 -> 8.5; 65536 x 1e5, r < 0.7, two thirds lost: 9.5 -> 8.5
-        // (r < 0.4, 2 % lost: 10.6 -> 10.9). With two wavefronts per SIMD it depends on
-        // the losses (131072 x 1e4: 1.82 -> 1.61 ms with few, 0.99 -> 1.01 with most).
+        // caller or the autotuner chose. In segments and in one launch, mu = 0.5, exact:
+        // 1e4 particles x 1e4 turns, r < 0.4, 0.98 and 0.87 ms; 32768 x 1e5 10.0 and 8.7;
+        // 65536 x 1e5 with none lost 12.1 and 10.9, 4 % lost 11.2 and 10.5, two thirds lost
+        // 10.0 and 9.0. Beyond, it depends on the losses (70000 x 1e5: 15.2 and 14.0 with
+        // none lost, 11.1 and 14.0 with a quarter).
         const bool one_launch = !a.segmented && (N + 63u) / 64u <= device_simds() && n_turns <= (1u << 20);
         if (one_launch || every < 0 || (uint32_t)every >= n_turns) {
             a.n_arg = a.grid_bound = N;
