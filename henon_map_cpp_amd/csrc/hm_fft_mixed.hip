@@ -976,7 +976,9 @@ __global__ void __launch_bounds__(NT, 4) k_wh_tune(WhArgs a)
     __syncthreads();
     if (threadIdx.x == 0) {
         auto mag = [&](uint32_t k) { return sqrt(square(k)); };
-        *o = interp_tune_at(mag, N, first == 0xffffffffu ? 0u : first, a.cos_n, a.sin_n);
+        // (a scan from entry 0 on never leaves one that is NaN, and passes later ones by)
+        const bool at_zero = first == 0xffffffffu || __builtin_isnan(square(0));
+        *o = interp_tune_at(mag, N, at_zero ? 0u : first, a.cos_n, a.sin_n);
     }
 }
 
