@@ -221,6 +221,8 @@ __device__ __forceinline__ void track_wave(const TrackArgs &A, uint32_t base, ui
             // before last used.
             const uint32_t last = n_turns - 2;
             TabEntry a0 = rec(0), a1 = rec(1), b0, b1;
+            ConstPtr<TabEntry> tp_next = tp - 1;
+            if (INV) asm("" : "+s"(tp_next));  // kept, not formed again at each use
             // At every 64th turn each lane takes one of the 64 records from 64 turns
             // ahead on: to see that all rotate before the turns get there, and so that
             // the scalar loads find the table in L2 also the first time it is read (64
@@ -236,13 +238,14 @@ __device__ __forceinline__ void track_wave(const TrackArgs &A, uint32_t base, ui
                 uint32_t m = min(blocks, 64 / kBlock);
                 blocks -= m;
                 do {
-                    const ConstPtr<TabEntry> p = INV ? tp - k : tp + k;
+                    // (from the lowest address of the block's records on, for fixed offsets)
+                    const ConstPtr<TabEntry> p = INV ? tp - (k + (kBlock - 1)) : tp + k;
 #pragma unroll
                     for (uint32_t q = 0; q < kBlock; q += 4) {
                         __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): a0, a1 are there
                         __builtin_amdgcn_sched_barrier(0);
-                        b0 = load_record(INV ? p - (q + 2) : p + (q + 2));
-                        b1 = load_record(INV ? p - (q + 3) : p + (q + 3));
+                        b0 = load_record(p + (INV ? kBlock - 1 - (q + 2) : q + 2));
+                        b1 = load_record(p + (INV ? kBlock - 1 - (q + 3) : q + 3));
                         // (keeps the loads ahead of the first turn)
                         asm volatile("" ::: "memory");
                         __builtin_amdgcn_sched_barrier(0);
@@ -250,9 +253,9 @@ __device__ __forceinline__ void track_wave(const TrackArgs &A, uint32_t base, ui
                         const uint32_t nx = min(k + q + 4, last);
                         __builtin_amdgcn_s_waitcnt(0xC07F);
                         __builtin_amdgcn_sched_barrier(0);
-                        const ConstPtr<TabEntry> pn = INV ? tp - nx : tp + nx;
-                        a0 = load_record(pn);
-                        a1 = load_record(INV ? pn - 1 : pn + 1);
+                        const ConstPtr<TabEntry> pn = INV ? tp_next - nx : tp + nx;
+                        a0 = load_record(INV ? pn + 1 : pn);
+                        a1 = load_record(INV ? pn : pn + 1);
                         __builtin_amdgcn_sched_barrier(0);
                         pair(b0, b1, k + q + 2);
                     }
