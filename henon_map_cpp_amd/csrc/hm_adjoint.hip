@@ -55,12 +55,14 @@ constexpr int kFwdBlock = 256;
 // With every % 8 == 0 (ALIGNED) the turns run eight to a pass of the loop, in pairs
 // with one loss test as the tracking kernel's (a point below safe1 after the first
 // turn is inside the barrier after the second), records and weights requested a pair
-// ahead by scalar loads and touched 64 to 128 turns ahead by a vector load. Otherwise
-// the turns run four at a time with scalar loads of two alternating prefetched pairs
-// of records and a test each.
-// With a test a turn and the records in an LDS ring before: 1e4 turns, mu = 0.5, exact, 1000 particles 1.17 -> 0.82 ms, 32768 1.20 ->
-// 0.98, 65536 1.36 -> 1.20, and 200000 x 4000 1.49 -> 1.20. At full load the chip's
-// power sets the pace: 34 FP64 operations a turn.
+// ahead by scalar loads; every 64 turns the lanes look at those of 64 to 128 turns
+// ahead, that all the records rotate and for L2. From a record on that does not, and
+// with other intervals, the turns run four at a time with scalar loads of two
+// alternating prefetched pairs of records and a test each.
+// With pairs instead of a test a turn and an LDS ring of records: 1e4 turns, mu = 0.5,
+// exact, 1000 particles 1.17 -> 0.84 ms, 32768 1.19 -> 0.88, 65536 1.23 -> 1.04, and
+// 200000 x 4000 1.37 -> 1.13. At full load the chip's power sets the pace: 34 FP64
+// operations a turn.
 template <int MODE, int OCT, bool ALIGNED>
 __global__ void __launch_bounds__(kFwdBlock) k_adjoint_forward(AdjointFwdArgs a)
 {
@@ -311,8 +313,8 @@ struct AdjRec {
 //    start of each 8-turn chunk after the first (sub-checkpoints). The segments
 //    are independent, so this part runs at full occupancy even for few particles.
 //  - the sweep (for every % 8 == 0 k_adjoint_sweep_split up to half a wavefront per
-//    SIMD and k_adjoint_sweep_fused beyond, else k_adjoint_sweep), a lane per particle, walks the window's chunks in reverse: the chunk's
-//    nine states S0..S8 (S8 = the next chunk's S0) come from its sub-checkpoint
+//    SIMD and k_adjoint_sweep_fused beyond, else k_adjoint_sweep), a lane per
+//    particle, walks the window's chunks in reverse: the chunk's nine states S0..S8 (S8 = the next chunk's S0) come from its sub-checkpoint
 //    (the segment's checkpoint for a first chunk), and the adjoint runs back
 //    through its turns. The states of the chunk before it are recomputed in the
 //    same straight-line block: the two dependency chains are independent and
@@ -705,9 +707,9 @@ __global__ void __launch_bounds__(kFusedBlock) k_adjoint_sweep_fused(AdjointSwee
 // and weights are uniform and come by scalar loads a pair of turns ahead; the
 // consumer's lanes touch those of 64 to 128 turns ahead. Same operations in the same
 // order, so the same results. Two pairs a workgroup, one wavefront on each SIMD of a
-// CU. Backward pass of 1e4 turns: 8192 particles 1.70 -> 1.15 ms, 32768 2.03 -> 1.57;
+// CU. Backward pass of 1e4 turns: 8192 particles 1.71 -> 1.18 ms, 32768 1.94 -> 1.54;
 // with more wavefronts than that the chip's power sets the pace, not the issue of
-// single wavefronts (65536: 2.74 ms in one wavefront, 2.87 in two).
+// single wavefronts (65536 in two wavefronts took 5 % longer than in one).
 // Wavefronts w < pairs (pairs = half the workgroup's) are consumers, w + pairs their
 // producers.
 constexpr int kSplitChunk = kChunk * 2 * 64;  // double2 entries: [turn][x px | y py][lane]
@@ -890,7 +892,7 @@ __global__ void __launch_bounds__(256) k_adjoint_sweep_split(AdjointSweepArgs a)
 }
 
 // Threads per workgroup: one wavefront up to two per CU, so that they spread over
-// the CUs (forward sweep, 1e4 turns, 16384 particles: 0.83 ms against 1.06); beyond
+// the CUs (forward sweep, 1e4 turns, 16384 particles: 0.84 ms against 1.06); beyond
 // that single wavefronts can come to share a SIMD while another has none (40000
 // particles 1.0 to 1.4 ms, 57344 1.49, against 1.10 and 1.12).
 static uint32_t adjoint_block(size_t n) { return (n + 63) / 64 <= device_simds() / 2 ? 64 : 256; }

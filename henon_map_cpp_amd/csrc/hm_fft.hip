@@ -350,8 +350,9 @@ __device__ __forceinline__ double last_lane(double v)
 // Bound by the angles, two thirds of what the rows' reading would take at full rate:
 // by the table (hm_angle.h) instead of the library 20000 rows of 10001 samples 2.04 ->
 // 1.70 ms (6.4 GB), 40000 of 501 0.235 -> 0.199; the neighbours' angles by lane moves
-// instead of four trips through LDS a sample 1.72 -> 1.57 and 0.200 -> 0.190. The sums' error against long double
-// is the same (rms 1.1e-15 at 2000 samples), that of adding them up.
+// instead of four trips through LDS a sample 1.72 -> 1.57 and 0.200 -> 0.190. The sums'
+// error against long double is the same (rms 1.1e-15 at 2000 samples), that of adding
+// them up.
 __global__ void __launch_bounds__(256) k_birkhoff_rows(const double *__restrict__ rows, uint64_t L, uint32_t n,
                                                        uint32_t p0, uint32_t nb, const double *__restrict__ means,
                                                        WindowSet ws, const double *__restrict__ w_flat,

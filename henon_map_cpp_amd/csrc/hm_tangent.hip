@@ -189,13 +189,14 @@ constexpr int ind_state_len(int V) { return V == 2 ? kIndConsState + 5 * kMaxBir
 // unfused matrix product and 33 the unfused map. With the norm's logarithm from
 // the table instead of a ratio's, the loss test by the reference's expression
 // alone and two turns per pass of the loop, a plain turn is 180 instructions
-// (256 before): 131072 particles x 1e5 turns, whole call, 105.7 -> 80.1 ms.
+// (256 before): 131072 particles x 1e5 turns, whole call, 104.6 -> 79.4 ms.
 // A call of few waves is bound by latency. Workgroups of 64 threads spread them over
-// the CUs and a vector load touches the records ahead, 65536 x 3000 without windows
-// 1.75 -> 1.73 ms (exact) and 1.37 -> 1.27 (fast), 4099 x 3000 1.46 -> 1.40. Turns with
+// the CUs and a vector load touches the records ahead: 65536 x 3000 without windows
+// 1.97 -> 1.69 ms (exact) and 1.55 -> 1.23 (fast), 4099 x 3000 1.70 -> 1.27, the shorter
+// turn included. Turns with
 // Birkhoff windows take two angles, which are most of what the windows cost: by the
 // table (hm_angle.h) instead of the library, 4099 x 3000 with two windows 3.40 ->
-// 2.81 ms, 131072 x 5000 8.36 -> 7.37 (both exact). Weights read ahead into lanes or
+// 2.74 ms, 131072 x 5000 8.36 -> 7.24 (both exact). Weights read ahead into lanes or
 // scalar registers cost more instructions than the loads they hide.
 // Variants V: 0 MEGNO/FLI only; 1 with Birkhoff windows; 2 with any of the
 // trajectory window and the construct windows as well. Every variant runs the

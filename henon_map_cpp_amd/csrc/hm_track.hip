@@ -54,9 +54,9 @@ static void launch_track(const TrackLaunch &a, hipStream_t s)
     const uint64_t waves = ((uint64_t)a.grid_bound + 63) / 64;
     // Up to one wavefront per SIMD, workgroups of one wavefront: they spread over
     // all CUs, where four of a workgroup would share one CU's scalar and
-    // instruction caches (1e4 turns of 1e4 particles, mu = 0.5: 0.93 ms against
-    // 1.16 ms; 65536 particles, one wavefront on every SIMD either way, 1.26
-    // against 1.27 ms, and no difference beyond).
+    // instruction caches (1e4 turns of 1e4 particles, mu = 0.5: 0.79 ms against
+    // 0.97 ms; 65536 particles, one wavefront on every SIMD either way, 1.08
+    // against 1.04 ms, and no difference beyond).
     const int block = a.block ? a.block : waves <= device_simds() ? 64 : kDefaultBlock;
     const uint64_t grid = (waves * 64 + block - 1) / block;
     if (grid == 0) return;

@@ -201,8 +201,8 @@ __device__ __forceinline__ void track_wave(const TrackArgs &A, uint32_t base, ui
             // turn is inside the barrier after the second, whatever it is, as far as
             // the records rotate. A turn is then 30 to 32 operations and half a test
             // (4 operations and a branch), where every turn had one: 1e6 particles on
-            // the 1000 x 1000 grid, 3e4 turns, mu = 0.5: 22.0 -> 19.3 ms (exact), 15.9
-            // -> 14.5 ms (fast).
+            // the 1000 x 1000 grid, 3e4 turns, mu = 0.5: 21.7 -> 19.1 ms (exact), 15.7
+            // -> 14.1 ms (fast).
             const double safe1 = A.safe1;
             auto pair = [&](const TabEntry &t0, const TabEntry &t1, uint32_t kk) {
                 turn(t0);
@@ -226,7 +226,7 @@ __device__ __forceinline__ void track_wave(const TrackArgs &A, uint32_t base, ui
             // At every 64th turn each lane takes one of the 64 records from 64 turns
             // ahead on: to see that all rotate before the turns get there, and so that
             // the scalar loads find the table in L2 also the first time it is read (64
-            // particles, 1e4 turns: 0.89 ms warm or cold; without 1.92 ms cold).
+            // particles, 1e4 turns: 0.79 ms; the first call 1.0 ms longer without).
             auto ahead = [&](uint32_t from) {
                 const uint32_t kk = min(from + lane, n_turns - 1);
                 return INV ? tab[s0 - 1 - kk] : tab[s0 + kk];

@@ -106,7 +106,7 @@ int hm_build_table(const double *omega_x, const double *omega_y, size_t n, doubl
 int hm_birkhoff_weights(uint32_t n_weights, double *out);
 
 /* ---- tracking ------------------------------------------------------------ */
-/* Launch configuration; zero fields take the tuned defaults. */
+/* Launch configuration; zero fields take the defaults. */
 typedef struct hm_launch_cfg {
     int32_t block;              /* threads per workgroup: 64, 128, 192 or 256 (0 = 64 up to one
                                    wavefront per SIMD, 256 beyond) */
@@ -116,7 +116,7 @@ typedef struct hm_launch_cfg {
     int32_t particles_per_lane; /* 0, 1 or 2, for callers that set it: every launch takes one
                                    particle per lane */
     int32_t table_staging;      /* HM_STAGING_*, for callers that set it: table records always come
-                                   by scalar loads, touched ahead of time by vector loads */
+                                   by scalar loads, looked at ahead of time by vector loads */
 } hm_launch_cfg;
 enum { HM_STAGING_AUTO = 0, HM_STAGING_SCALAR = 1, HM_STAGING_RING = 2 };
 
