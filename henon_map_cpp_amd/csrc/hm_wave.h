@@ -108,9 +108,10 @@ inline double safe_radius2(double barrier, double mu)
     if (!(std::fabs(barrier) > 0.0) || !(m < 1e100)) return 0.0;
     const double b = std::fmin(std::fabs(barrier), 1e100);
     const auto reach = [m](double r) { return r * (1.0 + r * (1.0 + m * r)); };
-    // Newton's steps from above (the function is convex): six of them for the usual
-    // barriers, 0.05 us a call, where 60 bisections took 0.6
-    double r = b;
+    // Newton's steps from above (the function is convex), from where one of the terms
+    // alone reaches b (none overflows there): at most six of them, 0.07 us a call, where
+    // 60 bisections took 0.6
+    double r = std::fmin(b, std::fmin(std::sqrt(b), std::cbrt(b / m)));
     for (int i = 0; i < 1100; ++i) {
         const double next = r - (reach(r) - b) / (1.0 + r * (2.0 + 3.0 * m * r));
         if (!(next < r * (1.0 - 1e-9))) break;
