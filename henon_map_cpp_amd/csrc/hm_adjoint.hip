@@ -314,9 +314,9 @@ struct AdjRec {
 //    are independent, so this part runs at full occupancy even for few particles.
 //  - the sweep (for every % 8 == 0 k_adjoint_sweep_split up to half a wavefront per
 //    SIMD and k_adjoint_sweep_fused beyond, else k_adjoint_sweep), a lane per
-//    particle, walks the window's chunks in reverse: the chunk's nine states S0..S8 (S8 = the next chunk's S0) come from its sub-checkpoint
-//    (the segment's checkpoint for a first chunk), and the adjoint runs back
-//    through its turns. The states of the chunk before it are recomputed in the
+//    particle, walks the window's chunks in reverse: the chunk's nine states S0..S8
+//    (S8 = the next chunk's S0) come from its sub-checkpoint (the segment's checkpoint
+//    for a first chunk), and the adjoint runs back through its turns. The states of the chunk before it are recomputed in the
 //    same straight-line block: the two dependency chains are independent and
 //    interleave, which matters at one wavefront per SIMD, where nothing else
 //    hides FP64 latency.
